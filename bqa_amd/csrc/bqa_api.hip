@@ -28,6 +28,7 @@
 #include "kernels_fast.hpp"
 #include "kernels_node.hpp"
 #include "kernels_sv.hpp"
+#include "node_gemm.hpp"
 
 using namespace bqa;
 
@@ -179,6 +180,7 @@ struct bqa_job {
   DevBuf msgs[2], lmbd, ext, canon, lmax, status, rho, bloch, edges, epart, gws, cws, conv, conv_msgs, zz, plist;
   std::vector<int32_t> node_cls, node_pos;  // qubit id -> (degree class, position in the class)
   bool zz_valid = false;  // zz holds the gates of the current simple update
+  bool hermitian = true;  // the messages are Hermitian; false after an upload of others, until BP replaces them
   BpStatus* st_host = nullptr;
   double* lmax_host = nullptr;
   hipStream_t stream = nullptr;
@@ -319,6 +321,14 @@ NodeLaunch plan_node(bqa_job* j, int n, size_t buf_bytes_total, size_t fixed_lds
     L.ws_elems = (long)elems_per_block;
   }
   return L;
+}
+
+// Workspace of the matrix-product kernels (node_gemm.hpp) for one class: nodes per round.
+int plan_gemm(bqa_job* j, const ClassDev& c, int chi, size_t csize) {
+  const int chunk = gemm_chunk(c.n, c.d, chi, csize);
+  const size_t need = (size_t)chunk * gemm_node_bytes(c.d, chi, csize);
+  if (need > j->gws.bytes) j->gws.ensure(need, j->dev_bytes, j->stream);
+  return chunk;
 }
 
 // Algorithmic bytes of one BP sweep over one class (the roofline numerator):
@@ -576,6 +586,11 @@ void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first) {
   }
   if (j->generic(kGenBP) || !fast_bp_launch<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0),
                          msg_ptr<R>(j, 1), reinterpret_cast<BpStatus*>(j->status.p), j->stream, variant)) {
+    if (!j->generic(kGenBP) && gemm_shape(c.d, chi) && j->hermitian) {
+      const int chunk = plan_gemm(j, c, chi, sizeof(cplx<R>));
+      gemm_bp<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0), msg_ptr<R>(j, 1),
+                 reinterpret_cast<BpStatus*>(j->status.p), j->gws.p, chunk, j->stream);
+    } else {
     const long S = 2 * ipow_l(chi, c.d);
     const size_t fixed = sizeof(cplx<R>) * (size_t)(kNT + 4 * chi * chi);
     NodeLaunch L = plan_node(j, c.n, sizeof(cplx<R>) * 3 * S, fixed, 3 * S, sizeof(cplx<R>));
@@ -583,6 +598,7 @@ void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first) {
                        reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0), msg_ptr<R>(j, 1),
                        reinterpret_cast<BpStatus*>(j->status.p), (cplx<R>*)nullptr, 0.0, (double*)nullptr,
                        (double*)nullptr, reinterpret_cast<cplx<R>*>(L.ws), L.ws_elems);
+    }
   }
   LAUNCH_CHECK();
   if (j->timing) {
@@ -838,6 +854,12 @@ void ext_class(bqa_job* j, ClassDev& c, double ztime, const cplx<double>* msgs64
     LAUNCH_CHECK();
     return;
   }
+  if (!j->generic(kGenExt) && gemm_shape(c.d, chi) && j->hermitian) {
+    const int chunk = plan_gemm(j, c, chi, sizeof(cplx<double>));
+    gemm_ext<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->gws.p, chunk, j->stream);
+    LAUNCH_CHECK();
+    return;
+  }
   const long S = 2 * ipow_l(chi, c.d);
   const cplx<double>* T64 = reinterpret_cast<const cplx<double>*>(T);
   if (sizeof(R) == sizeof(float)) {
@@ -879,9 +901,7 @@ void ext_and_canon(bqa_job* j, double ztime, double pinv_eps, bool sync = true, 
   bool need_generic = false;
   for (auto& c : j->cls)
     need_generic |= c.d != 0 && c.n > 0 &&
-                    (j->generic(kGenExt) || !((chi == 8 && c.d >= 2 && c.d <= 4) || small_shape(c.d, chi) ||
-                                              (chi == 16 && (c.d == 2 || c.d == 3)) ||
-                                              (sizeof(R) == sizeof(float) && c.d == 5 && small_bp_shape<R>(5, chi))));
+                    (j->generic(kGenExt) || !(ext_fast_shape<R>(c.d, chi) || (gemm_shape(c.d, chi) && j->hermitian)));
   if (sizeof(R) == sizeof(float) && need_generic) {
     const long cnt = (long)j->M * chi * chi;
     j->conv_msgs.ensure((size_t)cnt * sizeof(cplx<double>), j->dev_bytes, j->stream);
@@ -975,7 +995,10 @@ void local_update(bqa_job* j, int flags, int chi_out, double zz_time, double z_t
   const int chi_in = j->chi;
   const int n2 = 2 * chi_in;
   const int ccols = std::min(n2, j->chimax);
-  if (flags & kGauge) ensure_msgs(j, chi_out);
+  if (flags & kGauge) {
+    ensure_msgs(j, chi_out);
+    j->hermitian = true;   // the gauge sets every message to diag(lambda) / sum(lambda)
+  }
   for (auto& c : j->cls) {
     if (c.n == 0) continue;
     const int dst = 1 - c.tcur;
@@ -1182,6 +1205,7 @@ void project_impl(bqa_job* j, int count, const int32_t* ids, const int32_t* outc
 template <typename R>
 void init_state_impl(bqa_job* j) {
   j->chi = 1;
+  j->hermitian = true;
   j->mcur = 0;
   j->lstride = 1;
   ensure_msgs(j, 1);
@@ -1243,6 +1267,21 @@ void upload(bqa_job* j, void* dev, size_t count, const double* in) {
   HIPX(hipStreamSynchronize(j->stream));
 }
 
+// Whether `count` chi x chi complex matrices are Hermitian to 1e-10 of their largest element.
+bool hermitian(const double* m, long count, int chi) {
+  double most = 0.0, off = 0.0;
+  for (long q = 0; q < count; ++q, m += 2 * (size_t)chi * chi)
+    for (int a = 0; a < chi; ++a)
+      for (int b = 0; b <= a; ++b) {
+        const double *x = m + 2 * (a * chi + b), *y = m + 2 * (b * chi + a);
+        most = std::max({most, std::abs(x[0]), std::abs(x[1]), std::abs(y[0]), std::abs(y[1])});
+        const double diff = std::max(std::abs(x[0] - y[0]), std::abs(x[1] + y[1]));
+        if (!(diff < INFINITY)) return false;
+        off = std::max(off, diff);
+      }
+  return off <= 1e-10 * most;
+}
+
 template <typename F>
 void dispatch(bqa_job* j, F&& f) {
   HIPX(hipSetDevice(j->device));
@@ -1285,7 +1324,16 @@ size_t estimate(int N, int M, const std::vector<int>& deg, const std::vector<int
   // generic node kernels' global workspace (3 node buffers per workgroup, at most 1024 workgroups) once
   // their buffers leave LDS; FP64 elements for the extended-message and local kernels
   const double smax = 2.0 * ipow_d(chimax, dmax);
-  if (16.0 * 3.0 * smax > (double)kMaxLds) b += 1024.0 * 3.0 * smax * 16.0;
+  double gws = 16.0 * 3.0 * smax > (double)kMaxLds ? 1024.0 * 3.0 * smax * 16.0 : 0.0;
+  // products of the matrix-product kernels, at the bond dimensions where they serve a class
+  for (size_t c = 0; c < deg.size(); ++c)
+    for (int chi = 1; chi <= std::min(chimax, kGemmMaxChi); ++chi) {
+      const bool fast = prec == BQA_PREC_SINGLE ? bp_fast_shape<float>(deg[c], chi) && ext_fast_shape<float>(deg[c], chi)
+                                                : bp_fast_shape<double>(deg[c], chi) && ext_fast_shape<double>(deg[c], chi);
+      if (size[c] > 0 && !fast && gemm_shape(deg[c], chi))
+        gws = std::max(gws, (double)gemm_chunk(size[c], deg[c], chi, 16) * (double)gemm_node_bytes(deg[c], chi, 16));
+    }
+  b += gws;
   // FP32 jobs whose extended messages run the generic kernel widen tensors and messages to FP64: at
   // bond dimension 1 (the first step) always, at chimax when no specialised kernel serves the shape
   if (prec == BQA_PREC_SINGLE) {
@@ -2040,6 +2088,7 @@ int bqa_set_messages(bqa_job* j, int32_t chi, const double* in) {
     ensure_msgs(j, chi);
     const size_t count = (size_t)j->M * chi * chi;
     dispatch(j, [&](auto r) { upload<decltype(r)>(j, j->msgs[j->mcur].p, count, in); });
+    j->hermitian = hermitian(in, j->M, chi);
   });
 }
 

@@ -36,6 +36,14 @@ inline bool bp_fast_shape(int d, int chi) {
   return small_bp_shape<R>(d, chi);
 }
 
+// Shapes whose extended messages have one (fast_ext_launch returns true for them).
+template <typename R>
+inline bool ext_fast_shape(int d, int chi) {
+  if (chi == 8 && d >= 2 && d <= 4) return true;
+  if (chi == 16 && (d == 2 || d == 3)) return true;
+  return small_shape(d, chi) || (sizeof(R) == sizeof(float) && d == 5 && small_bp_shape<R>(5, chi));
+}
+
 template <typename R>
 const char* bp_variant_name(int d, int chi, int v);
 

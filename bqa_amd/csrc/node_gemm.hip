@@ -1,0 +1,579 @@
+// Node contractions as batched matrix products (interface and plan: node_gemm.hpp).
+//
+// A node tensor T[p, b_1 .. b_d] is too large for LDS at chi > 16 (512 KB at chi = 32, d = 3) and at
+// degree 5 from chi = 8, and a block per node leaves the chip idle on small graphs.  Here every
+// partial product of a class goes through a workspace in HBM (sized so a chunk of nodes stays in the
+// 256 MB Infinity Cache), one launch per level over (node, product, tiles of fibres), and one launch
+// of Grams over (node, output).  Both are complex products on MFMA tiles of 16 x 16 x 4 in the real
+// form of eight complex rows (a row for each real and imaginary part), so chi need only be a multiple
+// of 8 in the rows and of 4 in the summed index to waste nothing.  A wave keeps its message
+// fragments in registers and streams fibres straight from memory: 16 lanes read 16 neighbouring
+// fibres (128 bytes in FP32), nothing is staged through LDS, and the next tile is in flight
+// while this one multiplies.
+#include "node_gemm.hpp"
+
+#include <algorithm>
+
+namespace bqa {
+
+namespace {
+
+constexpr int kGemmThreads = 256;
+constexpr int kGemmWaves = kGemmThreads / 64;
+
+template <typename R>
+struct Vec4T {
+  typedef R type __attribute__((ext_vector_type(4)));
+};
+template <typename R>
+using vec4 = typename Vec4T<R>::type;
+
+__device__ __forceinline__ vec4<float> mfma4(float a, float b, vec4<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ vec4<double> mfma4(double a, double b, vec4<double> c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Value of lane ^ 1 (a quad permutation).
+__device__ __forceinline__ float swap1(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double swap1(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Row r of a 16-row tile holds part ri (0 real, 1 imaginary) of complex row a of eight, such that a
+// lane's four result registers are two whole complex numbers, rows a = 2 g and 2 g + 1 of its lane
+// group g = lane / 16 (FP32 results lie in rows 4 g + v, FP64 in g + 4 v).
+template <typename R>
+__device__ __forceinline__ void tile_row(int r, int& a, int& ri);
+template <>
+__device__ __forceinline__ void tile_row<float>(int r, int& a, int& ri) {
+  a = r >> 1;
+  ri = r & 1;
+}
+template <>
+__device__ __forceinline__ void tile_row<double>(int r, int& a, int& ri) {
+  a = 2 * (r & 3) + (r >> 3);
+  ri = (r >> 2) & 1;
+}
+// Result row of register v of lane group g.
+template <typename R>
+__device__ __forceinline__ int result_row(int g, int v) {
+  return sizeof(R) == 4 ? 4 * g + v : g + 4 * v;
+}
+
+// A wave's fragments of the matrix W (rows a < ma, columns b < kb, element (a, b) at w[a * sa + b * sb]):
+// re / im [mt][ks] multiply the real / imaginary part of source element b = 4 ks + g.
+template <typename R, int KS, int MT>
+struct MatFrag {
+  R re[MT][KS], im[MT][KS];
+  template <typename RM>
+  __device__ __forceinline__ void load(const cplx<RM>* __restrict__ w, int ma, int kb, int sa, int sb) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    int al, ri;
+    tile_row<R>(r, al, ri);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int a = 8 * mt + al, b = 4 * ks + g;
+        cplx<RM> v = mk<RM>(0, 0);
+        if (a < ma && b < kb) v = w[a * sa + b * sb];
+        re[mt][ks] = (R)(ri == 0 ? v.x : v.y);
+        im[mt][ks] = (R)(ri == 0 ? -v.y : v.x);
+      }
+  }
+};
+
+// dst[o, a, i] = sum_b W[a, b] src[o, b, i] for fibres f = o * inner + i in [f0, f1), 16 at a time;
+// this wave takes tiles `wave`, `wave + step`, ...
+template <typename R, typename RS, int KS, int MT>
+__device__ __forceinline__ void product_tiles(const MatFrag<R, KS, MT>& w, const cplx<RS>* __restrict__ src,
+                                              cplx<R>* __restrict__ dst, int kb, int ma, int inner, int f0, int f1,
+                                              int wave, int step) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int tiles = (f1 - f0 + 15) >> 4;
+  int soff = 0, doff = 0;
+  bool live = false;
+  cplx<RS> nx[KS];
+  auto fetch = [&](int t) {
+    const int f = f0 + 16 * t + r;
+    live = f < f1;
+    const int o = f / inner, i = f - o * inner;
+    soff = o * kb * inner + i;
+    doff = o * ma * inner + i;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int b = 4 * ks + g;
+      nx[ks] = mk<RS>(0, 0);
+      if (live && b < kb) nx[ks] = src[soff + b * inner];
+    }
+  };
+  if (wave < tiles) fetch(wave);
+  for (int t = wave; t < tiles; t += step) {
+    R xr[KS], xi[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      xr[ks] = (R)nx[ks].x;
+      xi[ks] = (R)nx[ks].y;
+    }
+    const int at = doff;
+    const bool on = live;
+    if (t + step < tiles) fetch(t + step);
+    vec4<R> acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = vec4<R>{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma4(w.re[mt][ks], xr[ks], acc[mt]);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma4(w.im[mt][ks], xi[ks], acc[mt]);
+    }
+    if (on) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int a = 8 * mt + 2 * g + h;
+          if (a < ma) dst[at + a * inner] = mk<R>(acc[mt][2 * h], acc[mt][2 * h + 1]);
+        }
+    }
+  }
+}
+
+// Two neighbouring elements in one access (an even element index).
+template <typename R>
+struct alignas(4 * sizeof(R) <= 16 ? 4 * sizeof(R) : 16) Pair {
+  cplx<R> a, b;
+};
+
+// acc[mt][nt] += tile (rows: parts of X's free index, columns: parts of Y's) of the real products of
+// X[f, c] and Y[f, e] over fibres [f0, f1), 16 at a time; this wave takes groups `wave`, `wave + step`.
+// Lanes of a pair load two fibres each for one row of eight and swap the parts the other needs,
+// so every element is read once and 16 fibres come as whole lines.
+template <typename R, int MT, bool PAIR, typename RX, typename RY>
+__device__ __forceinline__ void gram_tiles(vec4<R> (&acc)[MT][MT], const cplx<RX>* __restrict__ X,
+                                           const cplx<RY>* __restrict__ Y, int chi, int inner, int f0, int f1,
+                                           int wave, int step) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int cl = r >> 1, ri = r & 1;
+  const int groups = (f1 - f0 + 15) >> 4;
+  cplx<RX> nx[MT][2];
+  cplx<RY> ny[MT][2];
+  auto fetch = [&](int q) {
+    const int f = f0 + 16 * q + 4 * g + 2 * ri;
+    const int o0 = f / inner, i0 = f - o0 * inner;
+    const int at0 = o0 * chi * inner + i0;
+    int at1 = at0 + 1;
+    if constexpr (!PAIR) {
+      const int o1 = (f + 1) / inner;
+      at1 = o1 * chi * inner + (f + 1 - o1 * inner);
+    }
+    const bool on0 = f < f1, on1 = f + 1 < f1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int c = 8 * mt + cl;
+      nx[mt][0] = nx[mt][1] = mk<RX>(0, 0);
+      ny[mt][0] = ny[mt][1] = mk<RY>(0, 0);
+      if (c < chi) {
+        if constexpr (PAIR) {
+          if (on0) {
+            const Pair<RX> px = *reinterpret_cast<const Pair<RX>*>(X + at0 + c * inner);
+            const Pair<RY> py = *reinterpret_cast<const Pair<RY>*>(Y + at0 + c * inner);
+            nx[mt][0] = px.a;
+            nx[mt][1] = px.b;
+            ny[mt][0] = py.a;
+            ny[mt][1] = py.b;
+          }
+        } else {
+          if (on0) {
+            nx[mt][0] = X[at0 + c * inner];
+            ny[mt][0] = Y[at0 + c * inner];
+          }
+          if (on1) {
+            nx[mt][1] = X[at1 + c * inner];
+            ny[mt][1] = Y[at1 + c * inner];
+          }
+        }
+      }
+    }
+  };
+  auto spread = [&](const auto& v, R (&out)[4]) {
+    const R s0 = (R)(ri ? v[0].x : v[0].y), s1 = (R)(ri ? v[1].x : v[1].y);
+    const R m0 = (R)(ri ? v[0].y : v[0].x), m1 = (R)(ri ? v[1].y : v[1].x);
+    const R q0 = swap1(s0), q1 = swap1(s1);
+    out[0] = ri ? q0 : m0;
+    out[1] = ri ? q1 : m1;
+    out[2] = ri ? m0 : q0;
+    out[3] = ri ? m1 : q1;
+  };
+  if (wave < groups) fetch(wave);
+  for (int q = wave; q < groups; q += step) {
+    R a[MT][4], b[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      spread(nx[mt], a[mt]);
+      spread(ny[mt], b[mt]);
+    }
+    if (q + step < groups) fetch(q + step);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < MT; ++nt) acc[mt][nt] = mfma4(a[mt][t], b[nt][t], acc[mt][nt]);
+  }
+}
+
+template <typename R, int MT, typename RX, typename RY>
+__device__ __forceinline__ void gram_range(vec4<R> (&acc)[MT][MT], const cplx<RX>* X, const cplx<RY>* Y, int chi,
+                                           int inner, int f0, int f1, int wave, int step) {
+  if ((inner & 1) == 0)
+    gram_tiles<R, MT, true>(acc, X, Y, chi, inner, f0, f1, wave, step);
+  else
+    gram_tiles<R, MT, false>(acc, X, Y, chi, inner, f0, f1, wave, step);
+}
+
+// sum[row][col] (16 MT square) of the waves' tiles, one wave after the other, in FP64.
+template <typename R, int MT>
+__device__ __forceinline__ void add_tiles(double* sum, const vec4<R> (&acc)[MT][MT], bool first) {
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < MT; ++nt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        double* s = sum + (16 * mt + result_row<R>(g, v)) * 16 * MT + 16 * nt + col;
+        *s = first ? (double)acc[mt][nt][v] : *s + (double)acc[mt][nt][v];
+      }
+}
+
+// Element (c, e) of the Gram sum conj(X) Y from the summed real products.
+template <int MT>
+__device__ __forceinline__ cplx<double> gram_at(const double* sum, int c, int e) {
+  const double* u = sum + (2 * c) * 16 * MT + 2 * e;
+  const double* v = u + 16 * MT;
+  return mk(u[0] + v[1], u[1] - v[0]);
+}
+
+// Blocks of the same node follow each other on one XCD (blocks go to the eight XCDs in turn), so
+// a node's tensor and products are re-read through that XCD's L2.
+__device__ __forceinline__ bool node_item(int idx, int per, int count, int& node, int& sub) {
+  node = (idx / per) * 8 + (blockIdx.x & 7);
+  sub = idx % per;
+  return node < count;
+}
+
+// The products of one level: block (node, product, part of the fibres).
+template <typename R, typename RS, typename RM, int KS, int MT, bool BP>
+__global__ __launch_bounds__(kGemmThreads) void k_gemm_product(ClassView cv, GemmPlan plan, int level, int parts,
+                                                               int node0, int count, int chi,
+                                                               const cplx<RS>* __restrict__ T, const cplx<RM>* mA,
+                                                               const cplx<RM>* mB, BpStatus* st, cplx<R>* ws) {
+  const cplx<RM>* msg = mA;
+  if constexpr (BP) {
+    const int cur = bp_begin(st, cv.sweep);
+    if (cur < 0) return;
+    msg = cur ? mB : mA;
+  }
+  const int q0 = plan.first[level], nq = plan.first[level + 1] - q0;
+  int node, sub;
+  if (!node_item(blockIdx.x >> 3, nq * parts, count, node, sub)) return;
+  const int q = q0 + sub / parts, part = sub % parts;
+  const int i = node0 + node, bond = plan.bond[q], src = plan.src[q];
+  const long S = 2L * ipow(chi, plan.d);
+  const int inner = ipow(chi, plan.d - 1 - bond);
+  const int F = 2 * ipow(chi, plan.d - 1);
+  MatFrag<R, KS, MT> w;
+  w.load(msg + (size_t)cv.in_pos[bond * cv.n + i] * chi * chi, chi, chi, chi, 1);
+  cplx<R>* base = ws + (size_t)node * plan.products * S;
+  cplx<R>* dst = base + q * S;
+  const int wave = part * kGemmWaves + (threadIdx.x >> 6), step = parts * kGemmWaves;
+  if (src < 0)
+    product_tiles<R, RS, KS, MT>(w, T + (size_t)i * S, dst, chi, chi, inner, 0, F, wave, step);
+  else
+    product_tiles<R, R, KS, MT>(w, base + src * S, dst, chi, chi, inner, 0, F, wave, step);
+}
+
+template <typename R, typename RS, int MT>
+__device__ __forceinline__ void gram_sources(vec4<R> (&acc)[MT][MT], const GemmPlan& plan, int k, int chi,
+                                             const cplx<RS>* Ti, const cplx<R>* base, long S, int f0, int f1,
+                                             int wave, int step) {
+  const int inner = ipow(chi, plan.d - 1 - k);
+  const int bra = plan.bra[k], ket = plan.ket[k];
+  if constexpr (sizeof(R) == sizeof(RS)) {
+    const cplx<R>* X = bra < 0 ? reinterpret_cast<const cplx<R>*>(Ti) : base + bra * S;
+    const cplx<R>* Y = ket < 0 ? reinterpret_cast<const cplx<R>*>(Ti) : base + ket * S;
+    gram_range<R, MT>(acc, X, Y, chi, inner, f0, f1, wave, step);
+  } else {
+    if (bra >= 0)
+      gram_range<R, MT>(acc, base + bra * S, base + ket * S, chi, inner, f0, f1, wave, step);
+    else if (ket >= 0)
+      gram_range<R, MT>(acc, Ti, base + ket * S, chi, inner, f0, f1, wave, step);
+    else
+      gram_range<R, MT>(acc, Ti, Ti, chi, inner, f0, f1, wave, step);
+  }
+}
+
+// New messages: blocks take (node, output) items in turn and keep their distance maxima until the end.
+template <typename R, int MT>
+__global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_bp(ClassView cv, GemmPlan plan, int node0, int count,
+                                                               int chi, const cplx<R>* __restrict__ T, cplx<R>* mA,
+                                                               cplx<R>* mB, BpStatus* st, const cplx<R>* ws) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double shred[16];
+  double* sum = reinterpret_cast<double*>(smem_raw);
+  const int cur = bp_begin(st, cv.sweep);
+  if (cur < 0) return;
+  const cplx<R>* min = cur ? mB : mA;
+  cplx<R>* mout = cur ? mA : mB;
+  const int cc = chi * chi, d = plan.d, wave = threadIdx.x >> 6;
+  const long S = 2L * ipow(chi, d);
+  const int F = 2 * ipow(chi, d - 1);
+  double dnum = 0.0, dden = 0.0;
+  int node, k;
+  for (int idx = blockIdx.x >> 3; node_item(idx, d, count, node, k); idx += gridDim.x >> 3) {
+    const int i = node0 + node;
+    vec4<R> acc[MT][MT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+      for (int b = 0; b < MT; ++b) acc[a][b] = vec4<R>{0, 0, 0, 0};
+    gram_sources<R, R, MT>(acc, plan, k, chi, T + (size_t)i * S, ws + (size_t)node * plan.products * S, S, 0, F, wave,
+                           kGemmWaves);
+#pragma unroll 1
+    for (int w = 0; w < kGemmWaves; ++w) {
+      if (w == wave) add_tiles<R, MT>(sum, acc, w == 0);
+      __syncthreads();
+    }
+    double tr = 0.0;
+    for (int c = 0; c < chi; ++c) tr += gram_at<MT>(sum, c, c).x;
+    const double inv = 0.5 / tr;
+    const long pos = cv.out_pos[k * cv.n + i];
+    for (int o = threadIdx.x; o < cc; o += kGemmThreads) {
+      const int c = o / chi, e = o % chi;
+      const cplx<double> a = gram_at<MT>(sum, c, e), b = gram_at<MT>(sum, e, c);
+      const cplx<R> v = cast<R>(mk((a.x + b.x) * inv, (a.y - b.y) * inv));
+      const cplx<R> old = min[pos * cc + o];
+      dnum = fmax(dnum, (double)cabs(v - old));
+      dden = fmax(dden, (double)cabs(v + old));
+      mout[pos * cc + o] = v;
+    }
+    __syncthreads();
+  }
+  dnum = block_max(dnum, shred);
+  dden = block_max(dden, shred);
+  if (threadIdx.x == 0) bp_end(st, cv.sweep, dnum, dden);
+}
+
+// Extended messages: the Grams of the two physical halves (fibres [0, F / 2) and [F / 2, F), each
+// over half of the waves), assembled with the bond's ZZ-split gates (backends.py:393-404,519-526).
+template <typename RS, int MT>
+__global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_ext(ClassView cv, GemmPlan plan, int node0, int count,
+                                                                int chi, const cplx<RS>* __restrict__ T,
+                                                                cplx<double>* __restrict__ ext,
+                                                                const cplx<double>* ws) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int kSide = 16 * MT, kHalf = kGemmWaves / 2;
+  double* sum = reinterpret_cast<double*>(smem_raw);
+  const int d = plan.d, wave = threadIdx.x >> 6, p = wave / kHalf, n2 = 2 * chi;
+  const long S = 2L * ipow(chi, d);
+  const int half = ipow(chi, d - 1);
+  int node, k;
+  for (int idx = blockIdx.x >> 3; node_item(idx, d, count, node, k); idx += gridDim.x >> 3) {
+    const int i = node0 + node;
+    vec4<double> acc[MT][MT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+      for (int b = 0; b < MT; ++b) acc[a][b] = vec4<double>{0, 0, 0, 0};
+    gram_sources<double, RS, MT>(acc, plan, k, chi, T + (size_t)i * S, ws + (size_t)node * plan.products * S, S,
+                                 p * half, (p + 1) * half, wave % kHalf, kHalf);
+#pragma unroll 1
+    for (int w = 0; w < kHalf; ++w) {
+      if (w == wave % kHalf) add_tiles<double, MT>(sum + p * kSide * kSide, acc, w == 0);
+      __syncthreads();
+    }
+    const cplx<double>* g = cv.zz + 2 * (size_t)cv.lmbd_pos[k * cv.n + i];
+    const cplx<double> gs[2] = {g[0], g[1]};
+    const double weight = abs2(gs[0]) + abs2(gs[1]);
+    cplx<double> tr = mk(0.0, 0.0);
+    for (int c = 0; c < chi; ++c)
+      tr = tr + gram_at<MT>(sum, c, c) + gram_at<MT>(sum + kSide * kSide, c, c);
+    const cplx<double> inv = cinv(scale(tr, weight));
+    cplx<double>* out = ext + (size_t)cv.out_pos[k * cv.n + i] * n2 * n2;
+    for (int o = threadIdx.x; o < n2 * n2; o += kGemmThreads) {
+      const int row = o / n2, col = o % n2;
+      const int s = row / chi, c = row % chi, s2 = col / chi, e = col % chi;
+      const cplx<double> g0 = gram_at<MT>(sum, c, e), g1 = gram_at<MT>(sum + kSide * kSide, c, e);
+      out[o] = conj(gs[s]) * gs[s2] * (((s + s2) & 1) ? g0 - g1 : g0 + g1) * inv;
+    }
+    __syncthreads();
+  }
+}
+
+// Calls f.template operator()<KS, MT>() with the tile counts of bond dimension chi.
+template <typename F>
+void by_chi(int chi, F&& f) {
+  switch ((chi + 3) / 4) {
+    case 1: f.template operator()<1, 1>(); break;
+    case 2: f.template operator()<2, 1>(); break;
+    case 3: f.template operator()<3, 2>(); break;
+    case 4: f.template operator()<4, 2>(); break;
+    case 5: f.template operator()<5, 3>(); break;
+    case 6: f.template operator()<6, 3>(); break;
+    case 7: f.template operator()<7, 4>(); break;
+    default: f.template operator()<8, 4>(); break;
+  }
+}
+
+// Parts of a node's fibres: about eight tiles a wave to pay for the message fragments, fewer where
+// the launch would not give every CU four blocks.
+int product_parts(int count, int products, long fibres) {
+  const long tiles = (fibres + 15) / 16;
+  const long most = std::max<long>(1, (tiles + kGemmWaves - 1) / kGemmWaves);
+  const long least = std::max<long>(1, (tiles + 8 * kGemmWaves - 1) / (8 * kGemmWaves));
+  const long want = (1024 + (long)count * products - 1) / ((long)count * products);
+  return (int)std::min(most, std::max(least, want));
+}
+
+int padded8(int n) { return (n + 7) / 8 * 8; }
+
+template <typename R, typename RS, typename RM, bool BP>
+void launch_products(const ClassView& cv, const GemmPlan& plan, int chi, int node0, int count, const cplx<RS>* T,
+                     const cplx<RM>* mA, const cplx<RM>* mB, BpStatus* st, cplx<R>* ws, hipStream_t s) {
+  const long fibres = 2L * ipow(chi, plan.d - 1);
+  for (int level = 0; level < plan.levels; ++level) {
+    const int nq = plan.first[level + 1] - plan.first[level];
+    const int parts = product_parts(count, nq, fibres);
+    const dim3 grid((unsigned)(padded8(count) * nq * parts));
+    by_chi(chi, [&]<int KS, int MT>() {
+      hipLaunchKernelGGL((k_gemm_product<R, RS, RM, KS, MT, BP>), grid, dim3(kGemmThreads), 0, s, cv, plan, level,
+                         parts, node0, count, chi, T, mA, mB, st, ws);
+    });
+  }
+}
+
+constexpr int kGramBlocks = 2048;   // eight blocks a CU; each keeps its maxima over its items
+
+}  // namespace
+
+GemmPlan gemm_plan(int d) {
+  GemmPlan p{};
+  p.d = d;
+  // index sets of the products made so far; a product of a set multiplies one more bond onto the
+  // product of the set without it
+  int sets[kGemmMaxProducts], level[kGemmMaxProducts], n = 0;
+  auto find = [&](int set) {
+    for (int q = 0; q < n; ++q)
+      if (sets[q] == set) return q;
+    return -1;
+  };
+  struct Item {
+    int set, src, bond, level;
+  };
+  auto make = [&](auto&& self, int set) -> int {
+    if (set == 0) return -1;
+    const int have = find(set);
+    if (have >= 0) return have;
+    int from = -1, bond = -1;
+    for (int b = 0; b < d && bond < 0; ++b)
+      if ((set >> b & 1) && (set & (set - 1)) && find(set & ~(1 << b)) >= 0) bond = b;
+    if (bond < 0)
+      for (int b = d - 1; b >= 0 && bond < 0; --b)
+        if (set >> b & 1) bond = b;
+    from = self(self, set & ~(1 << bond));
+    sets[n] = set;
+    level[n] = from < 0 ? 0 : level[from] + 1;
+    p.src[n] = (int8_t)from;
+    p.bond[n] = (int8_t)bond;
+    return n++;
+  };
+  const int all = (1 << d) - 1;
+  const int low = (1 << (d / 2)) - 1, high = all & ~low;
+  for (int k = 0; k < d; ++k) {
+    int bra, ket;
+    if (d <= 3) {   // one message on each side
+      const int rest = all & ~(1 << k);
+      ket = rest & -rest;
+      bra = rest & ~ket;
+    } else {        // the other half whole, this half without k
+      ket = (low >> k & 1) ? high : low;
+      bra = all & ~ket & ~(1 << k);
+    }
+    p.ket[k] = (int8_t)make(make, ket);
+    p.bra[k] = (int8_t)make(make, bra);
+  }
+  p.products = n;
+  // order by level, renumbering the sources
+  int order[kGemmMaxProducts], place[kGemmMaxProducts], m = 0;
+  for (int l = 0; m < n; ++l) {
+    p.first[l] = m;
+    for (int q = 0; q < n; ++q)
+      if (level[q] == l) {
+        place[q] = m;
+        order[m++] = q;
+      }
+    p.levels = l + 1;
+    p.first[l + 1] = m;
+  }
+  GemmPlan out = p;
+  for (int x = 0; x < n; ++x) {
+    out.src[x] = p.src[order[x]] < 0 ? (int8_t)-1 : (int8_t)place[p.src[order[x]]];
+    out.bond[x] = p.bond[order[x]];
+  }
+  for (int k = 0; k < d; ++k) {
+    out.bra[k] = p.bra[k] < 0 ? (int8_t)-1 : (int8_t)place[p.bra[k]];
+    out.ket[k] = p.ket[k] < 0 ? (int8_t)-1 : (int8_t)place[p.ket[k]];
+  }
+  return out;
+}
+
+template <typename R>
+void gemm_bp(ClassView cv, int chi, const cplx<R>* T, cplx<R>* mA, cplx<R>* mB, BpStatus* st, void* ws, int chunk,
+             hipStream_t s) {
+  const GemmPlan plan = gemm_plan(cv.d);
+  cplx<R>* w = reinterpret_cast<cplx<R>*>(ws);
+  for (int node0 = 0; node0 < cv.n; node0 += chunk) {
+    const int count = std::min(chunk, cv.n - node0);
+    launch_products<R, R, R, true>(cv, plan, chi, node0, count, T, mA, mB, st, w, s);
+    const int grid = std::min(padded8(count) * cv.d, kGramBlocks);
+    by_chi(chi, [&]<int KS, int MT>() {
+      hipLaunchKernelGGL((k_gemm_gram_bp<R, MT>), dim3(grid), dim3(kGemmThreads), sizeof(double) * 256 * MT * MT, s,
+                         cv, plan, node0, count, chi, T, mA, mB, st, w);
+    });
+  }
+}
+
+template <typename R>
+void gemm_ext(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msgs, cplx<double>* ext, void* ws, int chunk,
+              hipStream_t s) {
+  const GemmPlan plan = gemm_plan(cv.d);
+  cplx<double>* w = reinterpret_cast<cplx<double>*>(ws);
+  for (int node0 = 0; node0 < cv.n; node0 += chunk) {
+    const int count = std::min(chunk, cv.n - node0);
+    launch_products<double, R, R, false>(cv, plan, chi, node0, count, T, msgs, msgs, nullptr, w, s);
+    const int grid = std::min(padded8(count) * cv.d, kGramBlocks);
+    by_chi(chi, [&]<int KS, int MT>() {
+      hipLaunchKernelGGL((k_gemm_gram_ext<R, MT>), dim3(grid), dim3(kGemmThreads), 2 * sizeof(double) * 256 * MT * MT,
+                         s, cv, plan, node0, count, chi, T, ext, w);
+    });
+  }
+}
+
+template void gemm_bp<float>(ClassView, int, const cplx<float>*, cplx<float>*, cplx<float>*, BpStatus*, void*, int,
+                             hipStream_t);
+template void gemm_bp<double>(ClassView, int, const cplx<double>*, cplx<double>*, cplx<double>*, BpStatus*, void*,
+                              int, hipStream_t);
+template void gemm_ext<float>(ClassView, int, const cplx<float>*, const cplx<float>*, cplx<double>*, void*, int,
+                              hipStream_t);
+template void gemm_ext<double>(ClassView, int, const cplx<double>*, const cplx<double>*, cplx<double>*, void*, int,
+                               hipStream_t);
+
+}  // namespace bqa
