@@ -16,7 +16,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
-SOURCES = ("bqa_api.hip", "node_gemm.hip")
+SOURCES = ("bqa_api.hip", "node_gemm.hip", "canon_wide.hip")
 OUT = os.path.join(HERE, "libbqa_hip.so")
 ARCH = os.environ.get("BQA_OFFLOAD_ARCH", "gfx950")
 

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/bqa_hip.h"
+#include "canon_wide.hpp"
 #include "common.hpp"
 #include "kernels_canon.hpp"
 #include "kernels_canon_h.hpp"
@@ -956,7 +957,12 @@ void canonicalise(bqa_job* j, double pinv_eps, bool sync) {
   canon_outputs(j);
   const size_t wsb = canon_ws_bytes(n2);
   const double deps = canon_deps(j);
-  if (j->generic(kGenCanon) || !canon_reg_dispatch(j, chi, ccols, pinv_eps, deps)) {
+  if (!j->generic(kGenCanon) && canon_wide_shape(chi)) {
+    j->cws.ensure(canon_wide_ws_bytes(j->E, chi), j->dev_bytes, j->stream);
+    canon_wide(reinterpret_cast<const cplx<double>*>(j->ext.p), j->E, chi, ccols, pinv_eps, deps,
+               reinterpret_cast<zd*>(j->canon.p), reinterpret_cast<double*>(j->lmbd.p), j->cws.p, j->stream);
+    LAUNCH_CHECK();
+  } else if (j->generic(kGenCanon) || !canon_reg_dispatch(j, chi, ccols, pinv_eps, deps)) {
     int grid;
     size_t lds;
     unsigned char* ws = nullptr;

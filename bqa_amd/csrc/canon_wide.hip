@@ -1,0 +1,464 @@
+// Canonicalisers and lambdas for n = 2 chi = 34..64, one edge per block of four waves.
+//
+// The algorithm is k_canon_h's (kernels_canon_h.hpp): the Hermitian extended messages are factored by
+// pivoted Cholesky, one-sided Jacobi on the factor gives their eigenbases without accumulating
+// rotations, and the bond matrix K is diagonalised the same way.  At n = 64 a matrix is 64 KB, so the
+// columns live in LDS instead of in one wave's registers: eight lanes share a pair of columns
+// (every eighth row each), a dot product is eight rows and three DPP steps, and a round ends with
+// one barrier.  The Cholesky keeps its two columns per lane group in registers and passes only the
+// pivot column through LDS.  What bounds it is the LDS traffic of the Jacobi rounds (a round reads and
+// writes the whole matrix, 128 KB at n = 64, against 640 cycles of FP64 arithmetic a wave).
+#include "canon_wide.hpp"
+
+#include <algorithm>
+
+namespace bqa {
+
+namespace {
+
+using zd = cplx<double>;
+
+constexpr int kWideThreads = 256;
+
+// Value of lane ^ M within eight lanes: quad permutations for 1 and 2, half-row mirror (^ 7) then ^ 3 for 4.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double sum8(double v) {
+  v += dpp_move<0xB1>(v);
+  v += dpp_move<0x4E>(v);
+  v += dpp_move<0x1B>(dpp_move<0x141>(v));
+  return v;
+}
+
+struct WideShared {
+  double dg[64], sqf[64], ipf[64], sqb[64], ipb[64], norm[64], il[64];
+  zd lcol[64];
+  int rank_of[64], col_of[64];
+  double red[4];
+  int rotated[3], unsettled[3];
+};
+
+__device__ __forceinline__ double block_max4(double v, double* red) {
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
+// Columns of the stride: eight lanes read 128 neighbouring bytes, and the next column's land in the
+// other half of the banks.
+template <int NR>
+constexpr int wide_ld() {
+  return NR % 16 == 8 ? NR : NR + 8;
+}
+
+// Pivoted Cholesky of the Hermitian part of M (n x n, row-major) into A's columns: column j holds a
+// column of L, or zero beyond the numerical rank.
+template <int NR>
+__device__ void wide_cholesky(const zd* __restrict__ M, int n, zd* A, WideShared& sh) {
+  constexpr int RPL = NR / 8, LD = wide_ld<NR>();
+  const int t = threadIdx.x, pair = t >> 3, l8 = t & 7, lane = t & 63;
+  const bool active = pair < n / 2;
+  const int ct = pair, cb = n - 1 - pair;
+  zd top[RPL], bot[RPL];
+#pragma unroll
+  for (int x = 0; x < RPL; ++x) {
+    const int r = l8 + 8 * x;
+    top[x] = bot[x] = mk(0.0, 0.0);
+    if (active && r < n) {
+      const zd a = M[r * n + ct], at = M[ct * n + r], b = M[r * n + cb], bt = M[cb * n + r];
+      top[x] = mk(0.5 * (a.x + at.x), 0.5 * (a.y - at.y));
+      bot[x] = mk(0.5 * (b.x + bt.x), 0.5 * (b.y - bt.y));
+    }
+  }
+  if (t < 64) sh.dg[t] = t < n ? M[t * n + t].x : -1.0;
+  __syncthreads();
+  bool dt = !active, db = !active;
+  double d0 = 0.0;
+#pragma unroll 1
+  for (int step = 0; step < n; ++step) {
+    // every wave finds the largest undone diagonal (ties to the lower column)
+    double bv = sh.dg[lane];
+    int bc = lane;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double ov = __shfl_xor(bv, o, 64);
+      const int oc = __shfl_xor(bc, o, 64);
+      if (ov > bv || (ov == bv && oc < bc)) {
+        bv = ov;
+        bc = oc;
+      }
+    }
+    if (step == 0) d0 = bv;
+    if (!(bv > 1e-20 * d0)) break;   // the same in every wave; also for a NaN
+    const double inv = 1.0 / sqrt(bv);
+    const bool pt = active && bc == ct, pb = active && bc == cb;
+    if (pt || pb) {
+#pragma unroll
+      for (int x = 0; x < RPL; ++x) sh.lcol[l8 + 8 * x] = scale(pt ? top[x] : bot[x], inv);
+    }
+    __syncthreads();
+    if (active) {
+      const zd lt = sh.lcol[ct], lb = sh.lcol[cb];
+      const double at = pt ? inv : 1.0, ab = pb ? inv : 1.0;
+      const double ut = (!dt && !pt) ? 1.0 : 0.0, ub = (!db && !pb) ? 1.0 : 0.0;
+      const double ltr = ut * lt.x, lti = ut * lt.y, lbr = ub * lb.x, lbi = ub * lb.y;
+#pragma unroll
+      for (int x = 0; x < RPL; ++x) {
+        const zd l = sh.lcol[l8 + 8 * x];
+        top[x].x = fma(at, top[x].x, -fma(l.x, ltr, l.y * lti));
+        top[x].y = fma(at, top[x].y, -fma(l.y, ltr, -(l.x * lti)));
+        bot[x].x = fma(ab, bot[x].x, -fma(l.x, lbr, l.y * lbi));
+        bot[x].y = fma(ab, bot[x].y, -fma(l.y, lbr, -(l.x * lbi)));
+      }
+      if (l8 == 0) {
+        if (pt)
+          sh.dg[ct] = -1.0;
+        else if (!dt)
+          sh.dg[ct] -= fma(ltr, ltr, lti * lti);
+        if (pb)
+          sh.dg[cb] = -1.0;
+        else if (!db)
+          sh.dg[cb] -= fma(lbr, lbr, lbi * lbi);
+      }
+      dt = dt || pt;
+      db = db || pb;
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  if (active) {
+#pragma unroll
+    for (int x = 0; x < RPL; ++x) {
+      const int r = l8 + 8 * x;
+      A[ct * LD + r] = dt ? top[x] : mk(0.0, 0.0);
+      A[cb * LD + r] = db ? bot[x] : mk(0.0, 0.0);
+    }
+  }
+  __syncthreads();
+}
+
+// Squared norm of a column over its eight lanes.
+template <int NR>
+__device__ __forceinline__ double wide_norm2(const zd* col, int l8) {
+  double s = 0.0;
+#pragma unroll
+  for (int x = 0; x < NR / 8; ++x) {
+    const zd v = col[l8 + 8 * x];
+    s = fma(v.x, v.x, fma(v.y, v.y, s));
+  }
+  return sum8(s);
+}
+
+// One-sided Jacobi on the n columns of A in a round-robin order, with the thresholds of
+// hjacobi_round (kernels_canon_h.hpp).
+template <int NR>
+__device__ void wide_jacobi(zd* A, int n, WideShared& sh) {
+  constexpr int RPL = NR / 8, LD = wide_ld<NR>();
+  constexpr double kSettledCos2 = 1e-16, kSettledSin2 = 1e-12;
+  const int t = threadIdx.x, pair = t >> 3, l8 = t & 7;
+  const bool active = pair < n / 2;
+  double sc = 0.0;
+  if (active)
+    sc = fmax(wide_norm2<NR>(A + (2 * pair) * LD, l8), wide_norm2<NR>(A + (2 * pair + 1) * LD, l8));
+  const double small2 = 1e-26 * block_max4(sc, sh.red);
+  const double tol = 2.2204460492503131e-16 * n;
+  if (t < 3) sh.rotated[t] = sh.unsettled[t] = 0;
+  __syncthreads();
+#pragma unroll 1
+  for (int sweep = 0; sweep < 30; ++sweep) {
+    // flags of the next sweep: last read two sweeps ago
+    if (t == 0) sh.rotated[(sweep + 1) % 3] = sh.unsettled[(sweep + 1) % 3] = 0;
+#pragma unroll 1
+    for (int round = 0; round < n - 1; ++round) {
+      if (active) {
+        const int m = n - 1;
+        int p = 0, q = n - 2 - pair + round;
+        if (pair > 0) {
+          p = pair - 1 + round;
+          p = (p >= m ? p - m : p) + 1;
+        }
+        q = (q >= m ? q - m : q) + 1;
+        zd* cp = A + p * LD + l8;
+        zd* cq = A + q * LD + l8;
+        zd u[RPL], v[RPL];
+        double a = 0.0, b = 0.0, gr = 0.0, gi = 0.0;
+#pragma unroll
+        for (int x = 0; x < RPL; ++x) {
+          u[x] = cp[8 * x];
+          v[x] = cq[8 * x];
+        }
+#pragma unroll
+        for (int x = 0; x < RPL; ++x) {
+          a = fma(u[x].x, u[x].x, fma(u[x].y, u[x].y, a));
+          b = fma(v[x].x, v[x].x, fma(v[x].y, v[x].y, b));
+          gr = fma(u[x].x, v[x].x, fma(u[x].y, v[x].y, gr));
+          gi = fma(u[x].x, v[x].y, fma(-u[x].y, v[x].x, gi));
+        }
+        a = sum8(a);
+        b = sum8(b);
+        gr = sum8(gr);
+        gi = sum8(gi);
+        const double g2 = gr * gr + gi * gi;
+        if (fmin(a, b) >= small2 && g2 > tol * tol * a * b) {
+          const double rga = rsqrt(g2);
+          const double zeta = 0.5 * (b - a) * rga;
+          const double w = fabs(zeta) + sqrt(fma(zeta, zeta, 1.0));
+          const double tt = (zeta >= 0.0 ? 1.0 : -1.0) / w;
+          const double c = rsqrt(fma(tt, tt, 1.0));
+          const double s = c * tt;
+          const double er = gr * rga, ei = -gi * rga;
+          if (l8 == 0) {
+            sh.rotated[sweep % 3] = 1;
+            if (g2 > kSettledCos2 * a * b || s * s > kSettledSin2) sh.unsettled[sweep % 3] = 1;
+          }
+#pragma unroll
+          for (int x = 0; x < RPL; ++x) {
+            const double xr = er * v[x].x - ei * v[x].y;
+            const double xi = er * v[x].y + ei * v[x].x;
+            cq[8 * x] = mk(s * u[x].x + c * xr, s * u[x].y + c * xi);
+            cp[8 * x] = mk(c * u[x].x - s * xr, c * u[x].y - s * xi);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (!sh.rotated[sweep % 3] || !sh.unsettled[sweep % 3]) break;
+  }
+  __syncthreads();
+}
+
+template <int NR>
+__global__ __launch_bounds__(kWideThreads) void k_canon_wide(const zd* __restrict__ ext, int E, int n, int ccols,
+                                                             double pinv_eps, double deps, zd* __restrict__ canon,
+                                                             double* __restrict__ lfull, zd* __restrict__ ws) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int RPL = NR / 8, LD = wide_ld<NR>();
+  zd* A = reinterpret_cast<zd*>(smem_raw);
+  WideShared& sh = *reinterpret_cast<WideShared*>(smem_raw + sizeof(zd) * LD * NR);
+  const int t = threadIdx.x, pair = t >> 3, l8 = t & 7;
+  const int nn = n * n;
+  zd* Uf = ws + (size_t)blockIdx.x * 2 * nn;
+  zd* Ub = Uf + nn;
+  const int a0 = 4 * (t >> 4), c0 = 2 * (t & 15);   // the products below: 4 rows x 2 columns a thread
+
+  for (int edge = blockIdx.x; edge < E; edge += gridDim.x) {
+    for (int side = 0; side < 2; ++side) {
+      wide_cholesky<NR>(ext + (size_t)(side ? E + edge : edge) * nn, n, A, sh);
+      wide_jacobi<NR>(A, n, sh);
+      // columns are V_M sigma: eigenvalue s = sigma^2, U = column / sigma
+      zd* U = side ? Ub : Uf;
+      if (pair < n / 2) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int j = 2 * pair + h;
+          const double sig = sqrt(wide_norm2<NR>(A + j * LD, l8));
+          const double sqv = sig * sig > pinv_eps ? sig : 0.0;
+          if (l8 == 0) {
+            (side ? sh.sqb : sh.sqf)[j] = sqv;
+            (side ? sh.ipb : sh.ipf)[j] = sqv > deps ? 1.0 / sqv : 0.0;
+          }
+          const double inv = sig > 0.0 ? 1.0 / sig : 0.0;
+#pragma unroll
+          for (int x = 0; x < RPL; ++x) {
+            const int r = l8 + 8 * x;
+            if (r < n) U[j * n + r] = scale(A[j * LD + r], inv);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    // K[i][j] = sq_f[i] sq_b[j] conj(sum_t U_f[t, i] U_b[t, j]), a 4 x 4 block a thread; K's columns to A
+    // (rows n .. NR stay zero)
+    {
+      const int i0 = 4 * (t >> 4), j0 = 4 * (t & 15);
+      if (i0 < n && j0 < n) {
+        double ar[4][4] = {}, ai[4][4] = {};
+        const int imax = n - 1 - i0, jmax = n - 1 - j0;
+        for (int x = 0; x < n; ++x) {
+          zd f[4], b[4];
+#pragma unroll
+          for (int y = 0; y < 4; ++y) {
+            f[y] = Uf[(i0 + (y < imax ? y : imax)) * n + x];
+            b[y] = Ub[(j0 + (y < jmax ? y : jmax)) * n + x];
+          }
+#pragma unroll
+          for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+              ar[y][z] = fma(f[y].x, b[z].x, fma(-f[y].y, b[z].y, ar[y][z]));
+              ai[y][z] = fma(f[y].x, b[z].y, fma(f[y].y, b[z].x, ai[y][z]));
+            }
+        }
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+          for (int z = 0; z < 4; ++z)
+            if (y <= imax && z <= jmax) {
+              const double w = sh.sqf[i0 + y] * sh.sqb[j0 + z];
+              A[(j0 + z) * LD + i0 + y] = mk(w * ar[y][z], -w * ai[y][z]);
+            }
+      }
+    }
+    __syncthreads();
+    wide_jacobi<NR>(A, n, sh);
+
+    // singular values, descending ranks, masks, normalised lambdas
+    if (pair < n / 2) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double s = sqrt(wide_norm2<NR>(A + (2 * pair + h) * LD, l8));
+        if (l8 == 0) sh.norm[2 * pair + h] = s;
+      }
+    }
+    __syncthreads();
+    if (t < n) {
+      const double s = sh.norm[t];
+      int rank = 0;
+      double nrm2 = 0.0;
+      for (int j = 0; j < n; ++j) {
+        const double o = sh.norm[j];
+        rank += (o > s || (o == s && j < t)) ? 1 : 0;
+        nrm2 += o > pinv_eps ? o * o : 0.0;
+      }
+      const bool keep = s > pinv_eps;
+      sh.col_of[rank] = t;
+      sh.il[rank] = keep ? 1.0 / s : 0.0;
+      lfull[(size_t)edge * n + rank] = (keep ? s : 0.0) / sqrt(nrm2);
+    }
+    __syncthreads();
+    // with Us the masked left vectors of K (its columns over Lambda, by rank):
+    // V = U_f diag(sq_f) Us and C_f = U_f diag(ip_f) Us
+    zd* Cb = canon + (size_t)edge * n * ccols;
+    zd* Cf = canon + (size_t)(E + edge) * n * ccols;
+    const bool mine = a0 < n && c0 < ccols;
+    const int amax = n - 1 - a0;                     // clamps the rows of a partial block
+    double xr[4][2] = {}, xi[4][2] = {}, yr[4][2] = {}, yi[4][2] = {};
+    if (mine) {
+      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+      const zd* k0 = A + sh.col_of[c0] * LD;
+      const zd* k1 = A + sh.col_of[c1] * LD;
+      const double l0 = sh.il[c0], l1 = sh.il[c1];
+      for (int x = 0; x < n; ++x) {
+        const zd us[2] = {scale(k0[x], l0), scale(k1[x], l1)};
+        const double sq = sh.sqf[x], ip = sh.ipf[x];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const zd f = Uf[x * n + a0 + (y < amax ? y : amax)];
+#pragma unroll
+          for (int z = 0; z < 2; ++z) {
+            const double sr = sq * us[z].x, si = sq * us[z].y, pr = ip * us[z].x, pi = ip * us[z].y;
+            xr[y][z] = fma(f.x, sr, fma(-f.y, si, xr[y][z]));
+            xi[y][z] = fma(f.x, si, fma(f.y, sr, xi[y][z]));
+            yr[y][z] = fma(f.x, pr, fma(-f.y, pi, yr[y][z]));
+            yi[y][z] = fma(f.x, pi, fma(f.y, pr, yi[y][z]));
+          }
+        }
+      }
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          if (y <= amax && c0 + z < ccols) Cf[(a0 + y) * ccols + c0 + z] = mk(yr[y][z], yi[y][z]);
+    }
+    __syncthreads();
+    zd* V = A;   // V[c][a]
+    if (mine) {
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          if (y <= amax && c0 + z < ccols) V[(c0 + z) * LD + a0 + y] = mk(xr[y][z], xi[y][z]);
+    }
+    __syncthreads();
+    // Z[c][j] = keep_b[j] conj(sum_u U_b[u, j] V[u, c]) / Lambda_c
+    double zr[4][2] = {}, zi[4][2] = {};
+    if (mine) {
+      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+      for (int x = 0; x < n; ++x) {
+        const zd v[2] = {V[c0 * LD + x], V[c1 * LD + x]};
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const zd b = Ub[(a0 + (y < amax ? y : amax)) * n + x];
+#pragma unroll
+          for (int z = 0; z < 2; ++z) {
+            zr[y][z] = fma(b.x, v[z].x, fma(-b.y, v[z].y, zr[y][z]));
+            zi[y][z] = fma(b.x, v[z].y, fma(b.y, v[z].x, zi[y][z]));
+          }
+        }
+      }
+    }
+    __syncthreads();
+    zd* Z = A;   // Z[c][j]
+    if (mine) {
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          if (y <= amax && c0 + z < ccols) {
+            const double w = sh.ipb[a0 + y] > 0.0 ? sh.il[c0 + z] : 0.0;
+            Z[(c0 + z) * LD + a0 + y] = mk(zr[y][z] * w, -zi[y][z] * w);
+          }
+    }
+    __syncthreads();
+    // C_b[a][c] = sum_j U_b[a, j] Z[c][j]
+    if (mine) {
+      double br[4][2] = {}, bi[4][2] = {};
+      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+      for (int x = 0; x < n; ++x) {
+        const zd z[2] = {Z[c0 * LD + x], Z[c1 * LD + x]};
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const zd b = Ub[x * n + a0 + (y < amax ? y : amax)];
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            br[y][q] = fma(b.x, z[q].x, fma(-b.y, z[q].y, br[y][q]));
+            bi[y][q] = fma(b.x, z[q].y, fma(b.y, z[q].x, bi[y][q]));
+          }
+        }
+      }
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          if (y <= amax && c0 + q < ccols) Cb[(a0 + y) * ccols + c0 + q] = mk(br[y][q], bi[y][q]);
+    }
+    __syncthreads();
+  }
+}
+
+template <int NR>
+void launch_wide(const zd* ext, int E, int n, int ccols, double pinv_eps, double deps, zd* canon, double* lambdas,
+                 zd* ws, hipStream_t s) {
+  constexpr int lds = sizeof(zd) * wide_ld<NR>() * NR + sizeof(WideShared);
+  static const bool once = [] {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_canon_wide<NR>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+  }();
+  (void)once;   // a refusal shows as the launch's own error
+  hipLaunchKernelGGL((k_canon_wide<NR>), dim3(std::min(E, kCanonWideBlocks)), dim3(kWideThreads), lds, s, ext, E, n,
+                     ccols, pinv_eps, deps, canon, lambdas, ws);
+}
+
+}  // namespace
+
+void canon_wide(const zd* ext, int E, int chi, int ccols, double pinv_eps, double dtype_eps, zd* canon,
+                double* lambdas, void* ws, hipStream_t s) {
+  const int n = 2 * chi;
+  zd* w = reinterpret_cast<zd*>(ws);
+  if (n <= 40)
+    launch_wide<40>(ext, E, n, ccols, pinv_eps, dtype_eps, canon, lambdas, w, s);
+  else if (n <= 48)
+    launch_wide<48>(ext, E, n, ccols, pinv_eps, dtype_eps, canon, lambdas, w, s);
+  else if (n <= 56)
+    launch_wide<56>(ext, E, n, ccols, pinv_eps, dtype_eps, canon, lambdas, w, s);
+  else
+    launch_wide<64>(ext, E, n, ccols, pinv_eps, dtype_eps, canon, lambdas, w, s);
+}
+
+}  // namespace bqa

@@ -1,0 +1,22 @@
+// Canonicalisers for bond dimensions 17..32 (n = 2 chi = 34..64): host interface of canon_wide.hip.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "common.hpp"
+
+namespace bqa {
+
+inline bool canon_wide_shape(int chi) { return chi >= 17 && chi <= 32; }
+
+// Blocks that run at once take the edges in turn, each with one workspace slot (the bases of both sides).
+constexpr int kCanonWideBlocks = 512;
+inline size_t canon_wide_ws_bytes(int E, int chi) {
+  const size_t blocks = E < kCanonWideBlocks ? E : kCanonWideBlocks;
+  return blocks * 2 * sizeof(cplx<double>) * 4 * chi * chi;
+}
+
+void canon_wide(const cplx<double>* ext, int E, int chi, int ccols, double pinv_eps, double dtype_eps,
+                cplx<double>* canon, double* lambdas, void* ws, hipStream_t s);
+
+}  // namespace bqa
