@@ -1017,6 +1017,17 @@ void local_update(bqa_job* j, int flags, int chi_out, double zz_time, double z_t
                               n2, ccols, zz_time, flags, z_time, x_time,
                               reinterpret_cast<const double*>(j->lmbd.p), j->lstride, msg_ptr<R>(j, j->mcur),
                               j->stream)) {
+      if (!j->generic(kGenLocal) && (flags & kAbsorb) && gemm_local_shape(c.d, chi_in, chi_out)) {
+        const int most = std::max(chi_in, chi_out), chunk = gemm_local_chunk(c.n, c.d, most);
+        const size_t need = (size_t)chunk * gemm_local_node_bytes(c.d, most);
+        if (need > j->gws.bytes) j->gws.ensure(need, j->dev_bytes, j->stream);
+        gemm_local<R>(v, chi_in, chi_out, Tin, Tout, reinterpret_cast<const zd*>(j->canon.p), ccols, zz_time, flags,
+                      z_time, x_time, reinterpret_cast<const double*>(j->lmbd.p), j->lstride, msg_ptr<R>(j, j->mcur),
+                      j->gws.p, chunk, j->stream);
+        LAUNCH_CHECK();
+        c.tcur = dst;
+        continue;
+      }
       const int cm = std::max(chi_in, chi_out);
       const long Smax = 2 * ipow_l(cm, c.d);
       NodeLaunch L = plan_node(j, c.n, sizeof(cplx<double>) * 2 * Smax, 0, 2 * Smax, sizeof(cplx<double>));

@@ -418,6 +418,133 @@ __global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_ext(ClassView cv, Ge
   }
 }
 
+// Fragments of the absorb operand of one physical half: W[c][a] = g0 C[c][a] + z g1 C[chi_in + c][a].
+template <int KS, int MT>
+__device__ __forceinline__ void absorb_frag(MatFrag<double, KS, MT>& w, const cplx<double>* __restrict__ C, int cols,
+                                            int chi_in, int chi_out, cplx<double> g0, cplx<double> gz) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  int al, ri;
+  tile_row<double>(r, al, ri);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int a = 8 * mt + al, c = 4 * ks + g;
+      cplx<double> v = mk(0.0, 0.0);
+      if (a < chi_out && c < chi_in) v = g0 * C[c * cols + a] + gz * C[(chi_in + c) * cols + a];
+      w.re[mt][ks] = ri == 0 ? v.x : v.y;
+      w.im[mt][ks] = ri == 0 ? -v.y : v.x;
+    }
+}
+
+// The absorb along bond k: block (node, physical half, part of the half's fibres).
+template <typename RS, int KS, int MT>
+__global__ __launch_bounds__(kGemmThreads) void k_gemm_absorb(ClassView cv, int k, int parts, int node0, int count,
+                                                              int chi_in, int chi_out, const cplx<RS>* __restrict__ src,
+                                                              long src_stride, cplx<double>* dst, long dst_stride,
+                                                              const cplx<double>* __restrict__ canon, int cols,
+                                                              double zz_time) {
+  int node, sub;
+  if (!node_item(blockIdx.x >> 3, 2 * parts, count, node, sub)) return;
+  const int p = sub / parts, part = sub % parts, i = node0 + node;
+  const int inner = ipow(chi_in, cv.d - 1 - k), half = ipow(chi_out, k) * inner;
+  cplx<double> g0, g1;
+  if (cv.zz) {
+    const cplx<double>* g = cv.zz + 2 * (size_t)cv.lmbd_pos[k * cv.n + i];
+    g0 = g[0];
+    g1 = g[1];
+  } else {
+    zz_split(cv.J[k * cv.n + i] * zz_time, g0, g1);
+  }
+  MatFrag<double, KS, MT> w;
+  absorb_frag<KS, MT>(w, canon + (size_t)cv.in_pos[k * cv.n + i] * 2 * chi_in * cols, cols, chi_in, chi_out, g0,
+                      p ? mk(-g1.x, -g1.y) : g1);
+  product_tiles<double, RS, KS, MT>(w, src + (size_t)node * src_stride, dst + (size_t)node * dst_stride, chi_in,
+                                    chi_out, inner, p * half, (p + 1) * half,
+                                    part * kGemmWaves + (threadIdx.x >> 6), parts * kGemmWaves);
+}
+
+constexpr int kGaugeThreads = 512;
+
+// Z and X gates, symmetric gauge, node normalisation and message re-initialisation of absorbed tensors
+// (state.py:142-156, 219-227), a block per node: the norm in a first pass over the tensor, the scaled
+// values in a second (a node's FP64 tensor is larger than the registers, and L2 still has it).  LDS: the
+// products of sqrt(lambda) over the last two bonds, then sqrt(lambda) of every bond.
+template <typename R>
+__global__ __launch_bounds__(kGaugeThreads) void k_gemm_gauge(ClassView cv, int node0, int chi,
+                                                              const cplx<double>* __restrict__ X, long stride,
+                                                              cplx<R>* __restrict__ Tout, int flags, double z_time,
+                                                              double x_time, const double* __restrict__ lmbd,
+                                                              int lstride, cplx<R>* msgs_init) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double shred[16];
+  double* low = reinterpret_cast<double*>(smem_raw);
+  const int d = cv.d, n = cv.n, t = threadIdx.x, i = node0 + blockIdx.x, cc = chi * chi;
+  double* root = low + cc;
+  const int A = ipow(chi, d);
+  const cplx<double>* x0 = X + (size_t)blockIdx.x * stride;
+  const cplx<double>* x1 = x0 + A;
+  const bool gates = flags & kGates, gauge = flags & kGauge;
+  if (gauge) {
+    for (int q = t; q < d * chi; q += kGaugeThreads)
+      root[q] = sqrt(lmbd[(size_t)cv.lmbd_pos[(q / chi) * n + i] * lstride + q % chi]);
+    __syncthreads();
+    for (int q = t; q < cc; q += kGaugeThreads) low[q] = root[(d - 2) * chi + q / chi] * root[(d - 1) * chi + q % chi];
+    __syncthreads();
+  }
+  const double phi = gates ? cv.h[i] * z_time : 0.0;
+  const double cz = cos(phi), sz = sin(phi), cx = cos(x_time), sx = sin(x_time);
+  const cplx<double> f0 = mk(cz, -sz), f1 = mk(cz, sz);
+  auto values = [&](int a, cplx<double>& y0, cplx<double>& y1) {
+    y0 = x0[a];
+    y1 = x1[a];
+    if (gates) {
+      const cplx<double> t0 = y0 * f0, t1 = y1 * f1;
+      // (cos x) t - i (sin x) X t
+      y0 = mk(cx * t0.x + sx * t1.y, cx * t0.y - sx * t1.x);
+      y1 = mk(cx * t1.x + sx * t0.y, cx * t1.y - sx * t0.x);
+    }
+    if (gauge) {
+      int hi = a / cc;
+      double f = low[a - hi * cc];
+      for (int k = d - 3; k >= 0; --k) {
+        f *= root[k * chi + hi % chi];
+        hi /= chi;
+      }
+      y0 = scale(y0, f);
+      y1 = scale(y1, f);
+    }
+  };
+  double inv = 1.0;
+  if (gauge) {
+    double ss = 0.0;
+    for (int a = t; a < A; a += kGaugeThreads) {
+      cplx<double> y0, y1;
+      values(a, y0, y1);
+      ss += abs2(y0) + abs2(y1);
+    }
+    inv = 1.0 / sqrt(block_sum(ss, shred));
+  }
+  cplx<R>* out = Tout + (size_t)i * 2 * A;
+  for (int a = t; a < A; a += kGaugeThreads) {
+    cplx<double> y0, y1;
+    values(a, y0, y1);
+    out[a] = cast<R>(scale(y0, inv));
+    out[A + a] = cast<R>(scale(y1, inv));
+  }
+  if (!gauge) return;
+  for (int k = 0; k < d; ++k) {
+    const double* lam = lmbd + (size_t)cv.lmbd_pos[k * n + i] * lstride;
+    double tr = 0.0;
+    for (int a = 0; a < chi; ++a) tr += lam[a];
+    const size_t pos = cv.in_pos[k * n + i];
+    for (int o = t; o < cc; o += kGaugeThreads) {
+      const int a = o / chi, b = o % chi;
+      msgs_init[pos * cc + o] = mk<R>(a == b ? (R)(lam[a] / tr) : (R)0, (R)0);
+    }
+  }
+}
+
 // Calls f.template operator()<KS, MT>() with the tile counts of bond dimension chi.
 template <typename F>
 void by_chi(int chi, F&& f) {
@@ -457,6 +584,30 @@ void launch_products(const ClassView& cv, const GemmPlan& plan, int chi, int nod
       hipLaunchKernelGGL((k_gemm_product<R, RS, RM, KS, MT, BP>), grid, dim3(kGemmThreads), 0, s, cv, plan, level,
                          parts, node0, count, chi, T, mA, mB, st, ws);
     });
+  }
+}
+
+// The same with independent counts for the summed index (chi_in) and the rows (chi_out).
+template <int KS, typename F>
+void by_rows(int rows, F&& f) {
+  switch ((rows + 7) / 8) {
+    case 1: f.template operator()<KS, 1>(); break;
+    case 2: f.template operator()<KS, 2>(); break;
+    case 3: f.template operator()<KS, 3>(); break;
+    default: f.template operator()<KS, 4>(); break;
+  }
+}
+template <typename F>
+void by_chi_pair(int chi_in, int chi_out, F&& f) {
+  switch ((chi_in + 3) / 4) {
+    case 1: by_rows<1>(chi_out, f); break;
+    case 2: by_rows<2>(chi_out, f); break;
+    case 3: by_rows<3>(chi_out, f); break;
+    case 4: by_rows<4>(chi_out, f); break;
+    case 5: by_rows<5>(chi_out, f); break;
+    case 6: by_rows<6>(chi_out, f); break;
+    case 7: by_rows<7>(chi_out, f); break;
+    default: by_rows<8>(chi_out, f); break;
   }
 }
 
@@ -567,6 +718,39 @@ void gemm_ext(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msgs, cplx
   }
 }
 
+template <typename R>
+void gemm_local(ClassView cv, int chi_in, int chi_out, const cplx<R>* Tin, cplx<R>* Tout, const cplx<double>* canon,
+                int canon_cols, double zz_time, int flags, double z_time, double x_time, const double* lmbd,
+                int lstride, cplx<R>* msgs_init, void* ws, int chunk, hipStream_t s) {
+  const int d = cv.d, most = std::max(chi_in, chi_out);
+  const long S_in = 2L * ipow(chi_in, d), S = 2L * ipow(most, d);
+  cplx<double>* buf[2] = {reinterpret_cast<cplx<double>*>(ws), reinterpret_cast<cplx<double>*>(ws) + chunk * S};
+  for (int node0 = 0; node0 < cv.n; node0 += chunk) {
+    const int count = std::min(chunk, cv.n - node0);
+    for (int k = 0; k < d; ++k) {
+      const long half = (long)ipow(chi_out, k) * ipow(chi_in, d - 1 - k);
+      const int parts = product_parts(count, 2, half);
+      const dim3 grid((unsigned)(padded8(count) * 2 * parts));
+      by_chi_pair(chi_in, chi_out, [&]<int KS, int MT>() {
+        if (k == 0)
+          hipLaunchKernelGGL((k_gemm_absorb<R, KS, MT>), grid, dim3(kGemmThreads), 0, s, cv, k, parts, node0, count,
+                             chi_in, chi_out, Tin + node0 * S_in, S_in, buf[0], S, canon, canon_cols, zz_time);
+        else
+          hipLaunchKernelGGL((k_gemm_absorb<double, KS, MT>), grid, dim3(kGemmThreads), 0, s, cv, k, parts, node0,
+                             count, chi_in, chi_out, buf[(k + 1) & 1], S, buf[k & 1], S, canon, canon_cols, zz_time);
+      });
+    }
+    const size_t lds = sizeof(double) * (chi_out * chi_out + d * chi_out);
+    hipLaunchKernelGGL((k_gemm_gauge<R>), dim3(count), dim3(kGaugeThreads), lds, s, cv, node0, chi_out,
+                       buf[(d + 1) & 1], S, Tout, flags, z_time, x_time, lmbd, lstride, msgs_init);
+  }
+}
+
+template void gemm_local<float>(ClassView, int, int, const cplx<float>*, cplx<float>*, const cplx<double>*, int, double,
+                                int, double, double, const double*, int, cplx<float>*, void*, int, hipStream_t);
+template void gemm_local<double>(ClassView, int, int, const cplx<double>*, cplx<double>*, const cplx<double>*, int,
+                                 double, int, double, double, const double*, int, cplx<double>*, void*, int,
+                                 hipStream_t);
 template void gemm_bp<float>(ClassView, int, const cplx<float>*, cplx<float>*, cplx<float>*, BpStatus*, void*, int,
                              hipStream_t);
 template void gemm_bp<double>(ClassView, int, const cplx<double>*, cplx<double>*, cplx<double>*, BpStatus*, void*,

@@ -67,4 +67,32 @@ template <typename R>
 void gemm_ext(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msgs, cplx<double>* ext, void* ws, int chunk,
               hipStream_t s);
 
+// Absorb (every bond k: T <- sum_c T[.., c, ..] W_p[c][.], W_p = g0 C_k[c] + (-1)^p g1 C_k[chi_in + c]) in FP64,
+// one launch per bond, then one launch with the gates and the symmetric gauge (the flags of k_node_local).  It
+// serves node tensors of which k_node_local cannot keep two FP64 copies in 64 KB of LDS (with them, one block
+// does a node in one launch).
+inline bool gemm_local_shape(int d, int chi_in, int chi_out) {
+  const int most = chi_in > chi_out ? chi_in : chi_out;
+  if (!gemm_shape(d, most) || chi_in < 2 || chi_out < 1) return false;
+  long s = 2;
+  for (int k = 0; k < d; ++k) s *= most;
+  return 2 * s * (long)sizeof(cplx<double>) > 64 * 1024;
+}
+// Nodes per round: two FP64 tensors each, within kGemmBudget and within what 1,024 blocks of the generic kernel take.
+inline size_t gemm_local_node_bytes(int d, int chi) {
+  size_t s = 4 * sizeof(cplx<double>);
+  for (int k = 0; k < d; ++k) s *= chi;
+  return s;
+}
+inline int gemm_local_chunk(int n, int d, int chi) {
+  size_t c = kGemmBudget / gemm_local_node_bytes(d, chi);
+  if (c > 1024) c = 1024;
+  if (c >= (size_t)n) return n;
+  return c >= 8 ? (int)(c / 8 * 8) : c > 0 ? (int)c : 1;
+}
+template <typename R>
+void gemm_local(ClassView cv, int chi_in, int chi_out, const cplx<R>* Tin, cplx<R>* Tout, const cplx<double>* canon,
+                int canon_cols, double zz_time, int flags, double z_time, double x_time, const double* lmbd,
+                int lstride, cplx<R>* msgs_init, void* ws, int chunk, hipStream_t s);
+
 }  // namespace bqa

@@ -114,3 +114,35 @@ def test_messages_that_are_not_hermitian():
         job.close()
     want = _sweep(ctx, t, m)
     assert np.abs(got - want).max() < 1e-10 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("d,chi,chi_max,n", [(3, 8, 16, 10), (3, 11, 13, 4), (3, 12, 12, 20), (3, 16, 32, 4), (3, 31, 32, 4),
+                                             (4, 5, 7, 6), (4, 8, 9, 6), (5, 4, 5, 8), (5, 5, 8, 6), (6, 3, 4, 8)])
+def test_local_step_matches_generic(d, chi, chi_max, n, precision, monkeypatch):
+    """Tensors and messages after the absorb alone and after the whole local step, from the same canonicalisers."""
+    ctx, t, m = _state(d, n, chi, precision)
+    ctx.max_bond_dim = chi_max
+    got = []
+    for mask in ("", "l"):
+        monkeypatch.setenv("BQA_GENERIC_KERNELS", mask)
+        one = []
+        job = _job(ctx, t, m, precision)
+        try:
+            job.simple_update(0.2, 1e-6)
+            one.append(job.get_tensors(0))
+        finally:
+            job.close()
+        job = _job(ctx, t, m, precision)
+        try:
+            job.run_layer(0.3, 0.2, 1e-6, 1, 0.0, 0.0)
+            one += [job.get_tensors(0), job.get_messages()]
+        finally:
+            job.close()
+        got.append(one)
+    u = 6e-8 if precision == "single" else 1.2e-16
+    for k, (a, b) in enumerate(zip(*got)):
+        # FP64 sums of d chi terms in both, rounded once to the storage type; the messages come from one sweep of them
+        tol = u * 64 if precision == "single" else u * 64 * d * chi
+        assert a.shape == b.shape
+        assert np.abs(a - b).max() < (tol if k < 2 else 64 * tol) * np.abs(b).max()
