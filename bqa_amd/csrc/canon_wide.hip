@@ -9,6 +9,7 @@
 // pivot column through LDS.  What bounds it is the LDS traffic of the Jacobi rounds (a round reads and
 // writes the whole matrix, 128 KB at n = 64, against 640 cycles of FP64 arithmetic a wave).
 #include "canon_wide.hpp"
+#include "jacobi.hpp"
 
 #include <algorithm>
 
@@ -96,7 +97,7 @@ __device__ void wide_cholesky(const zd* __restrict__ M, int n, zd* A, WideShared
     }
     if (step == 0) d0 = bv;
     if (!(bv > 1e-20 * d0)) break;   // the same in every wave; also for a NaN
-    const double inv = 1.0 / sqrt(bv);
+    const double inv = rsqrt_pos(bv);
     const bool pt = active && bc == ct, pb = active && bc == cb;
     if (pt || pb) {
 #pragma unroll
@@ -206,23 +207,17 @@ __device__ void wide_jacobi(zd* A, int n, WideShared& sh) {
         gi = sum8(gi);
         const double g2 = gr * gr + gi * gi;
         if (fmin(a, b) >= small2 && g2 > tol * tol * a * b) {
-          const double rga = rsqrt(g2);
-          const double zeta = 0.5 * (b - a) * rga;
-          const double w = fabs(zeta) + sqrt(fma(zeta, zeta, 1.0));
-          const double tt = (zeta >= 0.0 ? 1.0 : -1.0) / w;
-          const double c = rsqrt(fma(tt, tt, 1.0));
-          const double s = c * tt;
-          const double er = gr * rga, ei = -gi * rga;
+          const JacobiStep j = jacobi_step(a, b, gr, gi, g2);
           if (l8 == 0) {
             sh.rotated[sweep % 3] = 1;
-            if (g2 > kSettledCos2 * a * b || s * s > kSettledSin2) sh.unsettled[sweep % 3] = 1;
+            if (g2 > kSettledCos2 * a * b || j.s * j.s > kSettledSin2) sh.unsettled[sweep % 3] = 1;
           }
 #pragma unroll
           for (int x = 0; x < RPL; ++x) {
-            const double xr = er * v[x].x - ei * v[x].y;
-            const double xi = er * v[x].y + ei * v[x].x;
-            cq[8 * x] = mk(s * u[x].x + c * xr, s * u[x].y + c * xi);
-            cp[8 * x] = mk(c * u[x].x - s * xr, c * u[x].y - s * xi);
+            const double xr = j.er * v[x].x - j.ei * v[x].y;
+            const double xi = j.er * v[x].y + j.ei * v[x].x;
+            cq[8 * x] = mk(j.s * u[x].x + j.c * xr, j.s * u[x].y + j.c * xi);
+            cp[8 * x] = mk(j.c * u[x].x - j.s * xr, j.c * u[x].y - j.s * xi);
           }
         }
       }

@@ -6,12 +6,14 @@
 //     (k, h) = k + P2 h holds rows [h n/2, (h+1) n/2) of the two columns of
 //     pair k, so a column dot product is a lane-local sum plus one DPP
 //     exchange with the other half (lane ^ P2);
-//   * when n/2 is a power of two the Jacobi sweep pairs columns in a recursive
-//     xor order (all top x bot pairs with only the bot columns moving by one
-//     lane-xor per round, then each half split in two by one re-layout, and
-//     so on: n - 1 rounds), so a round moves one column per lane, through the
-//     LDS crossbar (ds_bpermute) rather than VALU moves and selects; other n
-//     use a round-robin with DPP row shifts;
+//   * the Jacobi sweep pairs columns in a recursive xor order (all top x bot
+//     pairs with only the bot columns moving by one lane-xor per round, then
+//     each half split in two by one re-layout, and so on: 2 P2 - 1 rounds), so
+//     a round moves one column per lane, through the LDS crossbar
+//     (ds_bpermute) rather than VALU moves and selects; other n than powers of
+//     two are padded with zero columns, which never rotate, and each column
+//     carries its number (at n = 24 a round-robin's DPP moves and selects took
+//     twice the rest of a round; 31 padded rounds are cheaper than 23 of them);
 //   * the Hermitian PSD extended messages are factored M = L L^H by pivoted
 //     Cholesky first; one-sided Jacobi on the columns of L then converges in
 //     about half the sweeps of Jacobi on M and yields V_M Sigma_L directly,
@@ -22,6 +24,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "jacobi.hpp"
 
 namespace bqa {
 
@@ -41,18 +44,6 @@ template <int NH>
 struct HCol {
   double re[NH], im[NH];
 };
-
-__device__ __forceinline__ double dpp_from_next(double x) {  // value of lane + 1 (row_shl:1)
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x101, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x101, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double dpp_from_prev(double x) {  // value of lane - 1 (row_shr:1)
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x111, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x111, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
 
 // 32-bit DPP move within 16-lane rows (every source lane valid for the
 // patterns used here).
@@ -86,23 +77,6 @@ __device__ __forceinline__ double half_sum(double v) {
     return v + xor_lane<HCanon<N>::P2>(v);
 }
 
-template <int N>
-__device__ __forceinline__ void hrotate_owners(HCol<N / 2>& top, HCol<N / 2>& bot, int k) {
-  constexpr int P = N / 2, NH = N / 2;
-  if (P == 1) return;
-#pragma unroll
-  for (int r = 0; r < NH; ++r) {
-    const double xr = dpp_from_next(top.re[r]), xi = dpp_from_next(top.im[r]);
-    const double yr = dpp_from_prev(bot.re[r]), yi = dpp_from_prev(bot.im[r]);
-    const double tr = k == 0 ? top.re[r] : (k < P - 1 ? xr : bot.re[r]);
-    const double ti = k == 0 ? top.im[r] : (k < P - 1 ? xi : bot.im[r]);
-    bot.re[r] = k == 0 ? xr : yr;
-    bot.im[r] = k == 0 ? xi : yi;
-    top.re[r] = tr;
-    top.im[r] = ti;
-  }
-}
-
 template <int NH>
 __device__ __forceinline__ double hnorm2(const HCol<NH>& c) {
   double s = 0.0;
@@ -114,11 +88,10 @@ __device__ __forceinline__ double hnorm2(const HCol<NH>& c) {
 // One Jacobi round: rotate the pair of split columns held by this lane pair
 // (top, bot) so that they become orthogonal; `rotated` / `unsettled` collect
 // whether the round rotated at all and whether a rotation was still large.
-// With TRACK the squared column norms a, b are carried (exact at each sweep's
-// start, updated by the rotation's a - t|g|, b + t|g|, moved with their
-// columns), otherwise they are recomputed here.
-template <int N, bool TRACK>
-__device__ __forceinline__ void hjacobi_round(HCol<N / 2>& top, HCol<N / 2>& bot, double& a, double& b, bool active,
+// The squared column norms a, b are carried (exact at each sweep's start,
+// updated by the rotation's a - t|g|, b + t|g|, moved with their columns).
+template <int N>
+__device__ __forceinline__ void hjacobi_round(HCol<N / 2>& top, HCol<N / 2>& bot, double& a, double& b,
                                               double small2, double tol, int& rotated, int& unsettled) {
   constexpr int NH = N / 2;
   // A sweep whose rotations all had column cosine |g| / sqrt(a b) < 1e-8 and
@@ -127,51 +100,33 @@ __device__ __forceinline__ void hjacobi_round(HCol<N / 2>& top, HCol<N / 2>& bot
   // the sweep that would only confirm convergence is skipped; near-degenerate
   // pairs, where tiny cosines give large rotations, keep the full test.
   constexpr double kSettledCos2 = 1e-16, kSettledSin2 = 1e-12;
-  double gr = 0.0, gi = 0.0;
-  if constexpr (!TRACK) {
-    a = hnorm2(top);
-    b = hnorm2(bot);
-  }
+  double gr = 0.0, gi = 0.0, hr = 0.0, hi = 0.0;   // two chains each
 #pragma unroll
   for (int r = 0; r < NH; ++r) {
-    gr = fma(top.re[r], bot.re[r], fma(top.im[r], bot.im[r], gr));
-    gi = fma(top.re[r], bot.im[r], fma(-top.im[r], bot.re[r], gi));
+    gr = fma(top.re[r], bot.re[r], gr);
+    hr = fma(top.im[r], bot.im[r], hr);
+    gi = fma(top.re[r], bot.im[r], gi);
+    hi = fma(-top.im[r], bot.re[r], hi);
   }
-  if constexpr (!TRACK) {
-    a = half_sum<N>(a);
-    b = half_sum<N>(b);
-  }
-  gr = half_sum<N>(gr);
-  gi = half_sum<N>(gi);
+  gr = half_sum<N>(gr + hr);
+  gi = half_sum<N>(gi + hi);
   const double g2 = gr * gr + gi * gi;
-  if (active && fmin(a, b) >= small2 && g2 > tol * tol * a * b) {
+  const double ab = a * b;
+  if (fmin(a, b) >= small2 && g2 > tol * tol * ab) {
     rotated = 1;
-    // rotation parameters from reciprocal square roots (c^2 + s^2 = 1 to a few ulp)
-    const double rga = rsqrt(g2);
-    const double zeta = 0.5 * (b - a) * rga;
-    const double w = fabs(zeta) + sqrt(fma(zeta, zeta, 1.0));
-    double rw = __builtin_amdgcn_rcp(w);
-    rw = fma(fma(-w, rw, 1.0), rw, rw);
-    rw = fma(fma(-w, rw, 1.0), rw, rw);
-    const double t = zeta >= 0.0 ? rw : -rw;
-    const double c = rsqrt(fma(t, t, 1.0));
-    const double s = c * t;
-    const double er = gr * rga, ei = -gi * rga;
-    unsettled |= (g2 > kSettledCos2 * a * b || s * s > kSettledSin2) ? 1 : 0;
-    if constexpr (TRACK) {
-      const double tg = t * (g2 * rga);  // t |g|
-      a -= tg;
-      b += tg;
-    }
+    const JacobiStep j = jacobi_step(a, b, gr, gi, g2);
+    unsettled |= (g2 > kSettledCos2 * ab || j.s * j.s > kSettledSin2) ? 1 : 0;
+    a -= j.tg;
+    b += j.tg;
 #pragma unroll
     for (int r = 0; r < NH; ++r) {
-      const double xr = er * bot.re[r] - ei * bot.im[r];
-      const double xi = er * bot.im[r] + ei * bot.re[r];
+      const double xr = j.er * bot.re[r] - j.ei * bot.im[r];
+      const double xi = j.er * bot.im[r] + j.ei * bot.re[r];
       const double pr = top.re[r], pi = top.im[r];
-      bot.re[r] = s * pr + c * xr;
-      bot.im[r] = s * pi + c * xi;
-      top.re[r] = c * pr - s * xr;
-      top.im[r] = c * pi - s * xi;
+      bot.re[r] = j.s * pr + j.c * xr;
+      bot.im[r] = j.s * pi + j.c * xi;
+      top.re[r] = j.c * pr - j.s * xr;
+      top.im[r] = j.c * pi - j.s * xi;
     }
   }
 }
@@ -184,64 +139,62 @@ __device__ __forceinline__ double bperm(double x, int addr4) {
   return __hiloint2double(hi, lo);
 }
 
-// One-sided Jacobi on the columns held by the lane pairs of an edge.
+// One-sided Jacobi on the columns held by the lane pairs of an edge.  it, ib: the columns'
+// numbers (-1: padding), which move with them when n / 2 is no power of two.
 template <int N>
-__device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int k, bool active) {
+__device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int& it, int& ib, int k) {
   constexpr int NH = N / 2, P = N / 2, P2 = HCanon<N>::P2;
-  double sc = active ? fmax(half_sum<N>(hnorm2(top)), half_sum<N>(hnorm2(bot))) : 0.0;
+  double sc = fmax(half_sum<N>(hnorm2(top)), half_sum<N>(hnorm2(bot)));
 #pragma unroll
   for (int o = 1; o < P2; o <<= 1) sc = fmax(sc, __shfl_xor(sc, o, 64));
   const double small2 = 1e-26 * sc;
   const double tol = 2.2204460492503131e-16 * N;
+  const int lane = threadIdx.x & 63;
   for (int sweep = 0; sweep < 30; ++sweep) {
     int rotated = 0, unsettled = 0;
-    if constexpr (P == P2) {
-      // recursive xor order: in the phase of group size L the tops and the
-      // bots of each group of L lanes meet all pairs (bot at lane k holds the
-      // bot that started at lane k ^ gray(t) in round t, so round t moves it by
-      // the lowest set bit of t); the re-layout at bit L / 2 then leaves the
-      // pairs within each half for size L / 2: lanes with the bit clear take
-      // (own top, partner's top), lanes with it set (own bot, partner's bot)
-      const int lane = threadIdx.x & 63;
-      double a = half_sum<N>(hnorm2(top)), b = half_sum<N>(hnorm2(bot));
+    // recursive xor order: in the phase of group size L the tops and the
+    // bots of each group of L lanes meet all pairs (bot at lane k holds the
+    // bot that started at lane k ^ gray(t) in round t, so round t moves it by
+    // the lowest set bit of t); the re-layout at bit L / 2 then leaves the
+    // pairs within each half for size L / 2: lanes with the bit clear take
+    // (own top, partner's top), lanes with it set (own bot, partner's bot)
+    double a = half_sum<N>(hnorm2(top)), b = half_sum<N>(hnorm2(bot));
 #pragma unroll 1
-      for (int L = P; L >= 1; L >>= 1) {
+    for (int L = P2; L >= 1; L >>= 1) {
 #pragma unroll 1
-        for (int t = 0; t < L; ++t) {
-          if (t > 0) {
-            const int addr = 4 * (lane ^ (t & -t));
-#pragma unroll
-            for (int r = 0; r < NH; ++r) {
-              bot.re[r] = bperm(bot.re[r], addr);
-              bot.im[r] = bperm(bot.im[r], addr);
-            }
-            b = bperm(b, addr);
-          }
-          hjacobi_round<N, true>(top, bot, a, b, active, small2, tol, rotated, unsettled);
-        }
-        if (L > 1) {
-          const int m = L >> 1, addr = 4 * (lane ^ m);
-          const bool hi = (k & m) != 0;
+      for (int t = 0; t < L; ++t) {
+        if (t > 0) {
+          const int addr = 4 * (lane ^ (t & -t));
 #pragma unroll
           for (int r = 0; r < NH; ++r) {
-            const double fr = bperm(hi ? top.re[r] : bot.re[r], addr);
-            const double fi = bperm(hi ? top.im[r] : bot.im[r], addr);
-            top.re[r] = hi ? bot.re[r] : top.re[r];
-            top.im[r] = hi ? bot.im[r] : top.im[r];
-            bot.re[r] = fr;
-            bot.im[r] = fi;
+            bot.re[r] = bperm(bot.re[r], addr);
+            bot.im[r] = bperm(bot.im[r], addr);
           }
-          const double fn = bperm(hi ? a : b, addr);
-          a = hi ? b : a;
-          b = fn;
+          b = bperm(b, addr);
+          if constexpr (P != P2) ib = __builtin_amdgcn_ds_bpermute(addr, ib);
         }
+        hjacobi_round<N>(top, bot, a, b, small2, tol, rotated, unsettled);
       }
-    } else {
-#pragma unroll 1
-      for (int rnd = 0; rnd < N - 1; ++rnd) {
-        double a, b;
-        hjacobi_round<N, false>(top, bot, a, b, active, small2, tol, rotated, unsettled);
-        hrotate_owners<N>(top, bot, k);
+      if (L > 1) {
+        const int m = L >> 1, addr = 4 * (lane ^ m);
+        const bool hi = (k & m) != 0;
+#pragma unroll
+        for (int r = 0; r < NH; ++r) {
+          const double fr = bperm(hi ? top.re[r] : bot.re[r], addr);
+          const double fi = bperm(hi ? top.im[r] : bot.im[r], addr);
+          top.re[r] = hi ? bot.re[r] : top.re[r];
+          top.im[r] = hi ? bot.im[r] : top.im[r];
+          bot.re[r] = fr;
+          bot.im[r] = fi;
+        }
+        const double fn = bperm(hi ? a : b, addr);
+        a = hi ? b : a;
+        b = fn;
+        if constexpr (P != P2) {
+          const int fid = __builtin_amdgcn_ds_bpermute(addr, hi ? it : ib);
+          it = hi ? ib : it;
+          ib = fid;
+        }
       }
     }
     if (!__any(rotated) || !__any(unsettled)) break;
@@ -308,7 +261,7 @@ __device__ void hcholesky(HCol<N / 2>& top, HCol<N / 2>& bot, int k, int h, bool
     // pair holding column bc
     const int owner_k = bc < N / 2 ? bc : N - 1 - bc;
     const bool own_top = bc == owner_k;
-    const double inv = 1.0 / sqrt(bv);
+    const double inv = rsqrt_pos(bv);
     if (k == owner_k) {
 #pragma unroll
       for (int r = 0; r < NH; ++r)
@@ -325,25 +278,23 @@ __device__ void hcholesky(HCol<N / 2>& top, HCol<N / 2>& bot, int k, int h, bool
     // conj(l[j]) for this lane's two columns j
     const double2 lt = lcol[ct], lb = lcol[cb];
     wave_lds_sync();
-    // one in-place form for every column: R[:, j] <- a R[:, j] - l conj(b l[j]),
-    // with (a, b) = (1, 1) to update, (1 / sqrt(R[bc][bc]), 0) for the pivot
-    // column (which becomes l) and (1, 0) once done
+    // one in-place form for every column: R[:, j] <- R[:, j] - l conj(x), with x = l[j] to update,
+    // sqrt(R[bc][bc]) - 1 for the pivot column (sqrt(R[bc][bc]) l, which so becomes l) and 0 once done
     const bool pt = active && bc == ct, pb = active && bc == cb;
-    const double at = pt ? inv : 1.0, ab = pb ? inv : 1.0;
-    const double ut = (!dt && !pt) ? 1.0 : 0.0, ub = (!db && !pb) ? 1.0 : 0.0;
-    const double ltr = ut * lt.x, lti = ut * lt.y, lbr = ub * lb.x, lbi = ub * lb.y;
+    const double less1 = fma(bv, inv, -1.0);
+    const double ut = dt ? 0.0 : 1.0, ub = db ? 0.0 : 1.0;
+    const double ltr = pt ? less1 : ut * lt.x, lti = pt ? 0.0 : ut * lt.y;
+    const double lbr = pb ? less1 : ub * lb.x, lbi = pb ? 0.0 : ub * lb.y;
 #pragma unroll
     for (int r = 0; r < NH; ++r) {
-      const double tr = fma(l.re[r], ltr, l.im[r] * lti), ti = fma(l.im[r], ltr, -(l.re[r] * lti));
-      const double br = fma(l.re[r], lbr, l.im[r] * lbi), bi = fma(l.im[r], lbr, -(l.re[r] * lbi));
-      top.re[r] = fma(at, top.re[r], -tr);
-      top.im[r] = fma(at, top.im[r], -ti);
-      bot.re[r] = fma(ab, bot.re[r], -br);
-      bot.im[r] = fma(ab, bot.im[r], -bi);
+      top.re[r] = fma(-l.re[r], ltr, fma(-l.im[r], lti, top.re[r]));
+      top.im[r] = fma(-l.im[r], ltr, fma(l.re[r], lti, top.im[r]));
+      bot.re[r] = fma(-l.re[r], lbr, fma(-l.im[r], lbi, bot.re[r]));
+      bot.im[r] = fma(-l.im[r], lbr, fma(l.re[r], lbi, bot.im[r]));
     }
-    // the diagonal element's update: (l[j] conj(l[j])) in the form above
-    dgt = fma(1.0, dgt, -fma(ltr, ltr, lti * lti));
-    dgb = fma(1.0, dgb, -fma(lbr, lbr, lbi * lbi));
+    // the diagonal element's update (l[j] conj(l[j]) in the form above)
+    dgt = fma(-ltr, ltr, fma(-lti, lti, dgt));
+    dgb = fma(-lbr, lbr, fma(-lbi, lbi, dgb));
     dt = dt || pt;
     db = db || pb;
   }
@@ -372,8 +323,10 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   double* ipb = sqb + N;
   const int r0 = h * NH;
 
-  __shared__ double2 lslots[S::EPW * N];
-  double2* lcol = lslots + (lane / G) * N;
+  // pivot columns, one slot an edge; the slots' stride puts the edges' and halves' rows on different banks
+  constexpr int kSlot = N + 2;
+  __shared__ double2 lslots[S::EPW * kSlot];
+  double2* lcol = lslots + (lane / G) * kSlot;
   HCol<NH> top, bot;
   for (int side = 0; side < 2; ++side) {
     const int ct = k, cb = N - 1 - k;
@@ -410,7 +363,8 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       dgb = M[cb * N + cb].x;
     }
     hcholesky<N>(top, bot, k, h, active, dgt, dgb, lcol);
-    hjacobi<N>(top, bot, k, active);
+    int it = k < P ? 2 * k : -1, ib = k < P ? 2 * k + 1 : -1;
+    hjacobi<N>(top, bot, it, ib, k);
     // columns are V_M sigma: eigenvalue s = sigma^2, U = column / sigma
     double* U = side ? Ub : Uf;
     double* sq = side ? sqb : sqf;
@@ -419,8 +373,8 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
     for (int hh = 0; hh < 2; ++hh) {
       const HCol<NH>& c = hh ? bot : top;
       const double sig = sqrt(half_sum<N>(hnorm2(c)));
-      if (active) {
-        const int slot = 2 * k + hh;
+      const int slot = hh ? ib : it;
+      if (valid && slot >= 0) {
         const double s = sig * sig;
         const bool keep = s > pinv_eps;
         const double sqv = keep ? sig : 0.0;
@@ -476,13 +430,16 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       }
     }
   }
-  hjacobi<N>(top, bot, k, active);
+  int it = k < P ? 2 * k : -1, ib = k < P ? 2 * k + 1 : -1;
+  hjacobi<N>(top, bot, it, ib, k);
+  const bool realt = valid && it >= 0, realb = valid && ib >= 0;
 
-  // singular values, descending ranks, masks, normalised lambdas
-  const double lt = sqrt(half_sum<N>(hnorm2(top))), lb = sqrt(half_sum<N>(hnorm2(bot)));
+  // singular values, descending ranks (padding below every column), masks, normalised lambdas
+  const double nt = sqrt(half_sum<N>(hnorm2(top))), nb = sqrt(half_sum<N>(hnorm2(bot)));
+  const double lt = it >= 0 ? nt : -1.0, lb = ib >= 0 ? nb : -1.0;
   int rt = 0, rb = 0;
 #pragma unroll 1
-  for (int q = 0; q < P; ++q) {
+  for (int q = 0; q < P2; ++q) {
     const double ot = __shfl(lt, base + q, 64), ob = __shfl(lb, base + q, 64);
     const int st = 2 * q, sb = 2 * q + 1;
     rt += (ot > lt || (ot == lt && st < 2 * k)) ? 1 : 0;
@@ -492,22 +449,20 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   }
   const bool keept = lt > pinv_eps, keepb = lb > pinv_eps;
   const double mt = keept ? lt : 0.0, mb = keepb ? lb : 0.0;
-  double nn = (active && h == 0) ? mt * mt + mb * mb : 0.0;
+  double nn = h == 0 ? mt * mt + mb * mb : 0.0;
 #pragma unroll
   for (int o = 1; o < G; o <<= 1) nn += __shfl_xor(nn, o, 64);
   const double nrm = sqrt(nn);
-  if (active && h == 0) {
-    lfull[(size_t)edge * N + rt] = mt / nrm;
-    lfull[(size_t)edge * N + rb] = mb / nrm;
-  }
+  if (realt && h == 0) lfull[(size_t)edge * N + rt] = mt / nrm;
+  if (realb && h == 0) lfull[(size_t)edge * N + rb] = mb / nrm;
   // Stage the sorted, masked Us columns (Us[:, c] = K column / Lambda) and 1/Lambda.
   double* Q = wsE + 4 * N * N + 4 * N;         // Q[t][i] = sum_u U_b[u][t] U_f[u][i] sq_f[i]
   double* Us = Q + 2 * N * N;                  // Us[c][row], c = rank
   double* Zc = Us + 2 * N * N;                 // Z[c][j] = keep_b[j] conj(sum_i Q[j][i] Us[c][i]) / Lambda_c
   double* il = Zc + 2 * N * N;                 // 1 / Lambda_c (0 when masked)
-  if (active) {
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
+  for (int hh = 0; hh < 2; ++hh) {
+    if (hh ? realb : realt) {
       const HCol<NH>& c = hh ? bot : top;
       const int rank = hh ? rb : rt;
       const double inv = (hh ? keepb : keept) ? 1.0 / (hh ? lb : lt) : 0.0;
@@ -701,7 +656,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
 }
 
 template <int N>
-__global__ __launch_bounds__(64, N <= 16 ? 3 : 1) void k_canon_h(const cplx<double>* __restrict__ ext, int E, int ccols,
+__global__ __launch_bounds__(64, N <= 16 ? 3 : 2) void k_canon_h(const cplx<double>* __restrict__ ext, int E, int ccols,
                                                 double pinv_eps, double deps, zd* __restrict__ canon,
                                                 double* __restrict__ lfull, double* __restrict__ ws) {
   canon_h_run<N>(ext, E, ccols, pinv_eps, deps, canon, lfull, ws, blockIdx.x);
@@ -722,7 +677,7 @@ struct CanonEntry {
 // The canonicalisers of several jobs (same n) in one launch: entry e takes blocks
 // block0_e .. block0_{e+1} - 1 (found by binary search; block0 ascending, block0_0 = 0).
 template <int N>
-__global__ __launch_bounds__(64, N <= 16 ? 3 : 1) void k_canon_h_multi(const CanonEntry* __restrict__ tab,
+__global__ __launch_bounds__(64, N <= 16 ? 3 : 2) void k_canon_h_multi(const CanonEntry* __restrict__ tab,
                                                                       int entries) {
   int lo = 0, hi = entries - 1;
   while (lo < hi) {
