@@ -104,7 +104,7 @@ bool fast_ext_launch(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msg
     return true;
   }
   if (chi == 8 && cv.d == 4) {
-    launch_ext_d4c8m<R, 4>(cv, T, msgs, ext, s);
+    launch_ext_d4c8<R, 8>(cv, T, msgs, ext, s);
     return true;
   }
   if (chi == 8 && (cv.d == 2 || cv.d == 3)) {
@@ -154,14 +154,13 @@ inline void launch_mfma16_bp3h(ClassView cv, const cplx<float>* T, cplx<float>* 
 //   k_mfma16_bp3h<8> (three products per node, 96 KB LDS);
 //   chi = 16, d = 2: k_mfma16_bp<2, 1>, one or two resident rounds;
 //   chi = 8, d = 2, 3: k_mfma8 (one wave per node) under the three grid policies;
-//   chi = 8, d = 4: k_bp_d4c8 with 256 or 512 threads per node, k_bp_d4c8m (MFMA);
+//   chi = 8, d = 4: k_bp_d4c8, eight waves per node and two nodes per CU;
 //   other served shapes: k_small under the three grid policies, and for degree 2, 3 with chi <= 4
 //   also k_small_npw with 2 and 4 nodes per wave.
 template <>
 inline int bp_variant_count<float>(int d, int chi) {
   if (chi == 16 && d == 3) return 3;
   if (chi == 16 && d == 2) return 2;
-  if (chi == 8 && d == 4) return 3;
   if (chi == 8 && (d == 2 || d == 3)) return kGridPolicies;
   if (npw_shape(d, chi)) return kGridPolicies + 2;
   return small_bp_shape<float>(d, chi) ? kGridPolicies : 1;
@@ -172,8 +171,7 @@ inline const char* bp_variant_name<float>(int d, int chi, int v) {
   if (chi == 16 && d == 3)
     return v == 0 ? "k_mfma16_bp<3,8>" : v == 1 ? "k_mfma16_bp<3,4>" : "k_mfma16_bp3h<8> (three products)";
   if (chi == 16 && d == 2) return v == 0 ? "k_mfma16_bp<2,1>, resident" : "k_mfma16_bp<2,1>, 2x resident";
-  if (chi == 8 && d == 4)
-    return v == 0 ? "k_bp_d4c8<256 threads>" : v == 1 ? "k_bp_d4c8<512 threads>" : "k_bp_d4c8m (FP32 MFMA)";
+  if (chi == 8 && d == 4) return "k_bp_d4c8";
   static const char* m8[kGridPolicies] = {"k_mfma8, resident SIMD-rounded", "k_mfma8, resident",
                                           "k_mfma8, 2x resident"};
   static const char* sm[kGridPolicies + 2] = {"k_small, 8192 blocks", "k_small, resident", "k_small, 2x resident",
@@ -212,12 +210,7 @@ inline bool fast_bp_launch<float>(ClassView cv, int chi, const cplx<float>* T, c
     return v == kGridPolicies ? launch_small_npw<2, float>(cv, chi, T, mA, mB, st, s)
                               : launch_small_npw<4, float>(cv, chi, T, mA, mB, st, s);
   if (chi == 8 && cv.d == 4 && cv.n > 0) {
-    if (v == 2)
-      launch_bp_d4c8m(cv, T, mA, mB, st, s);
-    else if (v == 1)
-      launch_bp_d4c8<float, 512>(cv, T, mA, mB, st, s);
-    else
-      launch_bp_d4c8<float, 256>(cv, T, mA, mB, st, s);
+    launch_bp_d4c8<float, 8>(cv, T, mA, mB, st, s);
     return true;
   }
   if (chi != 8 || cv.n == 0 || (cv.d != 2 && cv.d != 3))
@@ -233,13 +226,11 @@ inline bool fast_bp_launch<float>(ClassView cv, int chi, const cplx<float>* T, c
 //   chi = 8, d = 3: k_mfma8_bp64_3p<4> (six contractions per node over four waves) under the three
 //     grid policies, and k_mfma8_bp64_3p<2> (two waves per node);
 //   chi = 8, d = 2: k_mfma8_bp64<2, 1> (one wave per node) under the three grid policies;
-//   chi = 8, d = 4: k_bp_d4c8 with 256 or 512 threads per node, and k_bp_d4c8m64 (FP64 MFMA) with
-//     four or eight waves per node;
+//   chi = 8, d = 4: k_bp_d4c8, sixteen waves per node (1.18 ms a sweep of 9,604 nodes; eight: 1.30 ms);
 //   other served shapes: k_small under the three grid policies, and for degree 2, 3 with chi <= 4
 //   also k_small_npw with 2 and 4 nodes per wave.
 template <>
 inline int bp_variant_count<double>(int d, int chi) {
-  if (chi == 8 && d == 4) return 4;
   if (chi == 8 && d == 3) return kGridPolicies + 1;
   if (chi == 8 && d == 2) return kGridPolicies;
   if (npw_shape(d, chi)) return kGridPolicies + 2;
@@ -256,9 +247,7 @@ inline const char* bp_variant_name<double>(int d, int chi, int v) {
   static const char* sm[kGridPolicies + 2] = {"k_small, 8192 blocks", "k_small, resident", "k_small, 2x resident",
                                               "k_small_npw<2> (2 nodes per wave), resident",
                                               "k_small_npw<4> (4 nodes per wave), resident"};
-  static const char* b4[4] = {"k_bp_d4c8<256 threads>", "k_bp_d4c8<512 threads>", "k_bp_d4c8m64<4 waves>",
-                              "k_bp_d4c8m64<8 waves>"};
-  if (chi == 8 && d == 4) return b4[v % 4];
+  if (chi == 8 && d == 4) return "k_bp_d4c8";
   if (chi == 16 && (d == 2 || d == 3)) return d == 3 ? "k_mfma16_bp64<3,8>" : "k_mfma16_bp64<2,1>";
   if (chi == 8 && d == 3) return b3[v % (kGridPolicies + 1)];
   if (chi == 8 && d == 2) return b2[v % kGridPolicies];
@@ -289,14 +278,7 @@ inline bool fast_bp_launch<double>(ClassView cv, int chi, const cplx<double>* T,
     return v == kGridPolicies ? launch_small_npw<2, double>(cv, chi, T, mA, mB, st, s)
                               : launch_small_npw<4, double>(cv, chi, T, mA, mB, st, s);
   if (chi == 8 && cv.d == 4 && cv.n > 0) {
-    if (v == 1)
-      launch_bp_d4c8<double, 512>(cv, T, mA, mB, st, s);
-    else if (v == 2)
-      launch_bp_d4c8m64<4>(cv, T, mA, mB, st, s);
-    else if (v == 3)
-      launch_bp_d4c8m64<8>(cv, T, mA, mB, st, s);
-    else
-      launch_bp_d4c8<double, 256>(cv, T, mA, mB, st, s);
+    launch_bp_d4c8<double, 16>(cv, T, mA, mB, st, s);
     return true;
   }
   if (chi != 8 || cv.n == 0 || (cv.d != 2 && cv.d != 3))
