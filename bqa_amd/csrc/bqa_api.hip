@@ -1169,6 +1169,13 @@ void density_impl(bqa_job* j, double* rho_out, double* bloch_out) {
       LAUNCH_CHECK();
       continue;
     }
+    if (!j->generic(kGenDensity) && gemm_shape(c.d, chi) && j->hermitian) {
+      const int chunk = plan_gemm(j, c, chi, sizeof(cplx<R>));
+      gemm_density<R>(c.view(), chi, T, msg_ptr<R>(j, j->mcur), reinterpret_cast<double*>(j->rho.p),
+                      reinterpret_cast<double*>(j->bloch.p), j->gws.p, chunk, j->stream);
+      LAUNCH_CHECK();
+      continue;
+    }
     const long S = 2 * ipow_l(chi, c.d);
     const size_t fixed = sizeof(cplx<R>) * (size_t)(kNT + 4 * chi * chi);
     NodeLaunch L = plan_node(j, c.n, sizeof(cplx<R>) * 3 * S, fixed, 3 * S, sizeof(cplx<R>));
@@ -1345,8 +1352,9 @@ size_t estimate(int N, int M, const std::vector<int>& deg, const std::vector<int
   // products of the matrix-product kernels, at the bond dimensions where they serve a class
   for (size_t c = 0; c < deg.size(); ++c)
     for (int chi = 1; chi <= std::min(chimax, kGemmMaxChi); ++chi) {
-      const bool fast = prec == BQA_PREC_SINGLE ? bp_fast_shape<float>(deg[c], chi) && ext_fast_shape<float>(deg[c], chi)
-                                                : bp_fast_shape<double>(deg[c], chi) && ext_fast_shape<double>(deg[c], chi);
+      const bool fast = density_fast_shape(deg[c], chi) &&
+                        (prec == BQA_PREC_SINGLE ? bp_fast_shape<float>(deg[c], chi) && ext_fast_shape<float>(deg[c], chi)
+                                                 : bp_fast_shape<double>(deg[c], chi) && ext_fast_shape<double>(deg[c], chi));
       if (size[c] > 0 && !fast && gemm_shape(deg[c], chi))
         gws = std::max(gws, (double)gemm_chunk(size[c], deg[c], chi, 16) * (double)gemm_node_bytes(deg[c], chi, 16));
     }

@@ -44,6 +44,9 @@ inline bool ext_fast_shape(int d, int chi) {
   return small_shape(d, chi) || (sizeof(R) == sizeof(float) && d == 5 && small_bp_shape<R>(5, chi));
 }
 
+// Shapes whose readout has one (fast_density_launch returns true for them).
+inline bool density_fast_shape(int d, int chi) { return small_shape(d, chi) || (chi == 8 && (d == 2 || d == 3)); }
+
 template <typename R>
 const char* bp_variant_name(int d, int chi, int v);
 

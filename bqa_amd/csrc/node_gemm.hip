@@ -560,6 +560,58 @@ void by_chi(int chi, F&& f) {
   }
 }
 
+// rho[p, q] = sum_a X[p, a] conj(Z[q, a]), trace one, and the Bloch vector by qubit id: a block per node, X the last
+// product of the first chain and Z of the second (the node tensor for an empty one).  Sums in FP64.
+template <typename R>
+__global__ __launch_bounds__(kGemmThreads) void k_gemm_density(ClassView cv, int node0, int chi, int x_at, int z_at,
+                                                               int products, const cplx<R>* __restrict__ T,
+                                                               const cplx<R>* __restrict__ ws, double* rho_out,
+                                                               double* bloch_out) {
+  __shared__ double part[8][kGemmWaves];
+  const int i = node0 + blockIdx.x, t = threadIdx.x;
+  const long A = ipow(chi, cv.d), S = 2 * A;
+  const cplx<R>* base = ws + (size_t)blockIdx.x * products * S;
+  const cplx<R>* X = x_at < 0 ? T + (size_t)i * S : base + x_at * S;
+  const cplx<R>* Z = z_at < 0 ? T + (size_t)i * S : base + z_at * S;
+  cplx<double> r[4] = {};
+#pragma unroll 4
+  for (long a = t; a < A; a += kGemmThreads) {
+    const cplx<double> x0 = cast<double>(X[a]), x1 = cast<double>(X[A + a]);
+    const cplx<double> z0 = cast<double>(Z[a]), z1 = cast<double>(Z[A + a]);
+    cfma_cj(r[0], z0, x0);
+    cfma_cj(r[1], z1, x0);
+    cfma_cj(r[2], z0, x1);
+    cfma_cj(r[3], z1, x1);
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    double v = q & 1 ? r[q >> 1].y : r[q >> 1].x;
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((t & 63) == 0) part[q][t >> 6] = v;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      v[q] = part[q][0];
+#pragma unroll
+      for (int w = 1; w < kGemmWaves; ++w) v[q] += part[q][w];
+    }
+    const cplx<double> inv = cinv(mk(v[0] + v[6], v[1] + v[7]));
+    const cplx<double> r00 = mk(v[0], v[1]) * inv, r01 = mk(v[2], v[3]) * inv;
+    const cplx<double> r10 = mk(v[4], v[5]) * inv, r11 = mk(v[6], v[7]) * inv;
+    const long id = cv.node_ids[i];
+    double* ro = rho_out + id * 8;
+    ro[0] = r00.x; ro[1] = r00.y; ro[2] = r01.x; ro[3] = r01.y;
+    ro[4] = r10.x; ro[5] = r10.y; ro[6] = r11.x; ro[7] = r11.y;
+    double* bo = bloch_out + id * 3;
+    bo[0] = r01.x + r10.x;
+    bo[1] = r10.y - r01.y;
+    bo[2] = r00.x - r11.x;
+  }
+}
+
 // Parts of a node's fibres: about eight tiles a wave to pay for the message fragments, fewer where
 // the launch would not give every CU four blocks.
 int product_parts(int count, int products, long fibres) {
@@ -746,6 +798,40 @@ void gemm_local(ClassView cv, int chi_in, int chi_out, const cplx<R>* Tin, cplx<
   }
 }
 
+template <typename R>
+void gemm_density(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msgs, double* rho, double* bloch, void* ws,
+                  int chunk, hipStream_t s) {
+  // two chains of products, level by level: the upper half of the bonds from the last one down, and the lower half
+  const int d = cv.d, low = d / 2;
+  GemmPlan plan{};
+  plan.d = d;
+  int last_low = -1, last_high = -1;
+  for (int l = 0; l < d - low; ++l) {
+    plan.first[l] = plan.products;
+    plan.src[plan.products] = (int8_t)last_high;
+    plan.bond[plan.products] = (int8_t)(d - 1 - l);
+    last_high = plan.products++;
+    if (l < low) {
+      plan.src[plan.products] = (int8_t)last_low;
+      plan.bond[plan.products] = (int8_t)(low - 1 - l);
+      last_low = plan.products++;
+    }
+    plan.levels = l + 1;
+    plan.first[l + 1] = plan.products;
+  }
+  cplx<R>* w = reinterpret_cast<cplx<R>*>(ws);
+  for (int node0 = 0; node0 < cv.n; node0 += chunk) {
+    const int count = std::min(chunk, cv.n - node0);
+    launch_products<R, R, R, false>(cv, plan, chi, node0, count, T, msgs, msgs, nullptr, w, s);
+    hipLaunchKernelGGL((k_gemm_density<R>), dim3(count), dim3(kGemmThreads), 0, s, cv, node0, chi, last_high, last_low,
+                       plan.products, T, w, rho, bloch);
+  }
+}
+
+template void gemm_density<float>(ClassView, int, const cplx<float>*, const cplx<float>*, double*, double*, void*, int,
+                                  hipStream_t);
+template void gemm_density<double>(ClassView, int, const cplx<double>*, const cplx<double>*, double*, double*, void*,
+                                   int, hipStream_t);
 template void gemm_local<float>(ClassView, int, int, const cplx<float>*, cplx<float>*, const cplx<double>*, int, double,
                                 int, double, double, const double*, int, cplx<float>*, void*, int, hipStream_t);
 template void gemm_local<double>(ClassView, int, int, const cplx<double>*, cplx<double>*, const cplx<double>*, int,

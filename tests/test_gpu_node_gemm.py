@@ -146,3 +146,23 @@ def test_local_step_matches_generic(d, chi, chi_max, n, precision, monkeypatch):
         tol = u * 64 if precision == "single" else u * 64 * d * chi
         assert a.shape == b.shape
         assert np.abs(a - b).max() < (tol if k < 2 else 64 * tol) * np.abs(b).max()
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("d,chi,n", [(2, 9, 7), (2, 16, 40), (2, 32, 3), (3, 9, 12), (3, 16, 10), (3, 32, 4), (4, 5, 14),
+                                     (4, 8, 30), (5, 4, 8), (5, 8, 20), (6, 3, 8)])
+def test_density_matches_oracle(d, chi, n, precision):
+    ctx, t, m = _state(d, n, chi, precision)
+    job = _job(ctx, t, m, precision)
+    try:
+        rho, bloch = job.density()
+    finally:
+        job.close()
+    (_, lay), = ctx.degree_to_layout.items()
+    want = np.empty((n, 2, 2), dtype=np.complex128)
+    want[lay.node_ids] = O.density_matrices(t, [m[lay.input_msgs_position[j]] for j in range(d)])
+    # d products of chi terms each in the job's precision, summed in FP64 to entries of order one
+    u = 6e-8 if precision == "single" else 1.2e-16
+    tol = u * (8 * d * chi + 64)
+    assert np.abs(rho - want).max() < tol
+    assert np.abs(bloch[:, 2] - (want[:, 0, 0] - want[:, 1, 1]).real).max() < 2 * tol
