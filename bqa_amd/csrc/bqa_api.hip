@@ -341,7 +341,11 @@ double sweep_bytes(const bqa_job* j, const ClassDev& c, int chi) {
          (double)c.n * c.d * 8.0;
 }
 
+// One block of kSweepSlots threads.
 __global__ void k_bp_reset(BpStatus* st, int cur, int max_iters, double bp_eps) {
+  st->slot[threadIdx.x][0] = 0ULL;
+  st->slot[threadIdx.x][1] = 0ULL;
+  if (threadIdx.x != 0) return;
   st->num_bits = 0ULL;
   st->den_bits = 0ULL;
   st->cur = cur;
@@ -353,10 +357,6 @@ __global__ void k_bp_reset(BpStatus* st, int cur, int max_iters, double bp_eps) 
   st->max_iters = max_iters;
   st->marker = 0;
   st->base = 0;
-  for (int k = 0; k < kSweepSlots && k < max_iters; ++k) {
-    st->slot[k][0] = 0ULL;
-    st->slot[k][1] = 0ULL;
-  }
   st->bp_eps = bp_eps;
   st->last_dist = 0.0;
   st->best_dist = INFINITY;
@@ -681,6 +681,11 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants) {
   return exec;
 }
 
+// Bytes of a status block with its first `sweeps` slots.
+size_t status_bytes(int sweeps) {
+  return offsetof(BpStatus, slot) + sizeof(BpStatus::slot[0]) * std::min(sweeps, kSweepSlots);
+}
+
 // The rules of k_bp_finish (no damping, src/bqa/state.py:113-121) applied on the host to the
 // sweep slots [ruled, launched) of a run, stopping at the first that ends it.
 void apply_slot_rules(const BpStatus* sh, BpStatus& h, int& ruled, int launched, int max_iters, double bp_eps) {
@@ -712,7 +717,7 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
   if (max_iters <= 0)  // the reference asserts here (src/bqa/state.py:122)
     throw BqaError(BQA_ERR_NUMERIC, "max_bp_iter_number must be positive: BP ran no sweep");
   BpStatus* st = reinterpret_cast<BpStatus*>(j->status.p);
-  hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(1), 0, j->stream, st, j->mcur, max_iters, bp_eps);
+  hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kSweepSlots), 0, j->stream, st, j->mcur, max_iters, bp_eps);
   LAUNCH_CHECK();
   const long count = (long)j->M * j->chi * j->chi;
   const int damping_on = damping > 0.0 ? 1 : 0;
@@ -766,7 +771,7 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
       }
     }
     launched += c;
-    HIPX(hipMemcpyAsync(j->st_host, st, sizeof(BpStatus), hipMemcpyDeviceToHost, j->stream));
+    HIPX(hipMemcpyAsync(j->st_host, st, status_bytes(slots ? launched : 0), hipMemcpyDeviceToHost, j->stream));
     HIPX(hipStreamSynchronize(j->stream));
     if (slots) {
       apply_slot_rules(j->st_host, h, ruled, launched, max_iters, bp_eps);
@@ -803,11 +808,16 @@ template <int N>
 void launch_canon_h(bqa_job* j, int ccols, double pinv_eps, double deps) {
   using S = HCanon<N>;
   j->cws.ensure((size_t)j->E * S::WS * sizeof(double), j->dev_bytes, j->stream);
-  const int grid = (j->E + S::EPW - 1) / S::EPW;
-  hipLaunchKernelGGL((k_canon_h<N>), dim3(grid), dim3(64), 0, j->stream,
-                     reinterpret_cast<const cplx<double>*>(j->ext.p), j->E, ccols, pinv_eps, deps,
-                     reinterpret_cast<zd*>(j->canon.p), reinterpret_cast<double*>(j->lmbd.p),
-                     reinterpret_cast<double*>(j->cws.p));
+  auto launch = [&](auto kernel, int epw) {
+    hipLaunchKernelGGL(kernel, dim3((j->E + epw - 1) / epw), dim3(64), 0, j->stream,
+                       reinterpret_cast<const cplx<double>*>(j->ext.p), j->E, ccols, pinv_eps, deps,
+                       reinterpret_cast<zd*>(j->canon.p), reinterpret_cast<double*>(j->lmbd.p),
+                       reinterpret_cast<double*>(j->cws.p));
+  };
+  if (j->E <= S::kSplitEdges)
+    launch(k_canon_h<N, true>, S::EPWS);
+  else
+    launch(k_canon_h<N, false>, S::EPW);
   LAUNCH_CHECK();
 }
 
@@ -1391,8 +1401,8 @@ constexpr int kSvMaxGrid = 2048;
 int sv_grid(unsigned long long tiles) { return (int)std::min<unsigned long long>(tiles, kSvMaxGrid); }
 
 // The X rotations (MODE 0, with the diagonal phase when ez is given) or the readout sums
-// (MODE 1) of every qubit, pass by pass; `each` gets the block count, first qubit and qubit
-// count of a readout pass.
+// (MODE 1) of every qubit, pass by pass; `each` gets the block count, first qubit, qubit count
+// and first tile bit of a readout pass.
 template <int MODE, typename F>
 void sv_passes(bqa_sv* s, const double* ez, double ztime, double xtime, F&& each) {
   const int n = s->n;
@@ -1403,13 +1413,13 @@ void sv_passes(bqa_sv* s, const double* ez, double ztime, double xtime, F&& each
   const int g0 = sv_grid(1ULL << (n - tb));
   hipLaunchKernelGGL((k_sv_low<MODE>), dim3(g0), dim3(kSvThreads), 0, s->stream, psi, n, ez, ztime, c, sn, part);
   LAUNCH_CHECK();
-  each(g0, 0, tb);
+  each(g0, 0, tb, 0);
   for (int b0 = tb; b0 < n; b0 += kSvTileBits - kSvRowBits) {
     const int t = std::min(kSvTileBits - kSvRowBits, n - b0);
-    const int g = sv_grid(1ULL << (n - kSvRowBits - t));
+    const int g = sv_grid(1ULL << (n - kSvTileBits));
     hipLaunchKernelGGL((k_sv_high<MODE>), dim3(g), dim3(kSvThreads), 0, s->stream, psi, n, b0, t, c, sn, part);
     LAUNCH_CHECK();
-    each(g, b0, t);
+    each(g, b0, t, kSvTileBits - t);
   }
 }
 
@@ -1433,43 +1443,48 @@ struct bqa_batch {
 
 namespace {
 
-// Split-column canonicaliser geometry of n: workspace doubles per edge, edges per 64-lane block.
+// Split-column canonicaliser geometry of n: workspace doubles per edge, edges per 64-lane block of a job of E edges
+// (a job takes the same form of the kernel in a batch as alone).
 size_t canon_h_ws(int n) { return 10 * (size_t)n * n + 5 * (size_t)n; }
 int canon_h_epw(int n) {
   const int p = n / 2, p2 = p <= 1 ? 1 : p <= 2 ? 2 : p <= 4 ? 4 : p <= 8 ? 8 : 16;
   return 64 / (2 * p2);
 }
+bool canon_h_split(int n, int E) { return E <= 2048 * (canon_h_epw(n) / 2); }
 
 template <int N>
-void launch_canon_multi(const CanonEntry* tab, int entries, int blocks, hipStream_t s) {
-  hipLaunchKernelGGL((k_canon_h_multi<N>), dim3(blocks), dim3(64), 0, s, tab, entries);
+void launch_canon_multi(bool split, const CanonEntry* tab, int entries, int blocks, hipStream_t s) {
+  if (split)
+    hipLaunchKernelGGL((k_canon_h_multi<N, true>), dim3(blocks), dim3(64), 0, s, tab, entries);
+  else
+    hipLaunchKernelGGL((k_canon_h_multi<N, false>), dim3(blocks), dim3(64), 0, s, tab, entries);
 }
 
-bool canon_multi_dispatch(int n, const CanonEntry* tab, int entries, int blocks, hipStream_t s) {
+bool canon_multi_dispatch(int n, bool split, const CanonEntry* tab, int entries, int blocks, hipStream_t s) {
   switch (n) {
-    case 2: launch_canon_multi<2>(tab, entries, blocks, s); return true;
-    case 4: launch_canon_multi<4>(tab, entries, blocks, s); return true;
-    case 6: launch_canon_multi<6>(tab, entries, blocks, s); return true;
-    case 8: launch_canon_multi<8>(tab, entries, blocks, s); return true;
-    case 10: launch_canon_multi<10>(tab, entries, blocks, s); return true;
-    case 12: launch_canon_multi<12>(tab, entries, blocks, s); return true;
-    case 14: launch_canon_multi<14>(tab, entries, blocks, s); return true;
-    case 16: launch_canon_multi<16>(tab, entries, blocks, s); return true;
-    case 18: launch_canon_multi<18>(tab, entries, blocks, s); return true;
-    case 20: launch_canon_multi<20>(tab, entries, blocks, s); return true;
-    case 22: launch_canon_multi<22>(tab, entries, blocks, s); return true;
-    case 24: launch_canon_multi<24>(tab, entries, blocks, s); return true;
-    case 26: launch_canon_multi<26>(tab, entries, blocks, s); return true;
-    case 28: launch_canon_multi<28>(tab, entries, blocks, s); return true;
-    case 30: launch_canon_multi<30>(tab, entries, blocks, s); return true;
-    case 32: launch_canon_multi<32>(tab, entries, blocks, s); return true;
+    case 2: launch_canon_multi<2>(split, tab, entries, blocks, s); return true;
+    case 4: launch_canon_multi<4>(split, tab, entries, blocks, s); return true;
+    case 6: launch_canon_multi<6>(split, tab, entries, blocks, s); return true;
+    case 8: launch_canon_multi<8>(split, tab, entries, blocks, s); return true;
+    case 10: launch_canon_multi<10>(split, tab, entries, blocks, s); return true;
+    case 12: launch_canon_multi<12>(split, tab, entries, blocks, s); return true;
+    case 14: launch_canon_multi<14>(split, tab, entries, blocks, s); return true;
+    case 16: launch_canon_multi<16>(split, tab, entries, blocks, s); return true;
+    case 18: launch_canon_multi<18>(split, tab, entries, blocks, s); return true;
+    case 20: launch_canon_multi<20>(split, tab, entries, blocks, s); return true;
+    case 22: launch_canon_multi<22>(split, tab, entries, blocks, s); return true;
+    case 24: launch_canon_multi<24>(split, tab, entries, blocks, s); return true;
+    case 26: launch_canon_multi<26>(split, tab, entries, blocks, s); return true;
+    case 28: launch_canon_multi<28>(split, tab, entries, blocks, s); return true;
+    case 30: launch_canon_multi<30>(split, tab, entries, blocks, s); return true;
+    case 32: launch_canon_multi<32>(split, tab, entries, blocks, s); return true;
     default: return false;
   }
 }
 
 // The canonicalisers of the batch's jobs whose bond dimension has a split-column kernel (state.py:171-200
-// per job): once each job's extended messages are done (its own stream), one launch per n over all of
-// them on the batch stream, then each job's lambda maxima readback there; each job's stream then waits
+// per job): once each job's extended messages are done (its own stream), one launch per n and form over
+// all of them on the batch stream, then each job's lambda maxima readback there; each job's stream then waits
 // for that.  Jobs marked false in `shared` ran their own canonicaliser with their extended messages.
 void batch_canon(bqa_batch* b, int count, bqa_job* const* jobs, const double* pinv_eps,
                  const std::vector<char>& shared) {
@@ -1477,8 +1492,11 @@ void batch_canon(bqa_batch* b, int count, bqa_job* const* jobs, const double* pi
   for (int k = 0; k < count; ++k)
     if (shared[k]) order.push_back(k);
   if (order.empty()) return;
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int x, int y) { return canon_h_n(jobs[x]->chi) < canon_h_n(jobs[y]->chi); });
+  auto form = [&](int k) {
+    const int n = canon_h_n(jobs[k]->chi);
+    return std::make_pair(n, canon_h_split(n, jobs[k]->E));
+  };
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return form(x) < form(y); });
   for (int k : order) {
     bqa_job* j = jobs[k];
     canon_outputs(j);
@@ -1499,14 +1517,16 @@ void batch_canon(bqa_batch* b, int count, bqa_job* const* jobs, const double* pi
   b->ctab.ensure(entries * sizeof(CanonEntry), b->dev_bytes, b->stream);
   struct Launch {
     int n;
+    bool split;
     size_t first, count;
     int blocks;
   };
   std::vector<Launch> launches;
   for (size_t x = 0; x < entries; ++x) {
     bqa_job* j = jobs[order[x]];
-    const int n = canon_h_n(j->chi);
-    if (launches.empty() || launches.back().n != n) launches.push_back({n, x, 0, 0});
+    const auto [n, split] = form(order[x]);
+    if (launches.empty() || launches.back().n != n || launches.back().split != split)
+      launches.push_back({n, split, x, 0, 0});
     Launch& L = launches.back();
     CanonEntry& e = b->ctab_host[x];
     e.ext = reinterpret_cast<const cplx<double>*>(j->ext.p);
@@ -1518,7 +1538,8 @@ void batch_canon(bqa_batch* b, int count, bqa_job* const* jobs, const double* pi
     e.pinv_eps = pinv_eps[order[x]];
     e.deps = canon_deps(j);
     e.block0 = L.blocks;
-    const long blocks = (long)L.blocks + (j->E + canon_h_epw(n) - 1) / canon_h_epw(n);
+    const int epw = canon_h_epw(n) / (split ? 2 : 1);
+    const long blocks = (long)L.blocks + (j->E + epw - 1) / epw;
     require(blocks <= std::numeric_limits<int>::max(), "too many edges in one shared canonicaliser launch");
     L.blocks = (int)blocks;
     ++L.count;
@@ -1526,7 +1547,7 @@ void batch_canon(bqa_batch* b, int count, bqa_job* const* jobs, const double* pi
   HIPX(hipMemcpyAsync(b->ctab.p, b->ctab_host, entries * sizeof(CanonEntry), hipMemcpyHostToDevice, b->stream));
   const CanonEntry* tab = reinterpret_cast<const CanonEntry*>(b->ctab.p);
   for (const auto& L : launches) {
-    if (!canon_multi_dispatch(L.n, tab + L.first, (int)L.count, L.blocks, b->stream))
+    if (!canon_multi_dispatch(L.n, L.split, tab + L.first, (int)L.count, L.blocks, b->stream))
       throw BqaError(BQA_ERR_HIP, "no shared canonicaliser for n = " + std::to_string(L.n));
     LAUNCH_CHECK();
   }
@@ -1584,7 +1605,7 @@ void batch_bp(bqa_batch* b, int count, bqa_job* const* jobs, const int32_t* max_
     Run r{j, k, BpStatus{}, 0};
     r.h.cur = j->mcur;
     r.h.best_dist = INFINITY;
-    hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(1), 0, b->stream, reinterpret_cast<BpStatus*>(j->status.p),
+    hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kSweepSlots), 0, b->stream, reinterpret_cast<BpStatus*>(j->status.p),
                        j->mcur, max_iters[k], bp_eps[k]);
     LAUNCH_CHECK();
     runs.push_back(r);
@@ -1688,7 +1709,7 @@ void batch_bp(bqa_batch* b, int count, bqa_job* const* jobs, const int32_t* max_
     bool all = true;
     for (auto& r : runs) {
       if (r.h.done) continue;
-      HIPX(hipMemcpyAsync(r.j->st_host, r.j->status.p, sizeof(BpStatus), hipMemcpyDeviceToHost, b->stream));
+      HIPX(hipMemcpyAsync(r.j->st_host, r.j->status.p, status_bytes(launched), hipMemcpyDeviceToHost, b->stream));
     }
     HIPX(hipStreamSynchronize(b->stream));
     for (auto& r : runs) {
@@ -2406,7 +2427,7 @@ int bqa_sv_run_layer(bqa_sv* s, double xtime, double ztime) {
   return guarded([&] {
     require(s, "null simulator");
     HIPX(hipSetDevice(s->device));
-    sv_passes<0>(s, reinterpret_cast<const double*>(s->ez.p), ztime, xtime, [](int, int, int) {});
+    sv_passes<0>(s, reinterpret_cast<const double*>(s->ez.p), ztime, xtime, [](int, int, int, int) {});
     HIPX(hipStreamSynchronize(s->stream));
   });
 }
@@ -2421,9 +2442,9 @@ int bqa_sv_density(bqa_sv* s, double* rho_out, double* bloch_out) {
     double* rho = reinterpret_cast<double*>(res.p);
     double* bloch = rho + 8 * (size_t)s->n;
     try {
-      sv_passes<1>(s, nullptr, 0.0, 0.0, [&](int blocks, int q0, int nb) {
-        hipLaunchKernelGGL(k_sv_finish, dim3(1), dim3(64), 0, s->stream, reinterpret_cast<const double*>(s->part.p),
-                           blocks, q0, nb, rho, bloch);
+      sv_passes<1>(s, nullptr, 0.0, 0.0, [&](int blocks, int q0, int nb, int bit0) {
+        hipLaunchKernelGGL(k_sv_finish, dim3(nb), dim3(kSvThreads), 0, s->stream,
+                           reinterpret_cast<const double*>(s->part.p), blocks, q0, bit0, rho, bloch);
         LAUNCH_CHECK();
       });
       if (rho_out)

@@ -35,6 +35,12 @@ struct HCanon {
   static constexpr int G = 2 * P2;                                  // lanes per edge
   static constexpr int EPW = 64 / G;                                // edges per wave
   static constexpr int NH = N / 2;                                  // rows per lane
+  // Split form (both sides of an edge at once): lanes and edges per wave, and the edges up to which it is taken.
+  // A wave's serial chain of two factorisations and three Jacobi runs is then two thirds as long, but half of its
+  // lanes idle in the third, so it pays while the waves of all edges run at once (two a SIMD).
+  static constexpr int GS = 2 * G;
+  static constexpr int EPWS = 64 / GS;
+  static constexpr int kSplitEdges = 2048 * EPWS;
   // workspace doubles per edge: U_f, U_b, Q (N x N complex each), sorted Us and Z columns
   // (N x N complex each), sq/ip of both sides, 1/Lambda of the sorted columns
   static constexpr int WS = 10 * N * N + 5 * N;
@@ -300,20 +306,23 @@ __device__ void hcholesky(HCol<N / 2>& top, HCol<N / 2>& bot, int k, int h, bool
   }
 }
 
-// The edges of block `blk` of one job's launch: blk * EPW .. blk * EPW + EPW - 1.
-template <int N>
+// The edges of block `blk` of one job's launch: blk * EPW .. blk * EPW + EPW - 1.  SPLIT: the edge's two extended
+// messages are factored by two lane groups at once, and the first group goes on with the bond matrix.
+template <int N, bool SPLIT>
 __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext, int E, int ccols, double pinv_eps,
                                             double deps, zd* __restrict__ canon, double* __restrict__ lfull,
                                             double* __restrict__ ws, int blk) {
   using S = HCanon<N>;
   constexpr int P = S::P, P2 = S::P2, G = S::G, NH = S::NH;
+  constexpr int GL = SPLIT ? S::GS : G;        // lanes per edge
   const int lane = threadIdx.x;
-  const int w = lane % G;
-  const int base = lane - w;
-  const int h = w / P2, k = w % P2;
-  const int edge = blk * S::EPW + lane / G;
+  const int w = lane % GL;
+  const int base = lane - lane % G;
+  const int h = lane % G / P2, k = lane % P2;
+  const int edge = blk * (64 / GL) + lane / GL;
   const bool valid = edge < E;
   const bool active = valid && k < P;
+  const bool lead = w < G;                     // the lane group of the bond matrix
   double* wsE = ws + (size_t)(valid ? edge : 0) * S::WS;
   double* Uf = wsE;
   double* Ub = wsE + 2 * N * N;
@@ -325,10 +334,11 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
 
   // pivot columns, one slot an edge; the slots' stride puts the edges' and halves' rows on different banks
   constexpr int kSlot = N + 2;
-  __shared__ double2 lslots[S::EPW * kSlot];
+  __shared__ double2 lslots[S::EPW * kSlot];   // one per lane group
   double2* lcol = lslots + (lane / G) * kSlot;
   HCol<NH> top, bot;
-  for (int side = 0; side < 2; ++side) {
+  for (int pass = 0; pass < (SPLIT ? 1 : 2); ++pass) {
+    const int side = SPLIT ? w / G : pass;
     const int ct = k, cb = N - 1 - k;
     double dgt = 0.0, dgb = 0.0;
 #pragma unroll
@@ -404,7 +414,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       kc.re[r] = 0.0;
       kc.im[r] = 0.0;
     }
-    if (active) {
+    if (active && lead) {
       // t outermost with the NH row accumulators inside: each sum keeps its
       // order while the workspace loads stream through a small register window
       const double* ub = Ub + j * 2 * N;
@@ -430,7 +440,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       }
     }
   }
-  int it = k < P ? 2 * k : -1, ib = k < P ? 2 * k + 1 : -1;
+  int it = lead && k < P ? 2 * k : -1, ib = lead && k < P ? 2 * k + 1 : -1;
   hjacobi<N>(top, bot, it, ib, k);
   const bool realt = valid && it >= 0, realb = valid && ib >= 0;
 
@@ -480,13 +490,14 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       // chi = 8: the same products regrouped without the 16 x 16 Q,
       //   V = U_f diag(sq_f) Us and C_f = U_f diag(ip_f) Us in one pass,
       //   Z[c][j] = keep_b[j] conj((U_b^T V)[j][c]) / Lambda_c,  C_b = U_b Z,
-      // each lane taking a block of 4 rows x 2 columns so every row and column
+      // each lane taking a block of 4 (SPLIT: 2) rows x 2 columns so every row and column
       // it loads serves several outputs (about a quarter of the workspace
       // reads of the entry-per-lane form below).
       __syncthreads();
-      const int a0 = 4 * (w >> 2), c0 = 2 * (w & 3);
+      constexpr int RB = 64 / GL;
+      const int a0 = RB * (w >> 2), c0 = 2 * (w & 3);
       double* V = Q;  // V[c][a], 16 x ccols
-      double xr[4][2] = {}, xi[4][2] = {}, yr[4][2] = {}, yi[4][2] = {};
+      double xr[RB][2] = {}, xi[RB][2] = {}, yr[RB][2] = {}, yi[RB][2] = {};
       if (valid) {
 #pragma unroll 2
         for (int t = 0; t < N; ++t) {
@@ -501,7 +512,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
             pi[cc] = ipf[t] * ui;
           }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
+          for (int r = 0; r < RB; ++r) {
             const double fr = Uf[t * 2 * N + 2 * (a0 + r)], fi = Uf[t * 2 * N + 2 * (a0 + r) + 1];
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
@@ -518,7 +529,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
           const int c = c0 + cc;
           if (c < ccols) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < RB; ++r) {
               V[c * 2 * N + 2 * (a0 + r)] = xr[r][cc];
               V[c * 2 * N + 2 * (a0 + r) + 1] = xi[r][cc];
               Cf[(a0 + r) * ccols + c] = mk(yr[r][cc], yi[r][cc]);
@@ -528,7 +539,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       }
       __syncthreads();
       // Z rows j = a0..a0+3, columns c0, c0+1
-      double wr[4][2] = {}, wi[4][2] = {};
+      double wr[RB][2] = {}, wi[RB][2] = {};
       if (valid) {
 #pragma unroll 2
         for (int u = 0; u < N; ++u) {
@@ -540,7 +551,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
             vi[cc] = c < ccols ? V[c * 2 * N + 2 * u + 1] : 0.0;
           }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
+          for (int r = 0; r < RB; ++r) {
             const double br = Ub[(a0 + r) * 2 * N + 2 * u], bi = Ub[(a0 + r) * 2 * N + 2 * u + 1];
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
@@ -554,7 +565,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
           const int c = c0 + cc;
           if (c < ccols) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < RB; ++r) {
               const int j = a0 + r;
               const double g = ipb[j] > 0.0 ? il[c] : 0.0;
               Zc[(c * N + j) * 2] = wr[r][cc] * g;
@@ -566,7 +577,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
       __syncthreads();
       // C_b rows a0..a0+3, columns c0, c0+1
       if (valid) {
-        double br_[4][2] = {}, bi_[4][2] = {};
+        double br_[RB][2] = {}, bi_[RB][2] = {};
 #pragma unroll 2
         for (int t = 0; t < N; ++t) {
           double zr[2], zi[2];
@@ -577,7 +588,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
             zi[cc] = c < ccols ? Zc[(c * N + t) * 2 + 1] : 0.0;
           }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
+          for (int r = 0; r < RB; ++r) {
             const double vr = Ub[t * 2 * N + 2 * (a0 + r)], vi = Ub[t * 2 * N + 2 * (a0 + r) + 1];
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
@@ -592,7 +603,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
           const int c = c0 + cc;
           if (c < ccols) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Cb[(a0 + r) * ccols + c] = mk(br_[r][cc], bi_[r][cc]);
+            for (int r = 0; r < RB; ++r) Cb[(a0 + r) * ccols + c] = mk(br_[r][cc], bi_[r][cc]);
           }
         }
       }
@@ -601,7 +612,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   }
   // Q, one entry per lane per step over the group
   if (valid) {
-    for (int x = w; x < N * N; x += G) {
+    for (int x = w; x < N * N; x += GL) {
       const int t = x / N, i = x % N;
       double ar = 0.0, ai = 0.0;
       for (int u = 0; u < N; ++u) {
@@ -616,7 +627,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   }
   __syncthreads();
   if (valid) {
-    for (int x = w; x < ccols * N; x += G) {
+    for (int x = w; x < ccols * N; x += GL) {
       const int c = x / N, jj = x % N;
       double ar = 0.0, ai = 0.0;
       if (ipb[jj] > 0.0) {
@@ -636,7 +647,7 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   if (valid) {
     zd* Cb = canon + (size_t)edge * N * ccols;
     zd* Cf = canon + (size_t)(E + edge) * N * ccols;
-    for (int x = w; x < N * ccols; x += G) {
+    for (int x = w; x < N * ccols; x += GL) {
       const int a = x / ccols, c = x % ccols;
       double fr_ = 0.0, fi_ = 0.0, br_ = 0.0, bi_ = 0.0;
       for (int t = 0; t < N; ++t) {
@@ -655,11 +666,11 @@ __device__ __forceinline__ void canon_h_run(const cplx<double>* __restrict__ ext
   }
 }
 
-template <int N>
+template <int N, bool SPLIT>
 __global__ __launch_bounds__(64, N <= 16 ? 3 : 2) void k_canon_h(const cplx<double>* __restrict__ ext, int E, int ccols,
                                                 double pinv_eps, double deps, zd* __restrict__ canon,
                                                 double* __restrict__ lfull, double* __restrict__ ws) {
-  canon_h_run<N>(ext, E, ccols, pinv_eps, deps, canon, lfull, ws, blockIdx.x);
+  canon_h_run<N, SPLIT>(ext, E, ccols, pinv_eps, deps, canon, lfull, ws, blockIdx.x);
 }
 
 // One job's edges in a launch that covers several jobs' canonicalisers (the serving batch):
@@ -676,7 +687,7 @@ struct CanonEntry {
 
 // The canonicalisers of several jobs (same n) in one launch: entry e takes blocks
 // block0_e .. block0_{e+1} - 1 (found by binary search; block0 ascending, block0_0 = 0).
-template <int N>
+template <int N, bool SPLIT>
 __global__ __launch_bounds__(64, N <= 16 ? 3 : 2) void k_canon_h_multi(const CanonEntry* __restrict__ tab,
                                                                       int entries) {
   int lo = 0, hi = entries - 1;
@@ -688,7 +699,7 @@ __global__ __launch_bounds__(64, N <= 16 ? 3 : 2) void k_canon_h_multi(const Can
       hi = mid - 1;
   }
   const CanonEntry& e = tab[lo];
-  canon_h_run<N>(e.ext, e.E, e.ccols, e.pinv_eps, e.deps, e.canon, e.lfull, e.ws, (int)blockIdx.x - e.block0);
+  canon_h_run<N, SPLIT>(e.ext, e.E, e.ccols, e.pinv_eps, e.deps, e.canon, e.lfull, e.ws, (int)blockIdx.x - e.block0);
 }
 
 }  // namespace bqa

@@ -9,22 +9,24 @@
 // gate, exact_sim.py:51-63); the Z and ZZ gates are diagonal and the X gates on
 // different qubits commute.
 //
-// The X layer runs in passes over groups of qubits, each pass a tile kernel
-// that stages 1024 amplitudes in LDS and applies the rotations of its group
-// there: the first pass takes 1024 contiguous amplitudes (qubits 0..9, and the
-// diagonal phase on the way in); later passes take 16 contiguous amplitudes
-// (qubits 0..3, for 256-byte rows) times the 2^t values of t <= 6 higher
-// qubits.  The readout uses the same tiles: each pass accumulates, for the
-// qubits of its group, |psi|^2 split by the qubit's value and the off-diagonal
-// sum conj(psi[x]) psi[x | 2^q] over pairs inside the tile.
+// The X layer runs in passes over groups of qubits, and the readout in the same passes.  A pass takes tiles of 4,096
+// amplitudes, sixteen in a thread's registers at a time: the four tile bits that index a thread's registers are
+// rotated (or summed over pairs) there, and an exchange through LDS brings the next four into the registers.  The
+// first pass takes contiguous tiles (qubits 0..11, with the diagonal phase on the way in); later passes take 2^cb
+// contiguous amplitudes (cb >= 4: 256-byte rows and more) times the 2^t values of t = 12 - cb <= 8 higher qubits.
+// Bounded by memory: a rotation pass reads and writes the state once, a readout pass reads it.  At 26 qubits (1 GB)
+// a layer is three passes and the readout three reads; with tiles of 1,024 amplitudes and every rotation through
+// LDS they were four passes (2.0 ms a layer) and the readout took 9.6 ms, most of it in lane reductions of every
+// qubit of every tile and in a serial sum over the blocks.
 #pragma once
 
 #include "common.hpp"
+#include "kernels_mfma.hpp"
 
 namespace bqa {
 
-constexpr int kSvTileBits = 10;            // amplitudes per tile: 1024 (16 KB of complex128)
-constexpr int kSvRowBits = 4;              // contiguous amplitudes per row in the high-qubit passes
+constexpr int kSvTileBits = 12;            // amplitudes per tile: 4,096, sixteen per thread
+constexpr int kSvRowBits = 4;              // least contiguous amplitudes per row in the high-qubit passes
 constexpr int kSvThreads = 256;
 constexpr int kSvMaxEdges = 2048;          // edges kept in LDS by the energy kernel
 
@@ -62,144 +64,201 @@ __global__ void k_sv_init(cplx<double>* __restrict__ psi, int n) {
     psi[x] = mk(__popcll(x) & 1 ? -a : a, 0.0);
 }
 
-// Global index of tile element k (0 <= k < 16 * 2^t) in a pass over qubits b0..b0+t-1
-// (b0 >= kSvRowBits): row r = k >> 4 carries the t target bits, c = k & 15 the low bits,
-// the tile number T the remaining bits (those between 4 and b0, then those above b0 + t).
-__device__ __forceinline__ unsigned long long sv_high_index(unsigned long long T, int k, int b0, int t) {
-  const unsigned long long c = (unsigned long long)(k & ((1 << kSvRowBits) - 1));
-  const unsigned long long r = (unsigned long long)(k >> kSvRowBits);
-  const int mid = b0 - kSvRowBits;
-  const unsigned long long lo = T & ((1ULL << mid) - 1ULL);
-  const unsigned long long hi = T >> mid;
-  return c | (lo << kSvRowBits) | (r << b0) | (hi << (b0 + t));
+// Tile element of register j in the three layouts: the registers' tile bits are 8..11 (A), 4..7 (B) or 0..3 (C).
+enum SvLayout { kSvA, kSvB, kSvC };
+template <SvLayout L>
+__device__ __forceinline__ int sv_element(int j) {
+  const int t = threadIdx.x;
+  return L == kSvA ? j << 8 | t : L == kSvB ? (t >> 4) << 8 | j << 4 | (t & 15) : t << 4 | j;
 }
+constexpr int sv_first_bit(SvLayout l) { return l == kSvA ? 8 : l == kSvB ? 4 : 0; }
 
-// Rotations exp(-i xtime X) on the tile-local bits [0, nb) of an LDS tile: amplitude k's
-// partner for local bit b is k ^ (1 << (b + shift)).
-__device__ __forceinline__ void sv_rotate_tile(cplx<double>* s, int size, int nb, int shift, double c, double sn) {
-  const int half = size >> 1;
-  for (int b = 0; b < nb; ++b) {
-    const int m = 1 << (b + shift);
-    for (int p = threadIdx.x; p < half; p += blockDim.x) {
-      // p-th pair: insert a zero at bit position (b + shift)
-      const int k0 = ((p >> (b + shift)) << (b + shift + 1)) | (p & (m - 1));
-      const int k1 = k0 | m;
-      const cplx<double> a0 = s[k0], a1 = s[k1];
-      // (cos t) a - i (sin t) X a
-      s[k0] = mk(c * a0.x + sn * a1.y, c * a0.y - sn * a1.x);
-      s[k1] = mk(c * a1.x + sn * a0.y, c * a1.y - sn * a0.x);
-    }
-    __syncthreads();
-  }
-}
+// LDS position of tile element k: a linear permutation under which every layout's accesses spread over the banks.
+__device__ __forceinline__ constexpr int sv_slot(int k) { return k ^ ((k >> 4) & 15) ^ (((k >> 8) & 1) << 4); }
 
-// Per-qubit readout sums of the tile-local bits [0, nb) (partner bit b + shift), added to this
-// wave's slots wacc[4 b + k]: r00, r11, Re r10, Im r10 with r10 = sum conj(psi0) psi1.  Each
-// wave reduces its lanes with shuffles and its lane 0 alone writes its slots, so the order of
-// every sum is fixed.
-__device__ __forceinline__ void sv_read_tile(const cplx<double>* s, int size, int nb, int shift, double* wacc) {
-  const int half = size >> 1;
-  const int l = threadIdx.x & 63;
-  for (int b = 0; b < nb; ++b) {
-    const int m = 1 << (b + shift);
-    double v[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int p = threadIdx.x; p < half; p += blockDim.x) {
-      const int k0 = ((p >> (b + shift)) << (b + shift + 1)) | (p & (m - 1));
-      const cplx<double> a0 = s[k0], a1 = s[k0 | m];
-      v[0] += abs2(a0);
-      v[1] += abs2(a1);
-      v[2] += a0.x * a1.x + a0.y * a1.y;
-      v[3] += a0.x * a1.y - a0.y * a1.x;
-    }
+// The tile from layout L to layout M, one component at a time through 32 KB of LDS (so four blocks share a CU).
+template <SvLayout L, SvLayout M>
+__device__ __forceinline__ void sv_exchange(cplx<double> (&a)[16], double* s) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
-      if (l == 0) wacc[4 * b + k] += v[k];
+  for (int part = 0; part < 2; ++part) {
+    // opaque: one position per layout is kept, not sixteen
+    const int from = opaque(sv_slot(sv_element<L>(0))), to = opaque(sv_slot(sv_element<M>(0)));
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s[from ^ sv_slot(j << sv_first_bit(L))] = part ? a[j].y : a[j].x;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) (part ? a[j].y : a[j].x) = s[to ^ sv_slot(j << sv_first_bit(M))];
+  }
+}
+
+// exp(-i xtime X) on the registers' tile bits of layout L that lie in [first, last).
+template <SvLayout L>
+__device__ __forceinline__ void sv_rotate(cplx<double> (&a)[16], int first, int last, double c, double sn) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    if (sv_first_bit(L) + b < first || sv_first_bit(L) + b >= last) continue;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      if (j >> b & 1) continue;
+      const cplx<double> a0 = a[j], a1 = a[j | 1 << b];
+      // (cos t) a - i (sin t) X a
+      a[j] = mk(c * a0.x + sn * a1.y, c * a0.y - sn * a1.x);
+      a[j | 1 << b] = mk(c * a1.x + sn * a0.y, c * a1.y - sn * a0.x);
     }
   }
 }
 
-// Block partials part[block][4 nb] from the per-wave slots.
-__device__ __forceinline__ void sv_store_partials(const double (*wacc)[4 * kSvTileBits], int nb, double* part) {
+// Readout sums of the registers' four tile bits, added to this thread's v[b]: r00, r11, Re r10, Im r10 with
+// r10 = sum conj(psi0) psi1.
+__device__ __forceinline__ void sv_sums(const cplx<double> (&a)[16], double (&v)[4][4]) {
+  double norm[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) norm[j] = abs2(a[j]);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      if (j >> b & 1) continue;
+      const cplx<double> a0 = a[j], a1 = a[j | 1 << b];
+      v[b][0] += norm[j];
+      v[b][1] += norm[j | 1 << b];
+      v[b][2] = fma(a0.x, a1.x, fma(a0.y, a1.y, v[b][2]));
+      v[b][3] = fma(a0.x, a1.y, fma(-a0.y, a1.x, v[b][3]));
+    }
+}
+
+// part[block][tile bit][4] of the bits of layout L from the threads' sums, always in the same order.
+template <SvLayout L>
+__device__ __forceinline__ void sv_store(const double (&v)[4][4], double* s, double* part) {
   __syncthreads();
-  for (int k = threadIdx.x; k < 4 * nb; k += blockDim.x) {
-    double v = 0.0;
-    for (int w = 0; w < kSvThreads / 64; ++w) v += wacc[w][k];
-    part[(size_t)blockIdx.x * 4 * kSvTileBits + k] = v;
+#pragma unroll
+  for (int x = 0; x < 16; ++x) {
+    double r = v[x >> 2][x & 3];
+    for (int o = 32; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
+    if ((threadIdx.x & 63) == 0) s[x * (kSvThreads / 64) + (threadIdx.x >> 6)] = r;
+  }
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    double r = 0.0;
+    for (int w = 0; w < kSvThreads / 64; ++w) r += s[threadIdx.x * (kSvThreads / 64) + w];
+    part[(size_t)blockIdx.x * 4 * kSvTileBits + 4 * sv_first_bit(L) + threadIdx.x] = r;
   }
 }
 
-// First pass: tiles of 2^tb contiguous amplitudes (tb = min(n, 10)).  MODE 0: diagonal phase
-// exp(-i ztime Ez) (when ez != nullptr), then the X rotations of qubits 0..tb-1.  MODE 1: readout
-// sums of qubits 0..tb-1 into part.
+// First pass: tiles of 2^tb contiguous amplitudes (tb = min(n, 12); with fewer qubits the tile's other elements are
+// zero).  MODE 0: diagonal phase exp(-i ztime Ez) (when ez != nullptr), then the X rotations of qubits 0..tb-1.
+// MODE 1: readout sums of qubits 0..tb-1 into part.
 template <int MODE>
-__global__ __launch_bounds__(kSvThreads) void k_sv_low(cplx<double>* __restrict__ psi, int n,
+__global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_low(cplx<double>* __restrict__ psi, int n,
                                                        const double* __restrict__ ez, double ztime, double c,
                                                        double sn, double* part) {
-  __shared__ cplx<double> s[1 << kSvTileBits];
+  __shared__ double s[1 << kSvTileBits];
   const int tb = n < kSvTileBits ? n : kSvTileBits;
   const int size = 1 << tb;
   const unsigned long long tiles = 1ULL << (n - tb);
-  __shared__ double wacc[kSvThreads / 64][4 * kSvTileBits];
-  for (int k = threadIdx.x; k < kSvThreads / 64 * 4 * kSvTileBits; k += blockDim.x) (&wacc[0][0])[k] = 0.0;
-  __syncthreads();
+  double va[4][4] = {}, vb[4][4] = {}, vc[4][4] = {};
   for (unsigned long long T = blockIdx.x; T < tiles; T += gridDim.x) {
-    const unsigned long long base = T << tb;
-    for (int k = threadIdx.x; k < size; k += blockDim.x) {
-      cplx<double> a = psi[base + k];
-      if (MODE == 0 && ez) {
+    cplx<double>* p = psi + (T << tb);
+    cplx<double> a[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int k = sv_element<kSvA>(j);
+      a[j] = k < size ? p[k] : mk(0.0, 0.0);
+    }
+    if (MODE == 0 && ez) {
+      const double* e = ez + (T << tb);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int k = sv_element<kSvA>(j);
         double sp, cp;
-        sincos(-ztime * ez[base + k], &sp, &cp);
-        a = a * mk(cp, sp);
+        sincos(k < size ? -ztime * e[k] : 0.0, &sp, &cp);
+        a[j] = a[j] * mk(cp, sp);
+        __builtin_amdgcn_sched_barrier(0);   // one sincos's temporaries at a time
       }
-      s[k] = a;
     }
-    __syncthreads();
     if (MODE == 0) {
-      sv_rotate_tile(s, size, tb, 0, c, sn);
-      for (int k = threadIdx.x; k < size; k += blockDim.x) psi[base + k] = s[k];
+      sv_rotate<kSvA>(a, 0, tb, c, sn);
+      sv_exchange<kSvA, kSvC>(a, s);
+      sv_rotate<kSvC>(a, 0, tb, c, sn);
+      sv_exchange<kSvC, kSvB>(a, s);
+      sv_rotate<kSvB>(a, 0, tb, c, sn);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int k = sv_element<kSvB>(j);
+        if (k < size) p[k] = a[j];
+      }
     } else {
-      sv_read_tile(s, size, tb, 0, wacc[threadIdx.x >> 6]);
+      sv_sums(a, va);
+      sv_exchange<kSvA, kSvC>(a, s);
+      sv_sums(a, vc);
+      sv_exchange<kSvC, kSvB>(a, s);
+      sv_sums(a, vb);
     }
-    __syncthreads();
   }
-  if (MODE == 1) sv_store_partials(wacc, tb, part);
+  if (MODE == 1) {
+    sv_store<kSvA>(va, s, part);
+    sv_store<kSvB>(vb, s, part);
+    sv_store<kSvC>(vc, s, part);
+  }
 }
 
-// Later passes: qubits b0..b0+t-1 (t <= 6, b0 >= 4), tiles of 16 x 2^t amplitudes.
+// Later passes: qubits b0..b0+t-1 (1 <= t <= 8, b0 >= 12 > cb = 12 - t).  Tile element k: bits below cb the lowest
+// qubits, the t bits above them the pass's qubits; the tile number T the remaining bits (those between cb and b0,
+// then those above b0 + t).  Readout sums of tile bits below cb are not used.
 template <int MODE>
-__global__ __launch_bounds__(kSvThreads) void k_sv_high(cplx<double>* __restrict__ psi, int n, int b0, int t,
+__global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_high(cplx<double>* __restrict__ psi, int n, int b0, int t,
                                                         double c, double sn, double* part) {
-  __shared__ cplx<double> s[1 << kSvTileBits];
-  const int size = 1 << (kSvRowBits + t);
-  const unsigned long long tiles = 1ULL << (n - kSvRowBits - t);
-  __shared__ double wacc[kSvThreads / 64][4 * kSvTileBits];
-  for (int k = threadIdx.x; k < kSvThreads / 64 * 4 * kSvTileBits; k += blockDim.x) (&wacc[0][0])[k] = 0.0;
-  __syncthreads();
+  __shared__ double s[1 << kSvTileBits];
+  const int cb = kSvTileBits - t, mid = b0 - cb;
+  const unsigned long long tiles = 1ULL << (n - kSvTileBits);
+  double va[4][4] = {}, vb[4][4] = {};
   for (unsigned long long T = blockIdx.x; T < tiles; T += gridDim.x) {
-    for (int k = threadIdx.x; k < size; k += blockDim.x) s[k] = psi[sv_high_index(T, k, b0, t)];
-    __syncthreads();
+    cplx<double>* p = psi + ((T & ((1ULL << mid) - 1ULL)) << cb) + ((T >> mid) << (b0 + t));
+    auto at = [&](int k) { return (unsigned long long)(k & ((1 << cb) - 1)) | (unsigned long long)(k >> cb) << b0; };
+    cplx<double> a[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) a[j] = p[at(sv_element<kSvA>(j))];
     if (MODE == 0) {
-      sv_rotate_tile(s, size, t, kSvRowBits, c, sn);
-      for (int k = threadIdx.x; k < size; k += blockDim.x) psi[sv_high_index(T, k, b0, t)] = s[k];
+      sv_rotate<kSvA>(a, cb, kSvTileBits, c, sn);
+      if (t > 4) {
+        sv_exchange<kSvA, kSvB>(a, s);
+        sv_rotate<kSvB>(a, cb, kSvTileBits, c, sn);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p[at(sv_element<kSvB>(j))] = a[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p[at(sv_element<kSvA>(j))] = a[j];
+      }
     } else {
-      sv_read_tile(s, size, t, kSvRowBits, wacc[threadIdx.x >> 6]);
+      sv_sums(a, va);
+      if (t > 4) {
+        sv_exchange<kSvA, kSvB>(a, s);
+        sv_sums(a, vb);
+      }
     }
-    __syncthreads();
   }
-  if (MODE == 1) sv_store_partials(wacc, t, part);
+  if (MODE == 1) {
+    sv_store<kSvA>(va, s, part);
+    if (t > 4) sv_store<kSvB>(vb, s, part);
+  }
 }
 
-// Bloch vectors and densities of qubits q0..q0+nb-1 from the block partials of one readout pass.
-__global__ void k_sv_finish(const double* __restrict__ part, int blocks, int q0, int nb, double* rho, double* bloch) {
-  const int b = threadIdx.x;
-  if (b >= nb) return;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int blk = 0; blk < blocks; ++blk)
-    for (int k = 0; k < 4; ++k) s[k] += part[(size_t)blk * 4 * kSvTileBits + 4 * b + k];
+// Bloch vectors and densities of qubits q0.. from the block partials of one readout pass: block b takes tile bit
+// bit0 + b, a wave each of its four sums.
+__global__ __launch_bounds__(kSvThreads) void k_sv_finish(const double* __restrict__ part, int blocks, int q0, int bit0,
+                                                          double* rho, double* bloch) {
+  __shared__ double s[4];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  double v = 0.0;
+  for (int blk = l; blk < blocks; blk += 64) v += part[(size_t)blk * 4 * kSvTileBits + 4 * (bit0 + blockIdx.x) + w];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if (l == 0) s[w] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
   const double tr = s[0] + s[1];
   const double r00 = s[0] / tr, r11 = s[1] / tr, r10r = s[2] / tr, r10i = s[3] / tr;
-  const int q = q0 + b;
+  const int q = q0 + blockIdx.x;
   // rho[p][q'] = sum psi_p conj(psi_q'): rho10 = r10, rho01 = conj(r10)
   if (rho) {
     double* ro = rho + 8 * (size_t)q;

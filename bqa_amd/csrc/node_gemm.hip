@@ -163,9 +163,11 @@ __device__ __forceinline__ void gram_tiles(vec4<R> (&acc)[MT][MT], const cplx<RX
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int cl = r >> 1, ri = r & 1;
   const int groups = (f1 - f0 + 15) >> 4;
-  cplx<RX> nx[MT][2];
-  cplx<RY> ny[MT][2];
-  auto fetch = [&](int q) {
+  // groups in flight while one multiplies: more where a group is few loads
+  constexpr int kAhead = MT == 1 ? 4 : MT == 2 ? 2 : 1;
+  cplx<RX> bx[kAhead][MT][2];
+  cplx<RY> by[kAhead][MT][2];
+  auto fetch = [&](int q, cplx<RX>(&nx)[MT][2], cplx<RY>(&ny)[MT][2]) {
     const int f = f0 + 16 * q + 4 * g + 2 * ri;
     const int o0 = f / inner, i0 = f - o0 * inner;
     const int at0 = o0 * chi * inner + i0;
@@ -212,21 +214,28 @@ __device__ __forceinline__ void gram_tiles(vec4<R> (&acc)[MT][MT], const cplx<RX
     out[2] = ri ? m0 : q0;
     out[3] = ri ? m1 : q1;
   };
-  if (wave < groups) fetch(wave);
-  for (int q = wave; q < groups; q += step) {
-    R a[MT][4], b[MT][4];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      spread(nx[mt], a[mt]);
-      spread(ny[mt], b[mt]);
+  for (int u = 0; u < kAhead; ++u)
+    if (wave + u * step < groups) fetch(wave + u * step, bx[u], by[u]);
+  for (int q0 = wave; q0 < groups; q0 += kAhead * step) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int q = q0 + u * step;
+      if (u > 0 && q >= groups) break;
+      R a[MT][4], b[MT][4];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        spread(bx[u][mt], a[mt]);
+        spread(by[u][mt], b[mt]);
+      }
+      if (q + kAhead * step < groups) fetch(q + kAhead * step, bx[u], by[u]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < MT; ++nt) acc[mt][nt] = mfma4(a[mt][t], b[nt][t], acc[mt][nt]);
     }
-    if (q + step < groups) fetch(q + step);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < MT; ++nt) acc[mt][nt] = mfma4(a[mt][t], b[nt][t], acc[mt][nt]);
   }
 }
 
@@ -252,6 +261,37 @@ __device__ __forceinline__ void add_tiles(double* sum, const vec4<R> (&acc)[MT][
         double* s = sum + (16 * mt + result_row<R>(g, v)) * 16 * MT + 16 * nt + col;
         *s = first ? (double)acc[mt][nt][v] : *s + (double)acc[mt][nt][v];
       }
+}
+
+// LDS tile sums (2 MT^2 KB each) that WG waves share: 64 KB of them over `groups` groups of waves.
+template <int MT, int WG>
+constexpr int gram_slots(int groups) {
+  int s = WG;
+  while (s > 1 && s * groups * 2 * MT * MT > 64) s /= 2;
+  return s;
+}
+
+// The sum of the WG waves' tiles of each of `groups` groups, in FP64 in slot 0 of the group: the waves add to the
+// slots in turns, then all threads add the slots, always in the same order.
+template <typename R, int MT, int WG>
+__device__ __forceinline__ void sum_tiles(double* slots, const vec4<R> (&acc)[MT][MT], int group, int w, int groups) {
+  constexpr int SZ = 256 * MT * MT;
+  const int S = groups == 1 ? gram_slots<MT, WG>(1) : gram_slots<MT, WG>(2);
+  double* own = slots + group * S * SZ;
+#pragma unroll 1
+  for (int turn = 0; turn < WG / S; ++turn) {
+    if (w / S == turn) add_tiles<R, MT>(own + (w % S) * SZ, acc, turn == 0);
+    __syncthreads();
+  }
+  if (S > 1) {
+    for (int x = threadIdx.x; x < groups * SZ; x += groups * WG * 64) {
+      double* at = slots + (x / SZ) * S * SZ + x % SZ;
+      double v = at[0];
+      for (int q = 1; q < S; ++q) v += at[q * SZ];
+      at[0] = v;
+    }
+    __syncthreads();
+  }
 }
 
 // Element (c, e) of the Gram sum conj(X) Y from the summed real products.
@@ -321,9 +361,9 @@ __device__ __forceinline__ void gram_sources(vec4<R> (&acc)[MT][MT], const GemmP
   }
 }
 
-// New messages: blocks take (node, output) items in turn and keep their distance maxima until the end.
-template <typename R, int MT>
-__global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_bp(ClassView cv, GemmPlan plan, int node0, int count,
+// New messages: blocks of W waves take (node, output) items in turn and keep their distance maxima until the end.
+template <typename R, int MT, int W>
+__global__ __launch_bounds__(64 * W) void k_gemm_gram_bp(ClassView cv, GemmPlan plan, int node0, int count,
                                                                int chi, const cplx<R>* __restrict__ T, cplx<R>* mA,
                                                                cplx<R>* mB, BpStatus* st, const cplx<R>* ws) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -340,47 +380,42 @@ __global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_bp(ClassView cv, Gem
   int node, k;
   for (int idx = blockIdx.x >> 3; node_item(idx, d, count, node, k); idx += gridDim.x >> 3) {
     const int i = node0 + node;
+    const long pos = cv.out_pos[k * cv.n + i];
     vec4<R> acc[MT][MT];
 #pragma unroll
     for (int a = 0; a < MT; ++a)
 #pragma unroll
       for (int b = 0; b < MT; ++b) acc[a][b] = vec4<R>{0, 0, 0, 0};
-    gram_sources<R, R, MT>(acc, plan, k, chi, T + (size_t)i * S, ws + (size_t)node * plan.products * S, S, 0, F, wave,
-                           kGemmWaves);
-#pragma unroll 1
-    for (int w = 0; w < kGemmWaves; ++w) {
-      if (w == wave) add_tiles<R, MT>(sum, acc, w == 0);
-      __syncthreads();
-    }
+    gram_sources<R, R, MT>(acc, plan, k, chi, T + (size_t)i * S, ws + (size_t)node * plan.products * S, S, 0, F, wave, W);
+    sum_tiles<R, MT, W>(sum, acc, 0, wave, 1);
     double tr = 0.0;
     for (int c = 0; c < chi; ++c) tr += gram_at<MT>(sum, c, c).x;
     const double inv = 0.5 / tr;
-    const long pos = cv.out_pos[k * cv.n + i];
-    for (int o = threadIdx.x; o < cc; o += kGemmThreads) {
+    for (int o = threadIdx.x; o < cc; o += 64 * W) {
       const int c = o / chi, e = o % chi;
       const cplx<double> a = gram_at<MT>(sum, c, e), b = gram_at<MT>(sum, e, c);
       const cplx<R> v = cast<R>(mk((a.x + b.x) * inv, (a.y - b.y) * inv));
       const cplx<R> old = min[pos * cc + o];
-      dnum = fmax(dnum, (double)cabs(v - old));
-      dden = fmax(dden, (double)cabs(v + old));
+      dnum = fmax(dnum, abs2(cast<double>(v - old)));
+      dden = fmax(dden, abs2(cast<double>(v + old)));
       mout[pos * cc + o] = v;
     }
     __syncthreads();
   }
   dnum = block_max(dnum, shred);
   dden = block_max(dden, shred);
-  if (threadIdx.x == 0) bp_end(st, cv.sweep, dnum, dden);
+  if (threadIdx.x == 0) bp_end(st, cv.sweep, sqrt(dnum), sqrt(dden));
 }
 
 // Extended messages: the Grams of the two physical halves (fibres [0, F / 2) and [F / 2, F), each
 // over half of the waves), assembled with the bond's ZZ-split gates (backends.py:393-404,519-526).
-template <typename RS, int MT>
-__global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_ext(ClassView cv, GemmPlan plan, int node0, int count,
+template <typename RS, int MT, int W>
+__global__ __launch_bounds__(64 * W) void k_gemm_gram_ext(ClassView cv, GemmPlan plan, int node0, int count,
                                                                 int chi, const cplx<RS>* __restrict__ T,
                                                                 cplx<double>* __restrict__ ext,
                                                                 const cplx<double>* ws) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int kSide = 16 * MT, kHalf = kGemmWaves / 2;
+  constexpr int kSide = 16 * MT, kHalf = W / 2, kAt = gram_slots<MT, W / 2>(2) * kSide * kSide;
   double* sum = reinterpret_cast<double*>(smem_raw);
   const int d = plan.d, wave = threadIdx.x >> 6, p = wave / kHalf, n2 = 2 * chi;
   const long S = 2L * ipow(chi, d);
@@ -395,23 +430,19 @@ __global__ __launch_bounds__(kGemmThreads) void k_gemm_gram_ext(ClassView cv, Ge
       for (int b = 0; b < MT; ++b) acc[a][b] = vec4<double>{0, 0, 0, 0};
     gram_sources<double, RS, MT>(acc, plan, k, chi, T + (size_t)i * S, ws + (size_t)node * plan.products * S, S,
                                  p * half, (p + 1) * half, wave % kHalf, kHalf);
-#pragma unroll 1
-    for (int w = 0; w < kHalf; ++w) {
-      if (w == wave % kHalf) add_tiles<double, MT>(sum + p * kSide * kSide, acc, w == 0);
-      __syncthreads();
-    }
+    sum_tiles<double, MT, kHalf>(sum, acc, p, wave % kHalf, 2);
     const cplx<double>* g = cv.zz + 2 * (size_t)cv.lmbd_pos[k * cv.n + i];
     const cplx<double> gs[2] = {g[0], g[1]};
     const double weight = abs2(gs[0]) + abs2(gs[1]);
     cplx<double> tr = mk(0.0, 0.0);
     for (int c = 0; c < chi; ++c)
-      tr = tr + gram_at<MT>(sum, c, c) + gram_at<MT>(sum + kSide * kSide, c, c);
+      tr = tr + gram_at<MT>(sum, c, c) + gram_at<MT>(sum + kAt, c, c);
     const cplx<double> inv = cinv(scale(tr, weight));
     cplx<double>* out = ext + (size_t)cv.out_pos[k * cv.n + i] * n2 * n2;
-    for (int o = threadIdx.x; o < n2 * n2; o += kGemmThreads) {
+    for (int o = threadIdx.x; o < n2 * n2; o += 64 * W) {
       const int row = o / n2, col = o % n2;
       const int s = row / chi, c = row % chi, s2 = col / chi, e = col % chi;
-      const cplx<double> g0 = gram_at<MT>(sum, c, e), g1 = gram_at<MT>(sum + kSide * kSide, c, e);
+      const cplx<double> g0 = gram_at<MT>(sum, c, e), g1 = gram_at<MT>(sum + kAt, c, e);
       out[o] = conj(gs[s]) * gs[s2] * (((s + s2) & 1) ? g0 - g1 : g0 + g1) * inv;
     }
     __syncthreads();
@@ -663,6 +694,18 @@ void by_chi_pair(int chi_in, int chi_out, F&& f) {
   }
 }
 
+// Waves per Gram: with few (node, output) items a Gram of four waves leaves most of the chip waiting for the loads of
+// its long fibre loop, so up to sixteen share it, to six waves a SIMD over the chip, as long as each has a group of
+// 16 fibres.  (Wider tiles need the registers of eight waves a CU, the widest FP64 ones of four.)
+template <typename R, int MT, typename F>
+void by_waves(int items, long fibres, F&& f) {
+  const long most = std::min<long>(6144 / std::max(items, 1), (fibres + 15) / 16);
+  constexpr int kMost = MT <= 2 ? 16 : sizeof(R) == 8 && MT == 4 ? 4 : 8;
+  if (kMost >= 16 && most >= 16) f.template operator()<(kMost >= 16 ? 16 : 4)>();
+  else if (kMost >= 8 && most >= 8) f.template operator()<(kMost >= 8 ? 8 : 4)>();
+  else f.template operator()<4>();
+}
+
 constexpr int kGramBlocks = 2048;   // eight blocks a CU; each keeps its maxima over its items
 
 }  // namespace
@@ -746,10 +789,13 @@ void gemm_bp(ClassView cv, int chi, const cplx<R>* T, cplx<R>* mA, cplx<R>* mB, 
   for (int node0 = 0; node0 < cv.n; node0 += chunk) {
     const int count = std::min(chunk, cv.n - node0);
     launch_products<R, R, R, true>(cv, plan, chi, node0, count, T, mA, mB, st, w, s);
-    const int grid = std::min(padded8(count) * cv.d, kGramBlocks);
+    const int items = padded8(count) * cv.d;
     by_chi(chi, [&]<int KS, int MT>() {
-      hipLaunchKernelGGL((k_gemm_gram_bp<R, MT>), dim3(grid), dim3(kGemmThreads), sizeof(double) * 256 * MT * MT, s,
-                         cv, plan, node0, count, chi, T, mA, mB, st, w);
+      by_waves<R, MT>(items, 2L * ipow(chi, cv.d - 1), [&]<int W>() {
+        hipLaunchKernelGGL((k_gemm_gram_bp<R, MT, W>), dim3(std::min(items, kGramBlocks)), dim3(64 * W),
+                           (sizeof(double) * 256 * MT * MT * gram_slots<MT, W>(1)), s, cv, plan, node0, count, chi, T, mA,
+                           mB, st, w);
+      });
     });
   }
 }
@@ -762,10 +808,13 @@ void gemm_ext(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msgs, cplx
   for (int node0 = 0; node0 < cv.n; node0 += chunk) {
     const int count = std::min(chunk, cv.n - node0);
     launch_products<double, R, R, false>(cv, plan, chi, node0, count, T, msgs, msgs, nullptr, w, s);
-    const int grid = std::min(padded8(count) * cv.d, kGramBlocks);
+    const int items = padded8(count) * cv.d;
     by_chi(chi, [&]<int KS, int MT>() {
-      hipLaunchKernelGGL((k_gemm_gram_ext<R, MT>), dim3(grid), dim3(kGemmThreads), 2 * sizeof(double) * 256 * MT * MT,
-                         s, cv, plan, node0, count, chi, T, ext, w);
+      by_waves<double, MT>(items, 2L * ipow(chi, cv.d - 1), [&]<int W>() {
+        hipLaunchKernelGGL((k_gemm_gram_ext<R, MT, W>), dim3(std::min(items, kGramBlocks)), dim3(64 * W),
+                           (2 * sizeof(double) * 256 * MT * MT * gram_slots<MT, W / 2>(2)), s, cv, plan, node0, count, chi,
+                           T, ext, w);
+      });
     });
   }
 }

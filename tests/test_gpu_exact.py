@@ -120,3 +120,39 @@ def test_z2_symmetric_30_qubits_have_zero_z():
     assert np.abs(got[:, 2]).max() < 1e-12
     assert np.all(np.linalg.norm(got, axis=1) <= 1.0 + 1e-12)
     assert np.abs(got[:, :2]).max() > 1e-3          # the state moved
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 8, 11, 12, 13, 16, 17, 19])
+def test_passes_at_every_split_of_the_qubits(n):
+    """Amplitudes, densities and Bloch vectors of two layers: less than a tile, a whole one, and later passes over
+    1, 4, 5, 7 qubits (after 12) against NumPy."""
+    from bqa_amd.native import StateVector
+    rng = np.random.default_rng(n)
+    h = rng.normal(size=n)
+    lhs, rhs = np.arange(n - 1), np.arange(1, n)
+    J = rng.normal(size=n - 1)
+    sv = StateVector(n, h, lhs, rhs, J)
+    try:
+        sv.init_state()
+        for x, z in ((0.3, 0.2), (0.15, 0.4)):
+            sv.run_layer(x, z)
+        psi = np.array(sv.state()).reshape(-1)
+        rho, bloch = sv.density()
+    finally:
+        sv.close()
+    bit = 1.0 - 2.0 * ((np.arange(1 << n)[:, None] >> np.arange(n)) & 1)
+    e = bit @ h + sum(j * bit[:, a] * bit[:, b] for a, b, j in zip(lhs, rhs, J))
+    want = bit.prod(axis=1) * 2.0 ** (-n / 2) + 0j
+    for x, z in ((0.3, 0.2), (0.15, 0.4)):
+        want = want * np.exp(-1j * z * e)
+        for q in range(n):
+            v = want.reshape(-1, 2, 1 << q)
+            want = (np.cos(x) * v - 1j * np.sin(x) * v[:, ::-1]).reshape(-1)
+    # n rotations and a phase a layer, each within a few units of rounding of unit-norm data
+    tol = 1.2e-16 * 16 * (n + 8)
+    assert np.abs(psi - want).max() < tol
+    for q in range(n):
+        v = want.reshape(-1, 2, 1 << q).transpose(1, 0, 2).reshape(2, -1)
+        ref = v @ v.conj().T
+        assert np.abs(np.asarray(rho)[q] - ref).max() < 2 * tol
+        assert abs(np.asarray(bloch)[q][2] - (ref[0, 0] - ref[1, 1]).real) < 4 * tol
