@@ -1,4 +1,7 @@
-// Canonicalisers and lambdas for n = 2 chi = 34..64, one edge per block of four waves.
+// Canonicalisers and lambdas for n = 2 chi = 34..64: a launch that factors the extended messages, a block of four
+// waves per edge and side, then one with a block per edge.  Both sides at once fill the chip twice as well on the few
+// hundred edges of the graphs that reach these bond dimensions (252 edges at n = 64: 0.75 + 0.72 against 2.10 ms with one
+// block per edge doing both in turn).
 //
 // The algorithm is k_canon_h's (kernels_canon_h.hpp): the Hermitian extended messages are factored by
 // pivoted Cholesky, one-sided Jacobi on the factor gives their eigenbases without accumulating
@@ -36,7 +39,7 @@ __device__ __forceinline__ double sum8(double v) {
 }
 
 struct WideShared {
-  double dg[64], sqf[64], ipf[64], sqb[64], ipb[64], norm[64], il[64];
+  double dg[64], norm[64], il[64];
   zd lcol[64];
   int rank_of[64], col_of[64];
   double red[4];
@@ -228,216 +231,247 @@ __device__ void wide_jacobi(zd* A, int n, WideShared& sh) {
   __syncthreads();
 }
 
+// An edge's workspace: U_f, U_b (n x n each) and the root weights and their inverses, sq_f, ip_f, sq_b, ip_b.
+struct WideSlot {
+  zd *Uf, *Ub;
+  double *sqf, *ipf, *sqb, *ipb;
+  __device__ __forceinline__ WideSlot(unsigned char* ws, size_t slot, int n) {
+    Uf = reinterpret_cast<zd*>(ws + slot * (2 * sizeof(zd) * n * n + 4 * sizeof(double) * n));
+    Ub = Uf + n * n;
+    sqf = reinterpret_cast<double*>(Ub + n * n);
+    ipf = sqf + n;
+    sqb = ipf + n;
+    ipb = sqb + n;
+  }
+};
+
+// Eigenbasis and root weights of one extended message: block (edge, side) of the edges from edge0.
 template <int NR>
-__global__ __launch_bounds__(kWideThreads) void k_canon_wide(const zd* __restrict__ ext, int E, int n, int ccols,
-                                                             double pinv_eps, double deps, zd* __restrict__ canon,
-                                                             double* __restrict__ lfull, zd* __restrict__ ws) {
+__global__ __launch_bounds__(kWideThreads) void k_wide_factor(const zd* __restrict__ ext, int E, int edge0, int n,
+                                                              double pinv_eps, double deps, unsigned char* ws) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr int RPL = NR / 8, LD = wide_ld<NR>();
   zd* A = reinterpret_cast<zd*>(smem_raw);
   WideShared& sh = *reinterpret_cast<WideShared*>(smem_raw + sizeof(zd) * LD * NR);
   const int t = threadIdx.x, pair = t >> 3, l8 = t & 7;
-  const int nn = n * n;
-  zd* Uf = ws + (size_t)blockIdx.x * 2 * nn;
-  zd* Ub = Uf + nn;
-  const int a0 = 4 * (t >> 4), c0 = 2 * (t & 15);   // the products below: 4 rows x 2 columns a thread
-
-  for (int edge = blockIdx.x; edge < E; edge += gridDim.x) {
-    for (int side = 0; side < 2; ++side) {
-      wide_cholesky<NR>(ext + (size_t)(side ? E + edge : edge) * nn, n, A, sh);
-      wide_jacobi<NR>(A, n, sh);
-      // columns are V_M sigma: eigenvalue s = sigma^2, U = column / sigma
-      zd* U = side ? Ub : Uf;
-      if (pair < n / 2) {
+  const int slot = blockIdx.x >> 1, side = blockIdx.x & 1, edge = edge0 + slot;
+  const WideSlot w(ws, slot, n);
+  wide_cholesky<NR>(ext + (size_t)(side ? E + edge : edge) * n * n, n, A, sh);
+  wide_jacobi<NR>(A, n, sh);
+  // columns are V_M sigma: eigenvalue s = sigma^2, U = column / sigma
+  zd* U = side ? w.Ub : w.Uf;
+  if (pair < n / 2) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int j = 2 * pair + h;
-          const double sig = sqrt(wide_norm2<NR>(A + j * LD, l8));
-          const double sqv = sig * sig > pinv_eps ? sig : 0.0;
-          if (l8 == 0) {
-            (side ? sh.sqb : sh.sqf)[j] = sqv;
-            (side ? sh.ipb : sh.ipf)[j] = sqv > deps ? 1.0 / sqv : 0.0;
-          }
-          const double inv = sig > 0.0 ? 1.0 / sig : 0.0;
-#pragma unroll
-          for (int x = 0; x < RPL; ++x) {
-            const int r = l8 + 8 * x;
-            if (r < n) U[j * n + r] = scale(A[j * LD + r], inv);
-          }
-        }
+    for (int h = 0; h < 2; ++h) {
+      const int j = 2 * pair + h;
+      const double sig = sqrt(wide_norm2<NR>(A + j * LD, l8));
+      const double sqv = sig * sig > pinv_eps ? sig : 0.0;
+      if (l8 == 0) {
+        (side ? w.sqb : w.sqf)[j] = sqv;
+        (side ? w.ipb : w.ipf)[j] = sqv > deps ? 1.0 / sqv : 0.0;
       }
-      __syncthreads();
+      const double inv = sig > 0.0 ? 1.0 / sig : 0.0;
+#pragma unroll
+      for (int x = 0; x < RPL; ++x) {
+        const int r = l8 + 8 * x;
+        if (r < n) U[j * n + r] = scale(A[j * LD + r], inv);
+      }
     }
-    // K[i][j] = sq_f[i] sq_b[j] conj(sum_t U_f[t, i] U_b[t, j]), a 4 x 4 block a thread; K's columns to A
-    // (rows n .. NR stay zero)
-    {
-      const int i0 = 4 * (t >> 4), j0 = 4 * (t & 15);
-      if (i0 < n && j0 < n) {
-        double ar[4][4] = {}, ai[4][4] = {};
-        const int imax = n - 1 - i0, jmax = n - 1 - j0;
-        for (int x = 0; x < n; ++x) {
-          zd f[4], b[4];
+  }
+}
+
+// The bond matrix, lambdas and canonicalisers of one edge from its two factors.
+template <int NR>
+__global__ __launch_bounds__(kWideThreads) void k_canon_wide(int E, int edge0, int n, int ccols, double pinv_eps,
+                                                             zd* __restrict__ canon, double* __restrict__ lfull,
+                                                             unsigned char* ws) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int LD = wide_ld<NR>();
+  zd* A = reinterpret_cast<zd*>(smem_raw);
+  WideShared& sh = *reinterpret_cast<WideShared*>(smem_raw + sizeof(zd) * LD * NR);
+  const int t = threadIdx.x, pair = t >> 3, l8 = t & 7;
+  const WideSlot w(ws, blockIdx.x, n);
+  const zd *Uf = w.Uf, *Ub = w.Ub;
+  const int a0 = 4 * (t >> 4), c0 = 2 * (t & 15);   // the products below: 4 rows x 2 columns a thread
+  const int edge = edge0 + (int)blockIdx.x;
+  // rows n .. NR of the columns are zero
+  for (int x = t; x < LD * NR; x += kWideThreads) A[x] = mk(0.0, 0.0);
+  __syncthreads();
+  // K[i][j] = sq_f[i] sq_b[j] conj(sum_t U_f[t, i] U_b[t, j]), a 4 x 4 block a thread; K's columns to A
+  // (rows n .. NR stay zero)
+  {
+    const int i0 = 4 * (t >> 4), j0 = 4 * (t & 15);
+    if (i0 < n && j0 < n) {
+      double ar[4][4] = {}, ai[4][4] = {};
+      const int imax = n - 1 - i0, jmax = n - 1 - j0;
+      for (int x = 0; x < n; ++x) {
+        zd f[4], b[4];
 #pragma unroll
-          for (int y = 0; y < 4; ++y) {
-            f[y] = Uf[(i0 + (y < imax ? y : imax)) * n + x];
-            b[y] = Ub[(j0 + (y < jmax ? y : jmax)) * n + x];
-          }
-#pragma unroll
-          for (int y = 0; y < 4; ++y)
-#pragma unroll
-            for (int z = 0; z < 4; ++z) {
-              ar[y][z] = fma(f[y].x, b[z].x, fma(-f[y].y, b[z].y, ar[y][z]));
-              ai[y][z] = fma(f[y].x, b[z].y, fma(f[y].y, b[z].x, ai[y][z]));
-            }
+        for (int y = 0; y < 4; ++y) {
+          f[y] = Uf[(i0 + (y < imax ? y : imax)) * n + x];
+          b[y] = Ub[(j0 + (y < jmax ? y : jmax)) * n + x];
         }
 #pragma unroll
         for (int y = 0; y < 4; ++y)
 #pragma unroll
-          for (int z = 0; z < 4; ++z)
-            if (y <= imax && z <= jmax) {
-              const double w = sh.sqf[i0 + y] * sh.sqb[j0 + z];
-              A[(j0 + z) * LD + i0 + y] = mk(w * ar[y][z], -w * ai[y][z]);
-            }
+          for (int z = 0; z < 4; ++z) {
+            ar[y][z] = fma(f[y].x, b[z].x, fma(-f[y].y, b[z].y, ar[y][z]));
+            ai[y][z] = fma(f[y].x, b[z].y, fma(f[y].y, b[z].x, ai[y][z]));
+          }
       }
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+          if (y <= imax && z <= jmax) {
+            const double wt = w.sqf[i0 + y] * w.sqb[j0 + z];
+            A[(j0 + z) * LD + i0 + y] = mk(wt * ar[y][z], -wt * ai[y][z]);
+          }
     }
-    __syncthreads();
-    wide_jacobi<NR>(A, n, sh);
+  }
+  __syncthreads();
+  wide_jacobi<NR>(A, n, sh);
 
-    // singular values, descending ranks, masks, normalised lambdas
-    if (pair < n / 2) {
+  // singular values, descending ranks, masks, normalised lambdas
+  if (pair < n / 2) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const double s = sqrt(wide_norm2<NR>(A + (2 * pair + h) * LD, l8));
-        if (l8 == 0) sh.norm[2 * pair + h] = s;
-      }
+    for (int h = 0; h < 2; ++h) {
+      const double s = sqrt(wide_norm2<NR>(A + (2 * pair + h) * LD, l8));
+      if (l8 == 0) sh.norm[2 * pair + h] = s;
     }
-    __syncthreads();
-    if (t < n) {
-      const double s = sh.norm[t];
-      int rank = 0;
-      double nrm2 = 0.0;
-      for (int j = 0; j < n; ++j) {
-        const double o = sh.norm[j];
-        rank += (o > s || (o == s && j < t)) ? 1 : 0;
-        nrm2 += o > pinv_eps ? o * o : 0.0;
-      }
-      const bool keep = s > pinv_eps;
-      sh.col_of[rank] = t;
-      sh.il[rank] = keep ? 1.0 / s : 0.0;
-      lfull[(size_t)edge * n + rank] = (keep ? s : 0.0) / sqrt(nrm2);
+  }
+  __syncthreads();
+  if (t < n) {
+    const double s = sh.norm[t];
+    int rank = 0;
+    double nrm2 = 0.0;
+    for (int j = 0; j < n; ++j) {
+      const double o = sh.norm[j];
+      rank += (o > s || (o == s && j < t)) ? 1 : 0;
+      nrm2 += o > pinv_eps ? o * o : 0.0;
     }
-    __syncthreads();
-    // with Us the masked left vectors of K (its columns over Lambda, by rank):
-    // V = U_f diag(sq_f) Us and C_f = U_f diag(ip_f) Us
-    zd* Cb = canon + (size_t)edge * n * ccols;
-    zd* Cf = canon + (size_t)(E + edge) * n * ccols;
-    const bool mine = a0 < n && c0 < ccols;
-    const int amax = n - 1 - a0;                     // clamps the rows of a partial block
-    double xr[4][2] = {}, xi[4][2] = {}, yr[4][2] = {}, yi[4][2] = {};
-    if (mine) {
-      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
-      const zd* k0 = A + sh.col_of[c0] * LD;
-      const zd* k1 = A + sh.col_of[c1] * LD;
-      const double l0 = sh.il[c0], l1 = sh.il[c1];
-      for (int x = 0; x < n; ++x) {
-        const zd us[2] = {scale(k0[x], l0), scale(k1[x], l1)};
-        const double sq = sh.sqf[x], ip = sh.ipf[x];
+    const bool keep = s > pinv_eps;
+    sh.col_of[rank] = t;
+    sh.il[rank] = keep ? 1.0 / s : 0.0;
+    lfull[(size_t)edge * n + rank] = (keep ? s : 0.0) / sqrt(nrm2);
+  }
+  __syncthreads();
+  // with Us the masked left vectors of K (its columns over Lambda, by rank):
+  // V = U_f diag(sq_f) Us and C_f = U_f diag(ip_f) Us
+  zd* Cb = canon + (size_t)edge * n * ccols;
+  zd* Cf = canon + (size_t)(E + edge) * n * ccols;
+  const bool mine = a0 < n && c0 < ccols;
+  const int amax = n - 1 - a0;                     // clamps the rows of a partial block
+  double xr[4][2] = {}, xi[4][2] = {}, yr[4][2] = {}, yi[4][2] = {};
+  if (mine) {
+    const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+    const zd* k0 = A + sh.col_of[c0] * LD;
+    const zd* k1 = A + sh.col_of[c1] * LD;
+    const double l0 = sh.il[c0], l1 = sh.il[c1];
+    for (int x = 0; x < n; ++x) {
+      const zd us[2] = {scale(k0[x], l0), scale(k1[x], l1)};
+      const double sq = w.sqf[x], ip = w.ipf[x];
 #pragma unroll
-        for (int y = 0; y < 4; ++y) {
-          const zd f = Uf[x * n + a0 + (y < amax ? y : amax)];
+      for (int y = 0; y < 4; ++y) {
+        const zd f = Uf[x * n + a0 + (y < amax ? y : amax)];
 #pragma unroll
-          for (int z = 0; z < 2; ++z) {
-            const double sr = sq * us[z].x, si = sq * us[z].y, pr = ip * us[z].x, pi = ip * us[z].y;
-            xr[y][z] = fma(f.x, sr, fma(-f.y, si, xr[y][z]));
-            xi[y][z] = fma(f.x, si, fma(f.y, sr, xi[y][z]));
-            yr[y][z] = fma(f.x, pr, fma(-f.y, pi, yr[y][z]));
-            yi[y][z] = fma(f.x, pi, fma(f.y, pr, yi[y][z]));
-          }
-        }
-      }
-#pragma unroll
-      for (int y = 0; y < 4; ++y)
-#pragma unroll
-        for (int z = 0; z < 2; ++z)
-          if (y <= amax && c0 + z < ccols) Cf[(a0 + y) * ccols + c0 + z] = mk(yr[y][z], yi[y][z]);
-    }
-    __syncthreads();
-    zd* V = A;   // V[c][a]
-    if (mine) {
-#pragma unroll
-      for (int y = 0; y < 4; ++y)
-#pragma unroll
-        for (int z = 0; z < 2; ++z)
-          if (y <= amax && c0 + z < ccols) V[(c0 + z) * LD + a0 + y] = mk(xr[y][z], xi[y][z]);
-    }
-    __syncthreads();
-    // Z[c][j] = keep_b[j] conj(sum_u U_b[u, j] V[u, c]) / Lambda_c
-    double zr[4][2] = {}, zi[4][2] = {};
-    if (mine) {
-      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
-      for (int x = 0; x < n; ++x) {
-        const zd v[2] = {V[c0 * LD + x], V[c1 * LD + x]};
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-          const zd b = Ub[(a0 + (y < amax ? y : amax)) * n + x];
-#pragma unroll
-          for (int z = 0; z < 2; ++z) {
-            zr[y][z] = fma(b.x, v[z].x, fma(-b.y, v[z].y, zr[y][z]));
-            zi[y][z] = fma(b.x, v[z].y, fma(b.y, v[z].x, zi[y][z]));
-          }
+        for (int z = 0; z < 2; ++z) {
+          const double sr = sq * us[z].x, si = sq * us[z].y, pr = ip * us[z].x, pi = ip * us[z].y;
+          xr[y][z] = fma(f.x, sr, fma(-f.y, si, xr[y][z]));
+          xi[y][z] = fma(f.x, si, fma(f.y, sr, xi[y][z]));
+          yr[y][z] = fma(f.x, pr, fma(-f.y, pi, yr[y][z]));
+          yi[y][z] = fma(f.x, pi, fma(f.y, pr, yi[y][z]));
         }
       }
     }
-    __syncthreads();
-    zd* Z = A;   // Z[c][j]
-    if (mine) {
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+    for (int y = 0; y < 4; ++y)
 #pragma unroll
-        for (int z = 0; z < 2; ++z)
-          if (y <= amax && c0 + z < ccols) {
-            const double w = sh.ipb[a0 + y] > 0.0 ? sh.il[c0 + z] : 0.0;
-            Z[(c0 + z) * LD + a0 + y] = mk(zr[y][z] * w, -zi[y][z] * w);
-          }
-    }
-    __syncthreads();
-    // C_b[a][c] = sum_j U_b[a, j] Z[c][j]
-    if (mine) {
-      double br[4][2] = {}, bi[4][2] = {};
-      const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
-      for (int x = 0; x < n; ++x) {
-        const zd z[2] = {Z[c0 * LD + x], Z[c1 * LD + x]};
+      for (int z = 0; z < 2; ++z)
+        if (y <= amax && c0 + z < ccols) Cf[(a0 + y) * ccols + c0 + z] = mk(yr[y][z], yi[y][z]);
+  }
+  __syncthreads();
+  zd* V = A;   // V[c][a]
+  if (mine) {
 #pragma unroll
-        for (int y = 0; y < 4; ++y) {
-          const zd b = Ub[x * n + a0 + (y < amax ? y : amax)];
+    for (int y = 0; y < 4; ++y)
 #pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            br[y][q] = fma(b.x, z[q].x, fma(-b.y, z[q].y, br[y][q]));
-            bi[y][q] = fma(b.x, z[q].y, fma(b.y, z[q].x, bi[y][q]));
-          }
+      for (int z = 0; z < 2; ++z)
+        if (y <= amax && c0 + z < ccols) V[(c0 + z) * LD + a0 + y] = mk(xr[y][z], xi[y][z]);
+  }
+  __syncthreads();
+  // Z[c][j] = keep_b[j] conj(sum_u U_b[u, j] V[u, c]) / Lambda_c
+  double zr[4][2] = {}, zi[4][2] = {};
+  if (mine) {
+    const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+    for (int x = 0; x < n; ++x) {
+      const zd v[2] = {V[c0 * LD + x], V[c1 * LD + x]};
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const zd b = Ub[(a0 + (y < amax ? y : amax)) * n + x];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+          zr[y][z] = fma(b.x, v[z].x, fma(-b.y, v[z].y, zr[y][z]));
+          zi[y][z] = fma(b.x, v[z].y, fma(b.y, v[z].x, zi[y][z]));
         }
       }
-#pragma unroll
-      for (int y = 0; y < 4; ++y)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-          if (y <= amax && c0 + q < ccols) Cb[(a0 + y) * ccols + c0 + q] = mk(br[y][q], bi[y][q]);
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  zd* Z = A;   // Z[c][j]
+  if (mine) {
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+      for (int z = 0; z < 2; ++z)
+        if (y <= amax && c0 + z < ccols) {
+          const double wt = w.ipb[a0 + y] > 0.0 ? sh.il[c0 + z] : 0.0;
+          Z[(c0 + z) * LD + a0 + y] = mk(zr[y][z] * wt, -zi[y][z] * wt);
+        }
+  }
+  __syncthreads();
+  // C_b[a][c] = sum_j U_b[a, j] Z[c][j]
+  if (mine) {
+    double br[4][2] = {}, bi[4][2] = {};
+    const int c1 = c0 + 1 < ccols ? c0 + 1 : c0;
+    for (int x = 0; x < n; ++x) {
+      const zd z[2] = {Z[c0 * LD + x], Z[c1 * LD + x]};
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const zd b = Ub[x * n + a0 + (y < amax ? y : amax)];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          br[y][q] = fma(b.x, z[q].x, fma(-b.y, z[q].y, br[y][q]));
+          bi[y][q] = fma(b.x, z[q].y, fma(b.y, z[q].x, bi[y][q]));
+        }
+      }
+    }
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (y <= amax && c0 + q < ccols) Cb[(a0 + y) * ccols + c0 + q] = mk(br[y][q], bi[y][q]);
   }
 }
 
 template <int NR>
 void launch_wide(const zd* ext, int E, int n, int ccols, double pinv_eps, double deps, zd* canon, double* lambdas,
-                 zd* ws, hipStream_t s) {
+                 unsigned char* ws, hipStream_t s) {
   constexpr int lds = sizeof(zd) * wide_ld<NR>() * NR + sizeof(WideShared);
   static const bool once = [] {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_canon_wide<NR>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+    bool ok = true;
+    for (const void* k : {reinterpret_cast<const void*>(&k_wide_factor<NR>), reinterpret_cast<const void*>(&k_canon_wide<NR>)})
+      ok = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess && ok;
+    return ok;
   }();
   (void)once;   // a refusal shows as the launch's own error
-  hipLaunchKernelGGL((k_canon_wide<NR>), dim3(std::min(E, kCanonWideBlocks)), dim3(kWideThreads), lds, s, ext, E, n,
-                     ccols, pinv_eps, deps, canon, lambdas, ws);
+  for (int edge0 = 0; edge0 < E; edge0 += kCanonWideEdges) {
+    const int count = std::min(kCanonWideEdges, E - edge0);
+    hipLaunchKernelGGL((k_wide_factor<NR>), dim3(2 * count), dim3(kWideThreads), lds, s, ext, E, edge0, n, pinv_eps, deps,
+                       ws);
+    hipLaunchKernelGGL((k_canon_wide<NR>), dim3(count), dim3(kWideThreads), lds, s, E, edge0, n, ccols, pinv_eps, canon,
+                       lambdas, ws);
+  }
 }
 
 }  // namespace
@@ -445,7 +479,7 @@ void launch_wide(const zd* ext, int E, int n, int ccols, double pinv_eps, double
 void canon_wide(const zd* ext, int E, int chi, int ccols, double pinv_eps, double dtype_eps, zd* canon,
                 double* lambdas, void* ws, hipStream_t s) {
   const int n = 2 * chi;
-  zd* w = reinterpret_cast<zd*>(ws);
+  unsigned char* w = reinterpret_cast<unsigned char*>(ws);
   if (n <= 40)
     launch_wide<40>(ext, E, n, ccols, pinv_eps, dtype_eps, canon, lambdas, w, s);
   else if (n <= 48)

@@ -9,11 +9,12 @@ namespace bqa {
 
 inline bool canon_wide_shape(int chi) { return chi >= 17 && chi <= 32; }
 
-// Blocks that run at once take the edges in turn, each with one workspace slot (the bases of both sides).
-constexpr int kCanonWideBlocks = 512;
+// Edges per round of launches, each with one workspace slot (the bases and root weights of both sides).
+constexpr int kCanonWideEdges = 512;
+inline size_t canon_wide_slot(int n) { return 2 * sizeof(cplx<double>) * n * n + 4 * sizeof(double) * n; }
 inline size_t canon_wide_ws_bytes(int E, int chi) {
-  const size_t blocks = E < kCanonWideBlocks ? E : kCanonWideBlocks;
-  return blocks * 2 * sizeof(cplx<double>) * 4 * chi * chi;
+  const size_t edges = E < kCanonWideEdges ? E : kCanonWideEdges;
+  return edges * canon_wide_slot(2 * chi);
 }
 
 void canon_wide(const cplx<double>* ext, int E, int chi, int ccols, double pinv_eps, double dtype_eps,

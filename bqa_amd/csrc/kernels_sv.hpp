@@ -15,7 +15,7 @@
 // first pass takes contiguous tiles (qubits 0..11, with the diagonal phase on the way in); later passes take 2^cb
 // contiguous amplitudes (cb >= 4: 256-byte rows and more) times the 2^t values of t = 12 - cb <= 8 higher qubits.
 // Bounded by memory: a rotation pass reads and writes the state once, a readout pass reads it.  At 26 qubits (1 GB)
-// a layer is three passes and the readout three reads; with tiles of 1,024 amplitudes and every rotation through
+// a layer is three passes and the readout three reads (0.70 + 2 x 0.41 and 0.72 ms); with tiles of 1,024 amplitudes and every rotation through
 // LDS they were four passes (2.0 ms a layer) and the readout took 9.6 ms, most of it in lane reductions of every
 // qubit of every tile and in a serial sum over the blocks.
 #pragma once
@@ -146,11 +146,13 @@ __device__ __forceinline__ void sv_store(const double (&v)[4][4], double* s, dou
   }
 }
 
+// Two waves a SIMD: the sixteen sincos of a thread then run interleaved (26 qubits: 0.70 ms; held to the registers of
+// three or four waves 0.89 and 1.09 ms).
 // First pass: tiles of 2^tb contiguous amplitudes (tb = min(n, 12); with fewer qubits the tile's other elements are
 // zero).  MODE 0: diagonal phase exp(-i ztime Ez) (when ez != nullptr), then the X rotations of qubits 0..tb-1.
 // MODE 1: readout sums of qubits 0..tb-1 into part.
 template <int MODE>
-__global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_low(cplx<double>* __restrict__ psi, int n,
+__global__ __launch_bounds__(kSvThreads, 2) void k_sv_low(cplx<double>* __restrict__ psi, int n,
                                                        const double* __restrict__ ez, double ztime, double c,
                                                        double sn, double* part) {
   __shared__ double s[1 << kSvTileBits];
@@ -174,7 +176,6 @@ __global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_low(cplx<d
         double sp, cp;
         sincos(k < size ? -ztime * e[k] : 0.0, &sp, &cp);
         a[j] = a[j] * mk(cp, sp);
-        __builtin_amdgcn_sched_barrier(0);   // one sincos's temporaries at a time
       }
     }
     if (MODE == 0) {
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_low(cplx<d
 // qubits, the t bits above them the pass's qubits; the tile number T the remaining bits (those between cb and b0,
 // then those above b0 + t).  Readout sums of tile bits below cb are not used.
 template <int MODE>
-__global__ __launch_bounds__(kSvThreads, MODE == 0 ? 4 : 2) void k_sv_high(cplx<double>* __restrict__ psi, int n, int b0, int t,
+__global__ __launch_bounds__(kSvThreads, MODE == 0 ? 3 : 2) void k_sv_high(cplx<double>* __restrict__ psi, int n, int b0, int t,
                                                         double c, double sn, double* part) {
   __shared__ double s[1 << kSvTileBits];
   const int cb = kSvTileBits - t, mid = b0 - cb;
