@@ -185,11 +185,48 @@ __device__ inline int bp_begin(BpStatus* st, int sweep) {
   return st->cur ^ (sweep & 1);
 }
 
-// This block's distance maxima of sweep `sweep` (one thread per block).
+// This block's distance maxima of sweep `sweep` (one thread per block).  The atomics of a launch meet at one address
+// and take about 15 ns each, so in a launch of many blocks, whose ends spread over time, a block first looks whether
+// its maxima are above the ones so far (few are); in a small launch all blocks end together and the look only adds
+// its latency.
 __device__ inline void bp_end(BpStatus* st, int sweep, double dnum, double dden) {
   if (sweep >= 0) sweep += st->base;
-  atomic_max_nonneg(sweep < 0 ? &st->num_bits : &st->slot[sweep][0], dnum);
-  atomic_max_nonneg(sweep < 0 ? &st->den_bits : &st->slot[sweep][1], dden);
+  unsigned long long* num = sweep < 0 ? &st->num_bits : &st->slot[sweep][0];
+  unsigned long long* den = sweep < 0 ? &st->den_bits : &st->slot[sweep][1];
+  if (gridDim.x > 512) {
+    const double n0 = __longlong_as_double((long long)__hip_atomic_load(num, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const double d0 = __longlong_as_double((long long)__hip_atomic_load(den, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    // negated, so that a NaN on either side goes on to the atomic
+    if (!(dnum <= n0)) atomic_max_nonneg(num, dnum);
+    if (!(dden <= d0)) atomic_max_nonneg(den, dden);
+    return;
+  }
+  atomic_max_nonneg(num, dnum);
+  atomic_max_nonneg(den, dden);
+}
+
+// The same from several waves of a block (WAVES of them, from wave 0 on, with a value in every lane): one update per
+// block.  All threads call it; `sh` (2 WAVES doubles of LDS) is free by then.
+template <int WAVES>
+__device__ __forceinline__ void bp_end_waves(BpStatus* st, int sweep, double dnum2, double dden2, double* sh) {
+  for (int o = 32; o > 0; o >>= 1) {
+    dnum2 = fmax(dnum2, __shfl_xor(dnum2, o, 64));
+    dden2 = fmax(dden2, __shfl_xor(dden2, o, 64));
+  }
+  const int w = threadIdx.x >> 6;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0 && w < WAVES) {
+    sh[2 * w] = dnum2;
+    sh[2 * w + 1] = dden2;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < WAVES; ++q) {
+      dnum2 = fmax(dnum2, sh[2 * q]);
+      dden2 = fmax(dden2, sh[2 * q + 1]);
+    }
+    bp_end(st, sweep, sqrt(dnum2), sqrt(dden2));
+  }
 }
 
 }  // namespace bqa

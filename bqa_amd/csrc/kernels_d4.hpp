@@ -327,13 +327,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4 * (sizeof(R) == sizeof(float) ? 2 :
     }
     __syncthreads();  // the sums are read, the next node's messages in place
   }
-  if (io) {
-    for (int d = 32; d > 0; d >>= 1) {
-      dnum = fmax(dnum, __shfl_xor(dnum, d, 64));
-      dden = fmax(dden, __shfl_xor(dden, d, 64));
-    }
-    if (o == 0) bp_end(st, cv.sweep, sqrt(dnum), sqrt(dden));
-  }
+  bp_end_waves<4>(st, cv.sweep, dnum, dden, reinterpret_cast<double*>(d4_lds));
 }
 
 template <typename R, int NW>

@@ -11,6 +11,7 @@
 #include "kernels_local.hpp"
 #include "kernels_small.hpp"
 #include "kernels_d4.hpp"
+#include "kernels_d3.hpp"
 
 namespace bqa {
 
@@ -114,15 +115,13 @@ bool fast_ext_launch(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msg
     if constexpr (sizeof(R) == sizeof(float)) {
       // FP32 job: FP32 MFMA mode products, FP64 MFMA Gram
       if (cv.d == 3)
-        hipLaunchKernelGGL((k_mfma8_ext32<3, 4>), dim3(node_grid<k_mfma8_ext32<3, 4>, 256>(cv.n)), dim3(256), 0, s,
-                           cv, T, msgs, ext);
+        launch_ext_d3c8<R>(cv, T, msgs, ext, s);
       else
         hipLaunchKernelGGL((k_mfma8_ext32<2, 1>), dim3(node_grid<k_mfma8_ext32<2, 1>, 64>(cv.n)), dim3(64), 0, s, cv,
                            T, msgs, ext);
     } else {
       if (cv.d == 3)
-        hipLaunchKernelGGL((k_mfma8_ext64<3, 4, R>), dim3(node_grid<k_mfma8_ext64<3, 4, R>, 256>(cv.n)), dim3(256),
-                           0, s, cv, T, msgs, ext);
+        launch_ext_d3c8<R>(cv, T, msgs, ext, s);
       else
         hipLaunchKernelGGL((k_mfma8_ext64<2, 1, R>), dim3(node_grid<k_mfma8_ext64<2, 1, R>, 64>(cv.n)), dim3(64), 0,
                            s, cv, T, msgs, ext);
@@ -221,7 +220,7 @@ inline bool fast_bp_launch<float>(ClassView cv, int chi, const cplx<float>* T, c
   if (cv.d == 2)
     launch_mfma8_d<kModeBP, 2>(cv, T, mA, mB, st, nullptr, nullptr, s, v);
   else
-    launch_mfma8_d<kModeBP, 3>(cv, T, mA, mB, st, nullptr, nullptr, s, v);
+    launch_bp_d3c8<float>(cv, T, mA, mB, st, s, v);
   return true;
 }
 
@@ -242,9 +241,8 @@ inline int bp_variant_count<double>(int d, int chi) {
 
 template <>
 inline const char* bp_variant_name<double>(int d, int chi, int v) {
-  static const char* b3[kGridPolicies + 1] = {"k_mfma8_bp64_3p<4>, resident SIMD-rounded",
-                                              "k_mfma8_bp64_3p<4>, resident", "k_mfma8_bp64_3p<4>, 2x resident",
-                                              "k_mfma8_bp64_3p<2>, resident SIMD-rounded"};
+  static const char* b3[kGridPolicies + 1] = {"k_bp_d3c8, resident SIMD-rounded", "k_bp_d3c8, resident",
+                                              "k_bp_d3c8, 2x resident", "k_mfma8_bp64_3p<4>, resident SIMD-rounded"};
   static const char* b2[kGridPolicies] = {"k_mfma8_bp64<2,1>, resident SIMD-rounded", "k_mfma8_bp64<2,1>, resident",
                                           "k_mfma8_bp64<2,1>, 2x resident"};
   static const char* sm[kGridPolicies + 2] = {"k_small, 8192 blocks", "k_small, resident", "k_small, 2x resident",
@@ -288,11 +286,10 @@ inline bool fast_bp_launch<double>(ClassView cv, int chi, const cplx<double>* T,
     return launch_small<kModeBP, double, double>(cv, chi, T, mA, mB, st, nullptr, nullptr, nullptr, s, v);
   if (cv.d == 3) {
     if (v == kGridPolicies)
-      hipLaunchKernelGGL((k_mfma8_bp64_3p<2>), dim3(node_grid<k_mfma8_bp64_3p<2>, 128>(cv.n)), dim3(128), 0, s, cv,
+      hipLaunchKernelGGL((k_mfma8_bp64_3p<4>), dim3(node_grid<k_mfma8_bp64_3p<4>, 256>(cv.n)), dim3(256), 0, s, cv,
                          T, mA, mB, st);
     else
-      hipLaunchKernelGGL((k_mfma8_bp64_3p<4>), dim3(policy_grid<k_mfma8_bp64_3p<4>, 256>(cv.n, v)), dim3(256), 0, s,
-                         cv, T, mA, mB, st);
+      launch_bp_d3c8<double>(cv, T, mA, mB, st, s, v);
   } else {
     hipLaunchKernelGGL((k_mfma8_bp64<2, 1>), dim3(policy_grid<k_mfma8_bp64<2, 1>, 64>(cv.n, v)), dim3(64), 0, s, cv,
                        T, mA, mB, st);
@@ -354,8 +351,8 @@ inline bool launch_bp_multi(int fam, int d, int chi, const BpEntry* tab, int ent
         hipLaunchKernelGGL((k_mfma8_multi<2>), dim3(policy_grid<k_mfma8_multi<2>, 64>(total, 0)), dim3(64), 0, s, tab,
                            entries, sweep);
       else
-        hipLaunchKernelGGL((k_mfma8_multi<3>), dim3(policy_grid<k_mfma8_multi<3>, 64>(total, 0)), dim3(64), 0, s, tab,
-                           entries, sweep);
+        hipLaunchKernelGGL((k_bp_d3c8_multi<R>), dim3(policy_grid<k_bp_d3c8_multi<R>, 256>(total, 0)), dim3(256), 0, s,
+                           tab, entries, sweep);
       return true;
     }
     return false;
