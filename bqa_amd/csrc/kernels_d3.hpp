@@ -7,6 +7,10 @@
 // which also fill its LDS copy; Y_1 and Y_0 go from their product's registers into their first Gram's MFMAs, and
 // through LDS (Y_0 in T's place) only for out_2.  The messages are loaded from memory as MFMA operands.  Everything
 // a node reads from memory is loaded while the node before computes, its positions one node earlier.
+// What bounds it: 192 MFMAs a node (0.50 ms FP64, 0.25 ms FP32 a sweep of 100,000 nodes at the matrix rate), with four
+// short phases a node between barriers; three (FP64) and five (FP32) nodes share a CU.  Measured at 100,000 nodes:
+// FP64 0.85 ms a sweep, FP32 0.52 ms; extended messages 1.19 and 1.17 ms.  The kernels that ran products and Grams
+// through LDS took 1.05 ms (six contractions), 0.67 ms (nine), 1.68 and 1.14 ms.
 #pragma once
 
 #include "common.hpp"
@@ -338,7 +342,12 @@ __global__ __launch_bounds__(256, 3) void k_ext_d3c8(ClassView cv, const cplx<R>
 
 template <typename R>
 inline void launch_bp_d3c8(ClassView cv, const cplx<R>* T, cplx<R>* mA, cplx<R>* mB, BpStatus* st, hipStream_t s, int policy) {
-  hipLaunchKernelGGL((k_bp_d3c8<R>), dim3(policy_grid<k_bp_d3c8<R>, 256>(cv.n, policy)), dim3(256), 0, s, cv, T, mA, mB, st);
+  int grid = policy_grid<k_bp_d3c8<R>, 256>(cv.n, policy < kGridPolicies ? policy : 0);
+  if (policy >= kGridPolicies) {   // as many blocks as give each the same number of nodes, but for one
+    const int rounds = (cv.n + grid - 1) / grid;
+    grid = (cv.n + rounds - 1) / rounds;
+  }
+  hipLaunchKernelGGL((k_bp_d3c8<R>), dim3(grid), dim3(256), 0, s, cv, T, mA, mB, st);
 }
 
 template <typename R>

@@ -155,7 +155,7 @@ inline void launch_mfma16_bp3h(ClassView cv, const cplx<float>* T, cplx<float>* 
 //   chi = 16, d = 3: k_mfma16_bp<3, W>, W = 8 or 4 waves per node (one node per CU, 128 KB LDS),
 //   k_mfma16_bp3h<8> (three products per node, 96 KB LDS);
 //   chi = 16, d = 2: k_mfma16_bp<2, 1>, one or two resident rounds;
-//   chi = 8, d = 2, 3: k_mfma8 (one wave per node) under the three grid policies;
+//   chi = 8, d = 3: k_bp_d3c8, d = 2: k_mfma8 (one wave per node), under the three grid policies;
 //   chi = 8, d = 4: k_bp_d4c8, eight waves per node and two nodes per CU;
 //   other served shapes: k_small under the three grid policies, and for degree 2, 3 with chi <= 4
 //   also k_small_npw with 2 and 4 nodes per wave.
@@ -179,12 +179,14 @@ inline const char* bp_variant_name<float>(int d, int chi, int v) {
   static const char* sm[kGridPolicies + 2] = {"k_small, 8192 blocks", "k_small, resident", "k_small, 2x resident",
                                               "k_small_npw<2> (2 nodes per wave), resident",
                                               "k_small_npw<4> (4 nodes per wave), resident"};
-  if (chi == 8 && (d == 2 || d == 3)) return m8[v % kGridPolicies];
+  static const char* d3[kGridPolicies] = {"k_bp_d3c8, resident SIMD-rounded", "k_bp_d3c8, resident",
+                                          "k_bp_d3c8, 2x resident"};
+  if (chi == 8 && d == 3) return d3[v % kGridPolicies];
+  if (chi == 8 && d == 2) return m8[v % kGridPolicies];
   return small_bp_shape<float>(d, chi) ? sm[v % (kGridPolicies + 2)] : "generic";
 }
 
-// FP32, chi = 8, degree 2 or 3: k_mfma8, one wave per node (two and four waves per node for
-// degree 3 measured no faster).
+// FP32, chi = 8: k_mfma8, one wave per node (BP at degree 2, the readout at degrees 2 and 3).
 template <int MODE, int D>
 inline void launch_mfma8_d(ClassView cv, const cplx<float>* T, cplx<float>* mA, cplx<float>* mB, BpStatus* st,
                            double* rho, double* bloch, hipStream_t s, int policy) {
@@ -225,8 +227,8 @@ inline bool fast_bp_launch<float>(ClassView cv, int chi, const cplx<float>* T, c
 }
 
 // FP64 BP sweep variants.
-//   chi = 8, d = 3: k_mfma8_bp64_3p<4> (six contractions per node over four waves) under the three
-//     grid policies, and k_mfma8_bp64_3p<2> (two waves per node);
+//   chi = 8, d = 3: k_bp_d3c8 under the three grid policies, and with the nodes spread evenly over
+//     the rounds of a resident grid;
 //   chi = 8, d = 2: k_mfma8_bp64<2, 1> (one wave per node) under the three grid policies;
 //   chi = 8, d = 4: k_bp_d4c8, sixteen waves per node (1.18 ms a sweep of 9,604 nodes; eight: 1.30 ms);
 //   other served shapes: k_small under the three grid policies, and for degree 2, 3 with chi <= 4
@@ -242,7 +244,7 @@ inline int bp_variant_count<double>(int d, int chi) {
 template <>
 inline const char* bp_variant_name<double>(int d, int chi, int v) {
   static const char* b3[kGridPolicies + 1] = {"k_bp_d3c8, resident SIMD-rounded", "k_bp_d3c8, resident",
-                                              "k_bp_d3c8, 2x resident", "k_mfma8_bp64_3p<4>, resident SIMD-rounded"};
+                                              "k_bp_d3c8, 2x resident", "k_bp_d3c8, resident, even rounds"};
   static const char* b2[kGridPolicies] = {"k_mfma8_bp64<2,1>, resident SIMD-rounded", "k_mfma8_bp64<2,1>, resident",
                                           "k_mfma8_bp64<2,1>, 2x resident"};
   static const char* sm[kGridPolicies + 2] = {"k_small, 8192 blocks", "k_small, resident", "k_small, 2x resident",
@@ -285,11 +287,7 @@ inline bool fast_bp_launch<double>(ClassView cv, int chi, const cplx<double>* T,
   if (chi != 8 || cv.n == 0 || (cv.d != 2 && cv.d != 3))
     return launch_small<kModeBP, double, double>(cv, chi, T, mA, mB, st, nullptr, nullptr, nullptr, s, v);
   if (cv.d == 3) {
-    if (v == kGridPolicies)
-      hipLaunchKernelGGL((k_mfma8_bp64_3p<4>), dim3(node_grid<k_mfma8_bp64_3p<4>, 256>(cv.n)), dim3(256), 0, s, cv,
-                         T, mA, mB, st);
-    else
-      launch_bp_d3c8<double>(cv, T, mA, mB, st, s, v);
+    launch_bp_d3c8<double>(cv, T, mA, mB, st, s, v);
   } else {
     hipLaunchKernelGGL((k_mfma8_bp64<2, 1>), dim3(policy_grid<k_mfma8_bp64<2, 1>, 64>(cv.n, v)), dim3(64), 0, s, cv,
                        T, mA, mB, st);
@@ -298,10 +296,11 @@ inline bool fast_bp_launch<double>(ClassView cv, int chi, const cplx<double>* T,
 }
 
 // Multi-job BP launches (the serving batch): which kernel serves a class of a job of
-// precision R in a launch shared with other jobs -- 1 k_small_multi, 2 k_mfma8_multi, or 0
+// precision R in a launch shared with other jobs -- 1 k_small_multi, 2 the MFMA kernels, or 0
 // when the class keeps its own launches.  Only shapes whose single-job launch runs the same
 // node code are shared, so a job's results are the same in a batch as alone.
-// Shared-launch families: 1 k_small_multi (variant 0's arithmetic), 2 k_mfma8_multi, kFamNpw
+// Shared-launch families: 1 k_small_multi (variant 0's arithmetic), 2 k_mfma8_multi (d = 2) and
+// k_bp_d3c8_multi (d = 3), kFamNpw
 // k_small_npw_multi with kNpwShared nodes per wave (for jobs whose BP variants are autotuned: the
 // Grams' fibre split, and so the rounding, differs from variant 0), 0 none.
 constexpr int kFamNpw = 3;
