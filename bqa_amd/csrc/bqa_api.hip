@@ -611,20 +611,22 @@ void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first) {
 
 // ------------------------------------------------------- graph chunks --
 
-constexpr int kGraphSweeps = 4;
+// Sweeps of a replay: four, or sixteen where the chunk has that many left (a replay costs its launch, several times a
+// small job's sweep, so a long run takes few).
+constexpr int kGraphSweeps = 4, kGraphLongSweeps = 16;
 constexpr size_t kMaxGraphs = 8;
 // Eager BP runs at one bond dimension before its chunks are captured: a capture and
 // instantiation cost about as much as the launches of tens of sweeps, so graphs
 // serve the steady state, not the steps of the bond-dimension ramp.
 constexpr int kGraphWarmRuns = 8;
 
-// The chunk graph for the current buffers and launch variants, captured on first use.  Capture
+// The graph of `sweeps` sweeps for the current buffers and launch variants, captured on first use.  Capture
 // uses the thread-local mode: other threads (other jobs) keep calling the runtime meanwhile,
 // which the global mode would refuse, failing their calls.
 template <typename R>
-hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants) {
+hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants, int sweeps) {
   const int chi = j->chi;
-  std::vector<intptr_t> key = {chi, (intptr_t)j->msgs[0].p, (intptr_t)j->msgs[1].p, (intptr_t)j->status.p};
+  std::vector<intptr_t> key = {chi, sweeps, (intptr_t)j->msgs[0].p, (intptr_t)j->msgs[1].p, (intptr_t)j->status.p};
   for (size_t ci = 0; ci < j->cls.size(); ++ci) {
     const ClassDev& c = j->cls[ci];
     key.push_back((intptr_t)c.T[c.tcur].p);
@@ -638,7 +640,7 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants) {
   std::unique_lock<std::mutex> lock(g_capture_mu);
   HIPX(hipStreamBeginCapture(j->stream, hipStreamCaptureModeThreadLocal));
   try {
-    for (int s = 0; s < kGraphSweeps; ++s)
+    for (int s = 0; s < sweeps; ++s)
       for (size_t ci = 0; ci < j->cls.size(); ++ci) {
         ClassDev& c = j->cls[ci];
         if (c.d == 0 || c.n == 0) continue;
@@ -649,7 +651,7 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants) {
           throw BqaError(BQA_ERR_HIP, "no specialised BP kernel for a captured class");
         LAUNCH_CHECK();
       }
-    hipLaunchKernelGGL(k_bp_advance, dim3(1), dim3(1), 0, j->stream, st, kGraphSweeps);
+    hipLaunchKernelGGL(k_bp_advance, dim3(1), dim3(1), 0, j->stream, st, sweeps);
     LAUNCH_CHECK();
   } catch (...) {
     hipGraph_t dead = nullptr;
@@ -747,16 +749,20 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
   }
   while (launched < max_iters) {
     int c = std::min(chunk, max_iters - launched);
-    const hipGraphExec_t exec = graph ? bp_graph<R>(j, variants) : nullptr;
-    if (graph && !exec) graph = false;
+    // both graphs before the first replay: eager sweeps count from the run's first one, replays from the last
+    const hipGraphExec_t exec = graph ? bp_graph<R>(j, variants, kGraphSweeps) : nullptr;
+    const hipGraphExec_t exec_long = exec && c >= kGraphLongSweeps ? bp_graph<R>(j, variants, kGraphLongSweeps) : exec;
+    if (graph && !exec_long) graph = false;
     if (graph) {
       // whole replays: their sweeps beyond max_iters, or after convergence, exit at once
-      const int reps = (c + kGraphSweeps - 1) / kGraphSweeps;
-      for (int r = 0; r < reps; ++r) {
-        HIPX(hipGraphLaunch(exec, j->stream));
+      int replayed = 0;
+      while (replayed < c) {
+        const bool lengthy = c - replayed >= kGraphLongSweeps;
+        HIPX(hipGraphLaunch(lengthy ? exec_long : exec, j->stream));
         ++j->graph_launches;
+        replayed += lengthy ? kGraphLongSweeps : kGraphSweeps;
       }
-      c = reps * kGraphSweeps;
+      c = replayed;
     } else {
       for (int s = 0; s < c; ++s) {
         for (auto& cl : j->cls) launch_bp_class<R>(j, cl, slots ? launched + s : -1, launched + s == 0);
@@ -865,6 +871,13 @@ void ext_class(bqa_job* j, ClassDev& c, double ztime, const cplx<double>* msgs64
     LAUNCH_CHECK();
     return;
   }
+  if (!j->generic(kGenExt) && chi == 1) {
+    if (c.n > 0 && c.d > 0)
+      hipLaunchKernelGGL((k_ext_chi1<R>), dim3(grid_for((long)c.n * c.d)), dim3(256), 0, j->stream, v, T,
+                         msg_ptr<R>(j, j->mcur), ext);
+    LAUNCH_CHECK();
+    return;
+  }
   if (!j->generic(kGenExt) && gemm_shape(c.d, chi) && j->hermitian) {
     const int chunk = plan_gemm(j, c, chi, sizeof(cplx<double>));
     gemm_ext<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->gws.p, chunk, j->stream);
@@ -912,7 +925,7 @@ void ext_and_canon(bqa_job* j, double ztime, double pinv_eps, bool sync = true, 
   bool need_generic = false;
   for (auto& c : j->cls)
     need_generic |= c.d != 0 && c.n > 0 &&
-                    (j->generic(kGenExt) || !(ext_fast_shape<R>(c.d, chi) || (gemm_shape(c.d, chi) && j->hermitian)));
+                    (j->generic(kGenExt) || !(chi == 1 || ext_fast_shape<R>(c.d, chi) || (gemm_shape(c.d, chi) && j->hermitian)));
   if (sizeof(R) == sizeof(float) && need_generic) {
     const long cnt = (long)j->M * chi * chi;
     j->conv_msgs.ensure((size_t)cnt * sizeof(cplx<double>), j->dev_bytes, j->stream);

@@ -401,7 +401,10 @@ template <typename R>
 inline bool fast_local_mfma(ClassView cv, int chi_in, int chi_out, const cplx<R>* Tin, cplx<R>* Tout,
                             const cplx<double>* canon, int rows, int cols, double zz_time, int flags, double z_time,
                             double x_time, const double* lmbd, int lstride, cplx<R>* msgs_init, hipStream_t s) {
-  if (chi_in != chi_out || flags != (kAbsorb | kGates | kGauge) || cv.zz == nullptr) return false;
+  if (chi_in > chi_out || flags != (kAbsorb | kGates | kGauge) || cv.zz == nullptr) return false;
+  if (chi_in < chi_out)
+    return launch_small_local<R>(cv, chi_out, Tin, Tout, canon, rows, cols, z_time, x_time, lmbd, lstride, msgs_init,
+                                 s);
   if (launch_local_big<R>(cv, chi_in, Tin, Tout, canon, rows, cols, z_time, x_time, lmbd, lstride, msgs_init, s))
     return true;
   if (chi_in != 8 || cv.d != 3 || cv.n == 0)

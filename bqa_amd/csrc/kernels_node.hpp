@@ -267,6 +267,32 @@ __global__ __launch_bounds__(kNT) void k_node_contract(
 
 enum LocalFlags { kAbsorb = 1, kGates = 2, kGauge = 4 };
 
+// Extended messages at bond dimension 1 (the first step): a thread per node and bond; the Grams are the tensor's
+// squared magnitudes times the other bonds' scalar messages.  The generic kernel, a block per node, took 1.9 ms for
+// 100,000 degree-3 nodes.
+template <typename R>
+__global__ __launch_bounds__(256) void k_ext_chi1(ClassView cv, const cplx<R>* __restrict__ T, const cplx<R>* __restrict__ msgs,
+                                                  cplx<double>* __restrict__ ext) {
+  const int n = cv.n, d = cv.d;
+  const long total = (long)n * d;
+  for (long x = blockIdx.x * 256L + threadIdx.x; x < total; x += gridDim.x * 256L) {
+    const int k = (int)(x / n), i = (int)(x % n);
+    cplx<double> m = mk(1.0, 0.0);
+    for (int j = 0; j < d; ++j)
+      if (j != k) m = m * cast<double>(msgs[cv.in_pos[(long)j * n + i]]);
+    const double t0 = abs2(cast<double>(T[2L * i])), t1 = abs2(cast<double>(T[2L * i + 1]));
+    const cplx<double>* zg = cv.zz + 2 * (size_t)cv.lmbd_pos[(long)k * n + i];
+    const cplx<double> g0 = zg[0], g1 = zg[1];
+    const cplx<double> inv = cinv(scale(m, (t0 + t1) * (abs2(g0) + abs2(g1))));
+    const cplx<double> plus = scale(m, t0 + t1) * inv, minus = scale(m, t0 - t1) * inv;
+    cplx<double>* out = ext + (size_t)cv.out_pos[(long)k * n + i] * 4;
+    out[0] = conj(g0) * g0 * plus;
+    out[1] = conj(g0) * g1 * minus;
+    out[2] = conj(g1) * g0 * minus;
+    out[3] = conj(g1) * g1 * plus;
+  }
+}
+
 // Absorb canonicalisers (with the ZZ split), then the Z and X layers, then the
 // symmetric gauge with per-node L2 normalisation and message re-initialisation.
 // Tin: (n, 2, chi_in^d) -> Tout: (n, 2, chi_out^d).  Dynamic LDS:

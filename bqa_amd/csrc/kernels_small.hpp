@@ -508,7 +508,7 @@ __device__ __forceinline__ cplx<C> sgram_g(const cplx<C>* T, const cplx<C>* Y, i
 // Output message K of this group's node from the Gram sum over every bond but K of conj(A) B.
 template <int D, int CHI, int K, int NPW, typename R, typename C>
 __device__ __forceinline__ void sout_g(NpwSmem<D, CHI, NPW, C>& sm, const cplx<C>* A, const cplx<C>* Y,
-                                       const ClassView& cv, int i, bool valid, int gi, int gl,
+                                       const int (&pos)[D], bool valid, int gi, int gl,
                                        const cplx<R> (&old)[D], cplx<R>* mout, double& dnum, double& dden) {
   constexpr int GL = 64 / NPW, Q = CHI * CHI;
   const cplx<C> g = sgram_g<D, CHI, K, GL, C>(A, Y, gl);
@@ -525,7 +525,7 @@ __device__ __forceinline__ void sout_g(NpwSmem<D, CHI, NPW, C>& sm, const cplx<C
     const cplx<double> vd = cast<double>(v), od = cast<double>(old[K]);
     dnum = fmax(dnum, abs2(vd - od));
     dden = fmax(dden, abs2(vd + od));
-    mout[(long)cv.out_pos[K * cv.n + i] * Q + gl] = v;
+    mout[(size_t)pos[K] * Q + gl] = v;
   }
   small_sync();
 }
@@ -547,32 +547,66 @@ __device__ __forceinline__ void npw_run(NpwSmem<D, CHI, NPW, R>& sm, const Class
   const int n = cv.n;
   const int l = threadIdx.x & 63, gi = l / GL, gl = l % GL;
   double dnum = 0.0, dden = 0.0;
-  for (long i0 = start * NPW; i0 < n; i0 += (long)gridDim.x * NPW) {
-    const int i = (int)i0 + gi;
-    const bool valid = i < n;
-    const int ic = valid ? i : n - 1;  // a group past the end repeats the last node and stores nothing
-    const cplx<R>* Tg = T + (size_t)ic * M::S;
+  // A node's tensor, messages and old messages are loaded into registers while the group before computes, and its
+  // positions one group earlier, so that no load waits for another (100,000 nodes at chi = 4, FP64: 159 us a sweep
+  // without).  A group past the end repeats the last node and stores nothing.
+  constexpr int TPL = (M::S + GL - 1) / GL;
+  const long step = (long)gridDim.x * NPW;
+  cplx<R> nt[TPL], nm[D], nold[D];
+  int pin[D], pout[D], npos[D];
+  auto node = [&](long i0) { return (int)(i0 + gi < n ? i0 + gi : n - 1); };
+  auto positions = [&](long i0) {
+    const int i = node(i0);
 #pragma unroll
-    for (int q = 0; q < (M::S + GL - 1) / GL; ++q) {
-      const int x = gl + GL * q;
-      if (M::S % GL == 0 || x < M::S) sm.T[gi][x] = cast<C>(Tg[x]);
+    for (int k = 0; k < D; ++k) {
+      pin[k] = cv.in_pos[k * n + i];
+      pout[k] = cv.out_pos[k * n + i];
     }
+  };
+  auto fetch = [&](long i0) {
+    const cplx<R>* Tg = T + (size_t)node(i0) * M::S;
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const cplx<R>* mj = min + (size_t)cv.in_pos[j * n + ic] * M::Q;
-      if (gl < M::Q) sm.m[gi][j][gl] = cast<C>(mj[gl]);
+    for (int q = 0; q < TPL; ++q)
+      if (M::S % GL == 0 || gl + GL * q < M::S) nt[q] = Tg[gl + GL * q];
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      npos[k] = pout[k];
+      if (gl < M::Q) {
+        nm[k] = min[(size_t)pin[k] * M::Q + gl];
+        nold[k] = min[(size_t)pout[k] * M::Q + gl];
+      }
     }
+  };
+  if (start * NPW < n) {
+    positions(start * NPW);
+    fetch(start * NPW);
+    if (start * NPW + step < n) positions(start * NPW + step);
+  }
+  for (long i0 = start * NPW; i0 < n; i0 += step) {
+    const bool valid = i0 + gi < n;
     cplx<R> old[D];
+    int pos[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) old[k] = gl < M::Q ? min[(size_t)cv.out_pos[k * n + ic] * M::Q + gl] : mk<R>(0, 0);
+    for (int q = 0; q < TPL; ++q)
+      if (M::S % GL == 0 || gl + GL * q < M::S) sm.T[gi][gl + GL * q] = cast<C>(nt[q]);
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      if (gl < M::Q) sm.m[gi][k][gl] = cast<C>(nm[k]);
+      old[k] = nold[k];
+      pos[k] = npos[k];
+    }
+    if (i0 + step < n) {
+      fetch(i0 + step);
+      if (i0 + 2 * step < n) positions(i0 + 2 * step);
+    }
     small_sync();
     if constexpr (D == 2) {
       smp_g<D, CHI, 1, GL, C>(sm.T[gi], sm.X[gi], sm.m[gi][1], gl);  // Y0 = T x1 m1
       small_sync();
-      sout_g<D, CHI, 0, NPW, R, C>(sm, sm.T[gi], sm.X[gi], cv, ic, valid, gi, gl, old, mout, dnum, dden);
+      sout_g<D, CHI, 0, NPW, R, C>(sm, sm.T[gi], sm.X[gi], pos, valid, gi, gl, old, mout, dnum, dden);
       smp_g<D, CHI, 0, GL, C>(sm.T[gi], sm.X[gi], sm.m[gi][0], gl);  // Y1 = T x0 m0
       small_sync();
-      sout_g<D, CHI, 1, NPW, R, C>(sm, sm.T[gi], sm.X[gi], cv, ic, valid, gi, gl, old, mout, dnum, dden);
+      sout_g<D, CHI, 1, NPW, R, C>(sm, sm.T[gi], sm.X[gi], pos, valid, gi, gl, old, mout, dnum, dden);
     } else {
       // The incoming messages are Hermitian, so one moves to the bra side as a product of the
       // conjugated factor: with P_j = T x_j m_j, out_0 = sum conj(P_2) P_1, out_1 = sum conj(P_2) P_0,
@@ -581,11 +615,11 @@ __device__ __forceinline__ void npw_run(NpwSmem<D, CHI, NPW, R>& sm, const Class
       smp_g<D, CHI, 0, GL, C>(sm.T[gi], sm.X[gi], sm.m[gi][0], gl);  // P_0 = T x0 m0
       smp_g<D, CHI, 1, GL, C>(sm.T[gi], sm.Y[gi], sm.m[gi][1], gl);  // P_1 = T x1 m1
       small_sync();
-      sout_g<D, CHI, 2, NPW, R, C>(sm, sm.Y[gi], sm.X[gi], cv, ic, valid, gi, gl, old, mout, dnum, dden);
+      sout_g<D, CHI, 2, NPW, R, C>(sm, sm.Y[gi], sm.X[gi], pos, valid, gi, gl, old, mout, dnum, dden);
       smp_last_inplace<D, CHI, GL, C>(sm.T[gi], sm.m[gi][2], gl);  // T <- P_2 = T x2 m2
       small_sync();
-      sout_g<D, CHI, 0, NPW, R, C>(sm, sm.T[gi], sm.Y[gi], cv, ic, valid, gi, gl, old, mout, dnum, dden);
-      sout_g<D, CHI, 1, NPW, R, C>(sm, sm.T[gi], sm.X[gi], cv, ic, valid, gi, gl, old, mout, dnum, dden);
+      sout_g<D, CHI, 0, NPW, R, C>(sm, sm.T[gi], sm.Y[gi], pos, valid, gi, gl, old, mout, dnum, dden);
+      sout_g<D, CHI, 1, NPW, R, C>(sm, sm.T[gi], sm.X[gi], pos, valid, gi, gl, old, mout, dnum, dden);
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -723,12 +757,13 @@ inline bool launch_small_npw(ClassView cv, int chi, const cplx<R>* T, cplx<R>* m
   return false;
 }
 
-// Fused absorb + Z/X gates + symmetric gauge + message re-initialisation at
-// a fixed bond dimension (chi_in = chi_out = CHI), one wave per node, FP64
+// Fused absorb + Z/X gates + symmetric gauge + message re-initialisation at a bond dimension that stays or grows
+// (chi_in <= chi_out = CHI; a smaller tensor is padded with zeros in LDS: 100,000 degree-3 nodes from chi 1 to 2
+// and 2 to 4 took 0.8 and 0.9 ms in k_node_local's blocks), one wave per node, FP64
 // arithmetic on R storage; same operation as k_node_local with all three
 // flags (backends.py:416-432, state.py:142-156, 219-227).  Absorbing the
 // canonicaliser C_k of bond k with the ZZ split is a mode product with the
-// p-dependent matrix W_k^(p)[c][n] = g0 C_k[c][n] + (1 - 2p) g1 C_k[CHI + c][n]
+// p-dependent matrix W_k^(p)[c][n] = g0 C_k[c][n] + (1 - 2p) g1 C_k[chi_in + c][n]
 // (gates from cv.zz), built once per node in LDS.
 template <int D, int CHI>
 struct SmallLocalSmem {
@@ -768,19 +803,44 @@ __global__ __launch_bounds__(64) void k_small_local(ClassView cv, const cplx<R>*
   __shared__ __align__(16) SmallLocalSmem<D, CHI> sm;
   const int n = cv.n;
   const int l = threadIdx.x & 63;
+  const int cin = canon_rows >> 1;   // chi_in
   const double cx = cos(x_time), sx = sin(x_time);
   for (int i = blockIdx.x; i < n; i += gridDim.x) {
-    const cplx<R>* Tg = Tin + (size_t)i * M::S;
+    if (cin == CHI) {
+      const cplx<R>* Tg = Tin + (size_t)i * M::S;
 #pragma unroll 4
-    for (int q = 0; q < (M::S + 63) / 64; ++q) {
-      const int x = l + 64 * q;
-      if (M::S % 64 == 0 || x < M::S) sm.X[x] = cast<double>(Tg[x]);
+      for (int q = 0; q < (M::S + 63) / 64; ++q) {
+        const int x = l + 64 * q;
+        if (M::S % 64 == 0 || x < M::S) sm.X[x] = cast<double>(Tg[x]);
+      }
+    } else {
+      int sin = 2;
+#pragma unroll
+      for (int k = 0; k < D; ++k) sin *= cin;
+      const cplx<R>* Tg = Tin + (size_t)i * sin;
+      for (int x = l; x < M::S; x += 64) {
+        int rem = x, at = 0, place = 1;
+        bool in = true;
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          const int b = rem % CHI;
+          rem /= CHI;
+          in = in && b < cin;
+          at += b * place;
+          place *= cin;
+        }
+        sm.X[x] = in ? cast<double>(Tg[at + rem * place]) : mk(0.0, 0.0);
+      }
     }
     for (int q = l; q < D * M::Q; q += 64) {
       const int k = q / M::Q, o = q % M::Q, c = o / CHI, nn = o % CHI;
       const cplx<double>* C = canon + (size_t)cv.in_pos[k * n + i] * canon_rows * canon_cols;
       const cplx<double>* zg = cv.zz + 2 * (size_t)cv.lmbd_pos[k * n + i];
-      const cplx<double> u = zg[0] * C[c * canon_cols + nn], v = zg[1] * C[(CHI + c) * canon_cols + nn];
+      cplx<double> u = mk(0.0, 0.0), v = mk(0.0, 0.0);
+      if (c < cin) {
+        u = zg[0] * C[c * canon_cols + nn];
+        v = zg[1] * C[(cin + c) * canon_cols + nn];
+      }
       sm.W[k][0][o] = u + v;
       sm.W[k][1][o] = u - v;
     }
@@ -877,7 +937,7 @@ inline bool launch_small_local_d(int chi, ClassView cv, const cplx<R>* Tin, cplx
   return false;
 }
 
-// The fused simple-update tail at a fixed bond dimension; false when the shape
+// The fused simple-update tail to bond dimension chi from rows / 2 <= chi; false when the shape
 // is not served (the caller runs k_node_local).
 template <typename R>
 inline bool launch_small_local(ClassView cv, int chi, const cplx<R>* Tin, cplx<R>* Tout, const cplx<double>* canon,

@@ -166,3 +166,28 @@ def test_density_matches_oracle(d, chi, n, precision):
     tol = u * (8 * d * chi + 64)
     assert np.abs(rho - want).max() < tol
     assert np.abs(bloch[:, 2] - (want[:, 0, 0] - want[:, 1, 1]).real).max() < 2 * tol
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("d,chi,chi_max,n", [(2, 1, 2, 9), (2, 3, 4, 9), (2, 6, 8, 30), (3, 1, 2, 10), (3, 2, 3, 10), (3, 4, 7, 8),
+                                             (3, 5, 8, 20), (4, 1, 2, 14), (4, 2, 4, 8), (5, 1, 2, 8)])
+def test_growing_local_step_matches_generic(d, chi, chi_max, n, precision, monkeypatch):
+    """The local step from a smaller bond dimension (the tensor padded in LDS), from the bond dimension-1 extended
+    messages on."""
+    test_local_step_matches_generic(d, chi, chi_max, n, precision, monkeypatch)
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("d,n", [(2, 5), (3, 10), (4, 300), (5, 8)])
+def test_extended_messages_of_bond_dimension_one(d, n, precision, monkeypatch):
+    ctx, t, m = _state(d, n, 1, precision)
+    lam = []
+    for mask in ("", "e"):
+        monkeypatch.setenv("BQA_GENERIC_KERNELS", mask)
+        job = _job(ctx, t, m, precision)
+        try:
+            job.simple_update(0.2, 1e-6)
+            lam.append(job.get_lambdas().real)
+        finally:
+            job.close()
+    assert np.abs(lam[0] - lam[1]).max() < 1e-13   # a handful of FP64 products of numbers of order one
