@@ -519,6 +519,18 @@ int ceil_log2(long n) {
   return k;
 }
 
+// Keeps (restore = 0) or puts back (1) the distance maxima that a sweep's launches add to, so that every timed launch
+// updates them as a sweep's own does (a repeat would find them in place, and its blocks nothing to add).  Each protocol
+// keeps them in the other's place.
+__global__ void k_bp_tune_slot(BpStatus* st, int sweep, int restore) {
+  unsigned long long* at[2] = {&st->num_bits, &st->den_bits};
+  for (int k = 0; k < 2; ++k) {
+    unsigned long long* live = sweep < 0 ? at[k] : &st->slot[sweep][k];
+    unsigned long long* kept = sweep < 0 ? &st->slot[kSweepSlots - 1][k] : at[k];
+    *(restore ? live : kept) = *(restore ? kept : live);
+  }
+}
+
 template <typename R>
 int bp_variant(bqa_job* j, ClassDev& c, const ClassView& view, bool may_tune) {
   const int chi = j->chi;
@@ -536,27 +548,34 @@ int bp_variant(bqa_job* j, ClassDev& c, const ClassView& view, bool may_tune) {
   }
   const cplx<R>* T = reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p);
   BpStatus* st = reinterpret_cast<BpStatus*>(j->status.p);
-  std::vector<hipEvent_t> ev(nv + 1, nullptr);
+  std::vector<hipEvent_t> ev(2 * nv * kTuneReps, nullptr);
   TuneEntry res;
   try {
     for (auto& e : ev) HIPX(hipEventCreate(&e));
+    hipLaunchKernelGGL(k_bp_tune_slot, dim3(1), dim3(1), 0, j->stream, st, view.sweep, 0);
+    LAUNCH_CHECK();
     fast_bp_launch<R>(view, chi, T, msg_ptr<R>(j, 0), msg_ptr<R>(j, 1), st, j->stream, 0);  // warm-up
     LAUNCH_CHECK();
-    for (int v = 0; v < nv; ++v) {
-      HIPX(hipEventRecord(ev[v], j->stream));
+    for (int v = 0; v < nv; ++v)
       for (int r = 0; r < kTuneReps; ++r) {
+        const int e = 2 * (v * kTuneReps + r);
+        hipLaunchKernelGGL(k_bp_tune_slot, dim3(1), dim3(1), 0, j->stream, st, view.sweep, 1);
+        LAUNCH_CHECK();
+        HIPX(hipEventRecord(ev[e], j->stream));
         fast_bp_launch<R>(view, chi, T, msg_ptr<R>(j, 0), msg_ptr<R>(j, 1), st, j->stream, v);
         LAUNCH_CHECK();
+        HIPX(hipEventRecord(ev[e + 1], j->stream));
       }
-    }
-    HIPX(hipEventRecord(ev[nv], j->stream));
-    HIPX(hipEventSynchronize(ev[nv]));
+    HIPX(hipEventSynchronize(ev.back()));
     res.us.resize(nv);
     res.chosen = 0;
     for (int v = 0; v < nv; ++v) {
-      float ms = 0.f;
-      HIPX(hipEventElapsedTime(&ms, ev[v], ev[v + 1]));
-      res.us[v] = 1e3 * ms / kTuneReps;
+      for (int r = 0; r < kTuneReps; ++r) {
+        const int e = 2 * (v * kTuneReps + r);
+        float ms = 0.f;
+        HIPX(hipEventElapsedTime(&ms, ev[e], ev[e + 1]));
+        res.us[v] = r == 0 ? 1e3 * ms : std::min(res.us[v], 1e3 * (double)ms);
+      }
       if (res.us[v] < res.us[res.chosen]) res.chosen = v;
     }
   } catch (...) {
