@@ -341,10 +341,11 @@ double sweep_bytes(const bqa_job* j, const ClassDev& c, int chi) {
          (double)c.n * c.d * 8.0;
 }
 
-// One block of kSweepSlots threads.
-__global__ void k_bp_reset(BpStatus* st, int cur, int max_iters, double bp_eps) {
-  st->slot[threadIdx.x][0] = 0ULL;
-  st->slot[threadIdx.x][1] = 0ULL;
+constexpr int kResetThreads = 1024;
+__global__ __launch_bounds__(kResetThreads) void k_bp_reset(BpStatus* st, int cur, int max_iters, double bp_eps) {
+  const int used = slot_at(min(max_iters, kSweepSlots) + kSlotLine - 1, 0) / kSlotLine * kSlotLine;
+  for (int k = threadIdx.x; k < used && k < kSweepSlots * kSlotParts; k += kResetThreads)
+    st->slot[k][0] = st->slot[k][1] = 0ULL;
   if (threadIdx.x != 0) return;
   st->num_bits = 0ULL;
   st->den_bits = 0ULL;
@@ -519,18 +520,6 @@ int ceil_log2(long n) {
   return k;
 }
 
-// Keeps (restore = 0) or puts back (1) the distance maxima that a sweep's launches add to, so that every timed launch
-// updates them as a sweep's own does (a repeat would find them in place, and its blocks nothing to add).  Each protocol
-// keeps them in the other's place.
-__global__ void k_bp_tune_slot(BpStatus* st, int sweep, int restore) {
-  unsigned long long* at[2] = {&st->num_bits, &st->den_bits};
-  for (int k = 0; k < 2; ++k) {
-    unsigned long long* live = sweep < 0 ? at[k] : &st->slot[sweep][k];
-    unsigned long long* kept = sweep < 0 ? &st->slot[kSweepSlots - 1][k] : at[k];
-    *(restore ? live : kept) = *(restore ? kept : live);
-  }
-}
-
 template <typename R>
 int bp_variant(bqa_job* j, ClassDev& c, const ClassView& view, bool may_tune) {
   const int chi = j->chi;
@@ -552,15 +541,11 @@ int bp_variant(bqa_job* j, ClassDev& c, const ClassView& view, bool may_tune) {
   TuneEntry res;
   try {
     for (auto& e : ev) HIPX(hipEventCreate(&e));
-    hipLaunchKernelGGL(k_bp_tune_slot, dim3(1), dim3(1), 0, j->stream, st, view.sweep, 0);
-    LAUNCH_CHECK();
     fast_bp_launch<R>(view, chi, T, msg_ptr<R>(j, 0), msg_ptr<R>(j, 1), st, j->stream, 0);  // warm-up
     LAUNCH_CHECK();
     for (int v = 0; v < nv; ++v)
       for (int r = 0; r < kTuneReps; ++r) {
         const int e = 2 * (v * kTuneReps + r);
-        hipLaunchKernelGGL(k_bp_tune_slot, dim3(1), dim3(1), 0, j->stream, st, view.sweep, 1);
-        LAUNCH_CHECK();
         HIPX(hipEventRecord(ev[e], j->stream));
         fast_bp_launch<R>(view, chi, T, msg_ptr<R>(j, 0), msg_ptr<R>(j, 1), st, j->stream, v);
         LAUNCH_CHECK();
@@ -704,15 +689,19 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants, int sweeps
 
 // Bytes of a status block with its first `sweeps` slots.
 size_t status_bytes(int sweeps) {
-  return offsetof(BpStatus, slot) + sizeof(BpStatus::slot[0]) * std::min(sweeps, kSweepSlots);
+  const int lines = (std::min(sweeps, kSweepSlots) + kSlotLine - 1) / kSlotLine;
+  static_assert(sizeof(BpHeader) <= 128 && alignof(BpStatus) == 128, "the slots follow the header's line");
+  return 128 + sizeof(BpStatus::slot[0]) * lines * kSlotParts * kSlotLine;
 }
 
 // The rules of k_bp_finish (no damping, src/bqa/state.py:113-121) applied on the host to the
 // sweep slots [ruled, launched) of a run, stopping at the first that ends it.
-void apply_slot_rules(const BpStatus* sh, BpStatus& h, int& ruled, int launched, int max_iters, double bp_eps) {
+void apply_slot_rules(const BpStatus* sh, BpHeader& h, int& ruled, int launched, int max_iters, double bp_eps) {
   for (; ruled < launched && !h.done; ++ruled) {
-    const double num = bits_to_double(sh->slot[ruled][0]);
-    const double den = bits_to_double(sh->slot[ruled][1]);
+    unsigned long long bits[2] = {0, 0};
+    for (int part = 0; part < kSlotParts; ++part)
+      for (int k = 0; k < 2; ++k) bits[k] = std::max(bits[k], sh->slot[slot_at(ruled, part)][k]);
+    const double num = bits_to_double(bits[0]), den = bits_to_double(bits[1]);
     const double dist = num / den;
     h.iters += 1;
     h.last_dist = dist;
@@ -738,7 +727,7 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
   if (max_iters <= 0)  // the reference asserts here (src/bqa/state.py:122)
     throw BqaError(BQA_ERR_NUMERIC, "max_bp_iter_number must be positive: BP ran no sweep");
   BpStatus* st = reinterpret_cast<BpStatus*>(j->status.p);
-  hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kSweepSlots), 0, j->stream, st, j->mcur, max_iters, bp_eps);
+  hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kResetThreads), 0, j->stream, st, j->mcur, max_iters, bp_eps);
   LAUNCH_CHECK();
   const long count = (long)j->M * j->chi * j->chi;
   const int damping_on = damping > 0.0 ? 1 : 0;
@@ -748,7 +737,7 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
   // Without damping, sweeps run on the sweep-slot protocol: no kernel between
   // sweeps, the rules applied here to each chunk's slots.
   const bool slots = !damping_on && active_classes > 0 && max_iters <= kSweepSlots;
-  BpStatus h{};
+  BpHeader h{};
   h.cur = j->mcur;
   h.best_dist = INFINITY;
   int launched = 0, ruled = 0;
@@ -1609,7 +1598,7 @@ void batch_bp(bqa_batch* b, int count, bqa_job* const* jobs, const int32_t* max_
   struct Run {
     bqa_job* j;
     int k;
-    BpStatus h;
+    BpHeader h;
     int ruled;
   };
   std::vector<Run> runs;
@@ -1637,7 +1626,7 @@ void batch_bp(bqa_batch* b, int count, bqa_job* const* jobs, const int32_t* max_
     Run r{j, k, BpStatus{}, 0};
     r.h.cur = j->mcur;
     r.h.best_dist = INFINITY;
-    hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kSweepSlots), 0, b->stream, reinterpret_cast<BpStatus*>(j->status.p),
+    hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kResetThreads), 0, b->stream, reinterpret_cast<BpStatus*>(j->status.p),
                        j->mcur, max_iters[k], bp_eps[k]);
     LAUNCH_CHECK();
     runs.push_back(r);

@@ -137,6 +137,14 @@ __host__ __device__ inline int ipow(int b, int e) {
 // sequential measurement then spent 2.3 ms of 12.7 ms of kernels in 1,600 finish launches.
 constexpr int kSweepSlots = 512;
 
+// Parts of a sweep's slot, taken by the blocks in turn.  Atomics at one address take about 11 ns each, so the two of
+// each of 1,024 blocks were 21 us at the end of a launch, more than the sweep of a small job; parts on lines of their
+// own take them side by side.  A line holds one part of eight sweeps, of which only one is being written.
+constexpr int kSlotParts = 16, kSlotLine = 8;
+__host__ __device__ inline int slot_at(int sweep, int part) {
+  return (sweep / kSlotLine * kSlotParts + part) * kSlotLine + sweep % kSlotLine;
+}
+
 // BP control block living in device memory.  Two protocols:
 //  - status (sweep index < 0; damping runs): the sweep kernels read `cur` and
 //    `done`, and the finish kernel (one thread) updates them after every sweep;
@@ -144,7 +152,7 @@ constexpr int kSweepSlots = 512;
 //    its own slot, each launch decides from the previous sweep's slot whether
 //    the run is over, and the host applies the rules to the slots after every
 //    chunk of sweeps, so no kernel runs between sweeps.
-struct BpStatus {
+struct BpHeader {
   unsigned long long num_bits;  // max |new - old| as double bits
   unsigned long long den_bits;  // max |new + old|
   int cur;                      // index of the current message buffer (slots: of the run's first sweep)
@@ -159,7 +167,10 @@ struct BpStatus {
   double bp_eps;
   double last_dist;
   double best_dist;
-  unsigned long long slot[kSweepSlots][2];  // slots: the two maxima of each sweep (last: a copy takes those in use)
+};
+struct BpStatus : BpHeader {
+  // slots: the parts of the two maxima of each sweep at slot_at (last, so that a copy takes those in use)
+  alignas(128) unsigned long long slot[kSweepSlots * kSlotParts][2];
 };
 
 // Buffer index a BP launch of sweep `sweep` reads, or -1 when the run is over.
@@ -175,9 +186,18 @@ __device__ inline int bp_begin(BpStatus* st, int sweep) {
     // blocks of one launch may set the marker while others read it; either
     // outcome gives the same decision, since both follow from the same slot
     if (__hip_atomic_load(&st->marker, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return -1;
-    const double num = __longlong_as_double((long long)st->slot[sweep - 1][0]);
-    const double den = __longlong_as_double((long long)st->slot[sweep - 1][1]);
-    if (num / den < st->bp_eps) {
+    // the previous sweep's maxima: a part a lane, compared as bits (a NaN's are the largest)
+    const unsigned long long* part = st->slot[slot_at(sweep - 1, threadIdx.x & (kSlotParts - 1))];
+    unsigned long long nb = part[0], db = part[1];
+#pragma unroll
+    for (int o = 1; o < kSlotParts; o <<= 1) {
+      const unsigned long long n2 = __shfl_xor(nb, o, 64), d2 = __shfl_xor(db, o, 64);
+      nb = n2 > nb ? n2 : nb;
+      db = d2 > db ? d2 : db;
+    }
+    const double num = __longlong_as_double((long long)nb), den = __longlong_as_double((long long)db);
+    // the same in every lane; as a scalar, so that what follows stays uniform
+    if (__builtin_amdgcn_readfirstlane(num / den < st->bp_eps ? 1 : 0)) {
       if (threadIdx.x == 0) __hip_atomic_store(&st->marker, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return -1;
     }
@@ -185,21 +205,13 @@ __device__ inline int bp_begin(BpStatus* st, int sweep) {
   return st->cur ^ (sweep & 1);
 }
 
-// This block's distance maxima of sweep `sweep` (one thread per block).  The atomics of a launch meet at one address
-// and take about 15 ns each, so in a launch of many blocks, whose ends spread over time, a block first looks whether
-// its maxima are above the ones so far (few are); in a small launch all blocks end together and the look only adds
-// its latency.
+// This block's distance maxima of sweep `sweep` (one thread per block).
 __device__ inline void bp_end(BpStatus* st, int sweep, double dnum, double dden) {
-  if (sweep >= 0) sweep += st->base;
-  unsigned long long* num = sweep < 0 ? &st->num_bits : &st->slot[sweep][0];
-  unsigned long long* den = sweep < 0 ? &st->den_bits : &st->slot[sweep][1];
-  if (gridDim.x > 512) {
-    const double n0 = __longlong_as_double((long long)__hip_atomic_load(num, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    const double d0 = __longlong_as_double((long long)__hip_atomic_load(den, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    // negated, so that a NaN on either side goes on to the atomic
-    if (!(dnum <= n0)) atomic_max_nonneg(num, dnum);
-    if (!(dden <= d0)) atomic_max_nonneg(den, dden);
-    return;
+  unsigned long long* num = &st->num_bits;
+  unsigned long long* den = &st->den_bits;
+  if (sweep >= 0) {
+    num = st->slot[slot_at(sweep + st->base, blockIdx.x & (kSlotParts - 1))];
+    den = num + 1;
   }
   atomic_max_nonneg(num, dnum);
   atomic_max_nonneg(den, dden);
