@@ -66,7 +66,7 @@ HHEX_CELLS = 64              # heavy-hex lattice of 64 x 64 cells: 10,144 qubits
 HHEX_CHI = 16
 HHEX_STEPS = 300
 HHEX_TIMED = 10
-HHEX32_TIMED = 3             # chi = 32 runs the generic kernels (seconds per step)
+HHEX32_TIMED = 3             # chi = 32: batched MFMA products, a short window
 TAG = {"single": "fp32", "double": "fp64"}
 
 
@@ -376,7 +376,8 @@ def main():
         raise RuntimeError("no BP sweep kernel was timed at the target bond dimension")
     if s["chi_timed"] != [args.chi]:
         raise RuntimeError(f"timed steps ran at bond dimensions {s['chi_timed']}, not {args.chi}")
-    kname = {"double": "k_mfma8_bp64_3p<4> (FP64 MFMA, six contractions per node)", "single": "k_mfma8<3,kModeBP,1> (FP32 MFMA)"}
+    kname = {"double": "k_bp_d3c8<double> (FP64 MFMA, six contractions per node)",
+             "single": "k_bp_d3c8<float> (FP32 MFMA, six contractions per node)"}
     roofline = roofline_of(s, head["ctx"], args.chi, args.precision,
                            f"BP sweep at chi={args.chi}, d=3: {kname[args.precision] if args.chi == 8 else 'per shape'}"
                            " (one launch per degree class per sweep)")
@@ -448,16 +449,16 @@ def main():
                           "tensors/messages on FP32 MFMA with FP64 canonicalisers, fp64 = complex128 throughout")
         extra["heavy_hex_chi16"] = hx
         if not args.no_hhex32:
-            # the same lattice at chi = 32, FP32 storage: no chi = 32 kernels, so the generic node
-            # kernels and the generic canonicaliser run it; a short timed window
+            # the same lattice at chi = 32, FP32 storage, on the batched MFMA
+            # products and the wide canonicaliser; a short timed window
             ctx = config_to_context(hhex_config(32, HHEX_STEPS, "single"))
-            log(f"[bench] heavy-hex {ctx.nodes_number} qubits chi=32 fp32 (generic kernels): {HHEX32_TIMED} steps "
+            log(f"[bench] heavy-hex {ctx.nodes_number} qubits chi=32 fp32: {HHEX32_TIMED} steps "
                 f"timed at chi=32")
             r = run_anneal(ctx, "single", args.warmup, HHEX32_TIMED, finish=False)
             h32 = summarize(r, ctx.nodes_number, HHEX32_TIMED)
             h32.pop("full_anneal")
             h32["workload"] = (f"the heavy-hex lattice above at chi=32, fp32 storage, {HHEX32_TIMED} steps timed once "
-                               "the bond dimension is 32; generic node kernels and canonicaliser")
+                               "the bond dimension is 32; batched MFMA products")
             extra["heavy_hex_chi32"] = h32
             log(f"[bench] heavy-hex chi=32 fp32: {h32['qubit_steps_per_s']:.4g} qubit*steps/s, "
                 f"{h32['ms_per_step']:.1f} ms/step")

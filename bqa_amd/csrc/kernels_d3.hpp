@@ -9,8 +9,8 @@
 // a node reads from memory is loaded while the node before computes, its positions one node earlier.
 // What bounds it: 192 MFMAs a node (0.50 ms FP64, 0.25 ms FP32 a sweep of 100,000 nodes at the matrix rate), with four
 // short phases a node between barriers; three (FP64) and five (FP32) nodes share a CU.  Measured at 100,000 nodes:
-// FP64 0.85 ms a sweep, FP32 0.52 ms; extended messages 1.19 and 1.17 ms.  The kernels that ran products and Grams
-// through LDS took 1.05 ms (six contractions), 0.67 ms (nine), 1.68 and 1.14 ms.
+// FP64 0.85 ms a sweep, FP32 0.52 ms; FP64 extended messages 1.19 ms.  The kernels that ran products and Grams
+// through LDS took 1.05 ms (six contractions), 0.67 ms (nine) and 1.68 ms.
 #pragma once
 
 #include "common.hpp"
@@ -32,7 +32,7 @@ constexpr int d3_shift(int bond) { return 3 * (2 - bond); }
 // memory loads: a scalar load in flight would hold up the next wait for LDS until it arrives.
 __device__ __forceinline__ int d3_lane_index(int x) { return x + opaque(0); }
 
-// GT: the precision of the Grams (FP64 for the extended messages of FP32 jobs).
+// GT: the precision of the Grams.
 template <typename R, typename GT>
 struct D3 {
   static constexpr int NW = 4, S = 1024, TILES = 8 / NW, UNITS = 16 / NW;
@@ -289,10 +289,11 @@ __global__ __launch_bounds__(256, kD3Waves<R>) void k_bp_d3c8_multi(const BpEntr
 
 // Extended messages (state.py:127-139, backends.py:393-404,519-526): the same products with the Grams kept per
 // physical half, each 16 x 16 message assembled with its bond's ZZ-split gates as in k_ext_d4c8.
-template <typename R>
-__global__ __launch_bounds__(256, 3) void k_ext_d3c8(ClassView cv, const cplx<R>* __restrict__ T, const cplx<R>* __restrict__ msgs,
-                                                     cplx<double>* ext_out) {
-  using N = D3<R, double>;
+// FP64 jobs only: FP32 ones keep k_mfma8_ext32, whose Grams take the tensor itself on one side (1.14 ms; 1.17 here).
+__global__ __launch_bounds__(256, 3) void k_ext_d3c8(ClassView cv, const cplx<double>* __restrict__ T,
+                                                     const cplx<double>* __restrict__ msgs, cplx<double>* ext_out) {
+  using R = double;
+  using N = D3<R, R>;
   __shared__ __align__(16) unsigned char lds[N::BYTES];
   const N s(lds);
   cplx<double>* gm = reinterpret_cast<cplx<double>*>(s.T);   // [k][p][64] of the finished Grams (6 KB)
@@ -350,9 +351,8 @@ inline void launch_bp_d3c8(ClassView cv, const cplx<R>* T, cplx<R>* mA, cplx<R>*
   hipLaunchKernelGGL((k_bp_d3c8<R>), dim3(grid), dim3(256), 0, s, cv, T, mA, mB, st);
 }
 
-template <typename R>
-inline void launch_ext_d3c8(ClassView cv, const cplx<R>* T, const cplx<R>* msgs, cplx<double>* ext, hipStream_t s) {
-  hipLaunchKernelGGL((k_ext_d3c8<R>), dim3(node_grid<k_ext_d3c8<R>, 256>(cv.n)), dim3(256), 0, s, cv, T, msgs, ext);
+inline void launch_ext_d3c8(ClassView cv, const cplx<double>* T, const cplx<double>* msgs, cplx<double>* ext, hipStream_t s) {
+  hipLaunchKernelGGL(k_ext_d3c8, dim3(node_grid<k_ext_d3c8, 256>(cv.n)), dim3(256), 0, s, cv, T, msgs, ext);
 }
 
 }  // namespace bqa

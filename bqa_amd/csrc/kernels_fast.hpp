@@ -115,13 +115,14 @@ bool fast_ext_launch(ClassView cv, int chi, const cplx<R>* T, const cplx<R>* msg
     if constexpr (sizeof(R) == sizeof(float)) {
       // FP32 job: FP32 MFMA mode products, FP64 MFMA Gram
       if (cv.d == 3)
-        launch_ext_d3c8<R>(cv, T, msgs, ext, s);
+        hipLaunchKernelGGL((k_mfma8_ext32<3, 4>), dim3(node_grid<k_mfma8_ext32<3, 4>, 256>(cv.n)), dim3(256), 0, s,
+                           cv, T, msgs, ext);
       else
         hipLaunchKernelGGL((k_mfma8_ext32<2, 1>), dim3(node_grid<k_mfma8_ext32<2, 1>, 64>(cv.n)), dim3(64), 0, s, cv,
                            T, msgs, ext);
     } else {
       if (cv.d == 3)
-        launch_ext_d3c8<R>(cv, T, msgs, ext, s);
+        launch_ext_d3c8(cv, T, msgs, ext, s);
       else
         hipLaunchKernelGGL((k_mfma8_ext64<2, 1, R>), dim3(node_grid<k_mfma8_ext64<2, 1, R>, 64>(cv.n)), dim3(64), 0,
                            s, cv, T, msgs, ext);

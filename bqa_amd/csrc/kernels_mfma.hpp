@@ -921,8 +921,9 @@ __device__ __forceinline__ void ext_out8x(const float* T, const float* Y, double
 template <int D, int W>
 __global__ __launch_bounds__(64 * W, 6) void k_mfma8_ext32(ClassView cv, const cplx<float>* __restrict__ T,
                                                         const cplx<float>* __restrict__ msgs, cplx<double>* ext_out) {
-  static_assert(D == 2, "degree 2 (degree 3: k_ext_d3c8)");
+  static_assert(D == 2 || D == 3, "degree 2 or 3");
   static_assert(W == 1 || W % 2 == 0, "single-p Gram slices per wave");
+  static_assert(D == 2 || W * 256 <= Mf8<D>::S, "Gram partials fit in a dead work buffer");
   __shared__ __align__(16) Mf8ExtSmem<D, W> sm;
   const int n = cv.n;
   constexpr int S = Mf8<D>::S;
@@ -940,6 +941,20 @@ __global__ __launch_bounds__(64 * W, 6) void k_mfma8_ext32(ClassView cv, const c
       mp8<D, W, 0>(sm.T, sm.W2, bm[0], zl);          // Y1 = T x0 m0
       __syncthreads();
       ext_out8x<D, W, 1>(sm.T, sm.W2, sm.G, cv, i, ext_out, zl);
+    } else {
+      mp8<D, W, 2>(sm.T, sm.W1, bm[2], zl);          // W1 = T x2 m2
+      __syncthreads();
+      mp8<D, W, 1>(sm.W1, sm.W2, bm[1], zl);         // Y0 = W1 x1 m1
+      __syncthreads();
+      ext_out8x<D, W, 0>(sm.T, sm.W2, reinterpret_cast<double*>(sm.W2), cv, i, ext_out, zl);
+      mp8<D, W, 0>(sm.W1, sm.W2, bm[0], zl);         // Y1 = W1 x0 m0
+      __syncthreads();
+      ext_out8x<D, W, 1>(sm.T, sm.W2, reinterpret_cast<double*>(sm.W2), cv, i, ext_out, zl);
+      mp8<D, W, 0>(sm.T, sm.W1, bm[0], zl);          // W1 = T x0 m0
+      __syncthreads();
+      mp8<D, W, 1>(sm.W1, sm.W1, bm[1], zl);         // Y2 = W1 x1 m1 (in place)
+      __syncthreads();
+      ext_out8x<D, W, 2>(sm.T, sm.W1, reinterpret_cast<double*>(sm.W1), cv, i, ext_out, zl);
     }
   }
 }
