@@ -24,6 +24,7 @@
 #include "../../include/bqa_hip.h"
 #include "canon_wide.hpp"
 #include "common.hpp"
+#include "graph_cache.hpp"
 #include "kernels_canon.hpp"
 #include "kernels_canon_h.hpp"
 #include "kernels_fast.hpp"
@@ -203,17 +204,14 @@ struct bqa_job {
   // variant k wherever the shape has one (both read at job creation).
   bool autotune = true;
   int bp_variant_force = -1;
-  // Graph-captured BP chunks (BQA_GRAPHS=0 turns them off): kGraphSweeps sweeps of every class
-  // plus the sweep-index advance, captured once per key (bond dimension, buffers, variants)
-  // and replayed once the job has run BP kGraphWarmRuns times in a row at its bond dimension.
-  struct BpGraph {
-    std::vector<intptr_t> key;
-    hipGraphExec_t exec = nullptr;
-  };
+  // Graph-captured BP chunks (BQA_GRAPHS=0 turns them off): kGraphSweeps or kGraphLongSweeps sweeps of
+  // every class plus the sweep-index advance, captured once per key (bond dimension, sweeps, buffers,
+  // variants) and replayed once the job has run BP kGraphWarmRuns times in a row at its bond dimension.
+  // Eight graphs: two lengths times two tensor buffers at each of two bond dimensions.
   bool use_graphs = true;
   int graph_chi = 0;   // bond dimension of the last completed BP runs
   int graph_runs = 0;  // consecutive completed BP runs at graph_chi
-  std::vector<BpGraph> graphs;
+  GraphCache<hipGraphExec_t, 8> graphs;
   int64_t graph_captures = 0, graph_launches = 0, graph_failures = 0;
 
   bool single() const { return prec == BQA_PREC_SINGLE; }
@@ -618,7 +616,6 @@ void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first) {
 // Sweeps of a replay: four, or sixteen where the chunk has that many left (a replay costs its launch, several times a
 // small job's sweep, so a long run takes few).
 constexpr int kGraphSweeps = 4, kGraphLongSweeps = 16;
-constexpr size_t kMaxGraphs = 8;
 // Eager BP runs at one bond dimension before its chunks are captured: a capture and
 // instantiation cost about as much as the launches of tens of sweeps, so graphs
 // serve the steady state, not the steps of the bond-dimension ramp.
@@ -637,8 +634,7 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants, int sweeps
     key.push_back(c.n);
     key.push_back(variants[ci]);
   }
-  for (const auto& g : j->graphs)
-    if (g.key == key) return g.exec;
+  if (const hipGraphExec_t* kept = j->graphs.find(key)) return *kept;
   BpStatus* st = reinterpret_cast<BpStatus*>(j->status.p);
   hipGraph_t graph = nullptr;
   std::unique_lock<std::mutex> lock(g_capture_mu);
@@ -678,11 +674,7 @@ hipGraphExec_t bp_graph(bqa_job* j, const std::vector<int>& variants, int sweeps
   const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   HIPX(e);
-  if (j->graphs.size() >= kMaxGraphs) {
-    (void)hipGraphExecDestroy(j->graphs.front().exec);
-    j->graphs.erase(j->graphs.begin());
-  }
-  j->graphs.push_back({std::move(key), exec});
+  j->graphs.add(std::move(key), exec, [](hipGraphExec_t old) { (void)hipGraphExecDestroy(old); });
   ++j->graph_captures;
   return exec;
 }
@@ -748,24 +740,26 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
                j->graph_runs >= kGraphWarmRuns;
   for (auto& cl : j->cls)
     if (cl.d > 0 && cl.n > 0 && !bp_fast_shape<R>(cl.d, j->chi)) graph = false;
-  std::vector<int> variants;
+  // The run's graphs, taken once before its first replay, so that it is replays or eager launches as a whole: eager
+  // sweeps count from the run's first one, replays from the one before.  The long one only where the first chunk has
+  // room for it (later chunks are short), and the short one in its place if its capture fails.
+  hipGraphExec_t exec = nullptr, exec_long = nullptr;
   if (graph) {
+    std::vector<int> variants;
     for (auto& cl : j->cls) {
       ClassView view = cl.view();
       variants.push_back(cl.d > 0 && cl.n > 0 ? bp_variant<R>(j, cl, view, false) : 0);
     }
+    exec = bp_graph<R>(j, variants, kGraphSweeps);
+    if (exec && chunk >= kGraphLongSweeps) exec_long = bp_graph<R>(j, variants, kGraphLongSweeps);
   }
   while (launched < max_iters) {
     int c = std::min(chunk, max_iters - launched);
-    // both graphs before the first replay: eager sweeps count from the run's first one, replays from the last
-    const hipGraphExec_t exec = graph ? bp_graph<R>(j, variants, kGraphSweeps) : nullptr;
-    const hipGraphExec_t exec_long = exec && c >= kGraphLongSweeps ? bp_graph<R>(j, variants, kGraphLongSweeps) : exec;
-    if (graph && !exec_long) graph = false;
-    if (graph) {
+    if (exec) {
       // whole replays: their sweeps beyond max_iters, or after convergence, exit at once
       int replayed = 0;
       while (replayed < c) {
-        const bool lengthy = c - replayed >= kGraphLongSweeps;
+        const bool lengthy = exec_long && c - replayed >= kGraphLongSweeps;
         HIPX(hipGraphLaunch(lengthy ? exec_long : exec, j->stream));
         ++j->graph_launches;
         replayed += lengthy ? kGraphLongSweeps : kGraphSweeps;
@@ -1927,7 +1921,7 @@ int bqa_job_destroy(bqa_job* j) {
   return guarded([&] {
     (void)hipSetDevice(j->device);
     if (j->stream) (void)hipStreamSynchronize(j->stream);
-    for (auto& g : j->graphs) (void)hipGraphExecDestroy(g.exec);
+    j->graphs.clear([](hipGraphExec_t old) { (void)hipGraphExecDestroy(old); });
     for (auto& c : j->cls) {
       c.layout.release(j->dev_bytes);
       c.T[0].release(j->dev_bytes);

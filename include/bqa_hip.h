@@ -253,8 +253,9 @@ int bqa_tuning_reset(void);
 /* Graph-captured BP chunks (no counterpart in the reference, whose sweeps are
  * host-driven library calls, state.py:105-121).  Once a job has run BP eight
  * times in a row at one bond dimension, its sweeps run as replays of a HIP graph
- * holding four sweeps of every degree class; a graph is captured once per bond dimension, buffer set and
- * launch variants (thread-local capture mode) and replayed until the run
+ * holding four sweeps of every degree class, or of one holding sixteen where the run is
+ * expected to need that many more; a graph is captured once per bond dimension, length, buffer set and
+ * launch variants (thread-local capture mode; a job keeps the eight last used) and replayed until the run
  * converges.  Kernel timing (bqa_timing_enable) and BQA_GRAPHS=0 keep the
  * launches eager, and so does a capture that a runtime call from outside this
  * library invalidates (counted as a failure; the job continues eagerly).  Counts
