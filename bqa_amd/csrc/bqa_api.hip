@@ -182,7 +182,9 @@ struct bqa_job {
   DevBuf msgs[2], lmbd, ext, canon, lmax, status, rho, bloch, edges, epart, gws, cws, conv, conv_msgs, zz, plist;
   std::vector<int32_t> node_cls, node_pos;  // qubit id -> (degree class, position in the class)
   bool zz_valid = false;  // zz holds the gates of the current simple update
-  bool hermitian = true;  // the messages are Hermitian; false after an upload of others, until BP replaces them
+  // Whether the messages are Hermitian, as BP sweeps, the gauge and the initial state write them; an upload is looked
+  // at (k_check_msgs).  Others run the kernels that apply them to the ket only, until a sweep has replaced them.
+  bool hermitian = true;
   BpStatus* st_host = nullptr;
   double* lmax_host = nullptr;
   hipStream_t stream = nullptr;
@@ -573,23 +575,25 @@ int bp_variant(bqa_job* j, ClassDev& c, const ClassView& view, bool may_tune) {
 }
 
 // One class's launch of a BP sweep; sweep >= 0 selects the sweep-slot protocol.
-// `first` marks the run's first sweep, where the autotuner may time the shape.
+// `first` marks the run's first sweep, where the autotuner may time the shape; `any` a sweep whose messages need not
+// be Hermitian.
 template <typename R>
-void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first) {
+void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first, bool any = false) {
   const int chi = j->chi;
   if (c.d == 0 || c.n == 0) return;
   ClassView view = c.view();
   view.sweep = sweep;
-  const int variant = j->generic(kGenBP) ? 0 : bp_variant<R>(j, c, view, first);
+  const bool fast = !j->generic(kGenBP) && (!any || bp_ket_shape<R>(c.d, chi));
+  const int variant = !fast || any ? 0 : bp_variant<R>(j, c, view, first);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (j->timing) {
     e0 = take_event(j);
     e1 = take_event(j);
     HIPX(hipEventRecord(e0, j->stream));
   }
-  if (j->generic(kGenBP) || !fast_bp_launch<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0),
+  if (!fast || !fast_bp_launch<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0),
                          msg_ptr<R>(j, 1), reinterpret_cast<BpStatus*>(j->status.p), j->stream, variant)) {
-    if (!j->generic(kGenBP) && gemm_shape(c.d, chi) && j->hermitian) {
+    if (!j->generic(kGenBP) && gemm_shape(c.d, chi) && (!any || c.d == 2)) {   // degree 2: its message on the ket
       const int chunk = plan_gemm(j, c, chi, sizeof(cplx<R>));
       gemm_bp<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0), msg_ptr<R>(j, 1),
                  reinterpret_cast<BpStatus*>(j->status.p), j->gws.p, chunk, j->stream);
@@ -734,9 +738,10 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
   h.best_dist = INFINITY;
   int launched = 0, ruled = 0;
   int chunk = std::max(1, std::min(j->pred_sweeps, max_iters));
-  // Graph replays once this bond dimension has had an eager run (its variants chosen and the
-  // kernels' launch shapes computed), with kernel timing off and a specialised kernel per class.
-  bool graph = slots && j->use_graphs && !j->timing && !j->generic(kGenBP) && j->graph_chi == j->chi &&
+  // Graph replays once this bond dimension has had eager runs (its variants chosen and the kernels' launch shapes
+  // computed), with kernel timing off, a specialised kernel per class and Hermitian messages.
+  const bool any = !j->hermitian;
+  bool graph = slots && !any && j->use_graphs && !j->timing && !j->generic(kGenBP) && j->graph_chi == j->chi &&
                j->graph_runs >= kGraphWarmRuns;
   for (auto& cl : j->cls)
     if (cl.d > 0 && cl.n > 0 && !bp_fast_shape<R>(cl.d, j->chi)) graph = false;
@@ -767,7 +772,9 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
       c = replayed;
     } else {
       for (int s = 0; s < c; ++s) {
-        for (auto& cl : j->cls) launch_bp_class<R>(j, cl, slots ? launched + s : -1, launched + s == 0);
+        // without damping only the first sweep reads the run's own messages; damping mixes them into all
+        const bool first = launched + s == 0;
+        for (auto& cl : j->cls) launch_bp_class<R>(j, cl, slots ? launched + s : -1, first, any && (first || damping_on));
         if (slots) continue;
         hipLaunchKernelGGL(k_bp_finish, dim3(1), dim3(1), 0, j->stream, st, damping_on);
         LAUNCH_CHECK();
@@ -801,6 +808,8 @@ void run_bp_impl(bqa_job* j, int max_iters, double bp_eps, double damping, int* 
     flush_timing(j);
   }
   j->mcur = h.cur;
+  // the kept messages are a sweep's, unless the run converged on its first sweep or on a damped mixture
+  if (any && (!h.converged || (!damping_on && h.iters > 1))) j->hermitian = true;
   if (slots) {
     j->graph_runs = j->graph_chi == j->chi ? j->graph_runs + 1 : 1;
     j->graph_chi = j->chi;
@@ -869,7 +878,8 @@ void ext_class(bqa_job* j, ClassDev& c, double ztime, const cplx<double>* msgs64
   cplx<double>* ext = reinterpret_cast<cplx<double>*>(j->ext.p);
   ClassView v = c.view();
   v.zz = reinterpret_cast<const cplx<double>*>(j->zz.p);
-  if (!j->generic(kGenExt) && fast_ext_launch<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->stream)) {
+  if (!j->generic(kGenExt) && (j->hermitian || ext_ket_shape<R>(c.d, chi)) &&
+      fast_ext_launch<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->stream)) {
     LAUNCH_CHECK();
     return;
   }
@@ -880,7 +890,7 @@ void ext_class(bqa_job* j, ClassDev& c, double ztime, const cplx<double>* msgs64
     LAUNCH_CHECK();
     return;
   }
-  if (!j->generic(kGenExt) && gemm_shape(c.d, chi) && j->hermitian) {
+  if (!j->generic(kGenExt) && gemm_shape(c.d, chi) && (j->hermitian || c.d == 2)) {
     const int chunk = plan_gemm(j, c, chi, sizeof(cplx<double>));
     gemm_ext<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->gws.p, chunk, j->stream);
     LAUNCH_CHECK();
@@ -927,7 +937,9 @@ void ext_and_canon(bqa_job* j, double ztime, double pinv_eps, bool sync = true, 
   bool need_generic = false;
   for (auto& c : j->cls)
     need_generic |= c.d != 0 && c.n > 0 &&
-                    (j->generic(kGenExt) || !(chi == 1 || ext_fast_shape<R>(c.d, chi) || (gemm_shape(c.d, chi) && j->hermitian)));
+                    (j->generic(kGenExt) ||
+                     !(chi == 1 || (j->hermitian ? ext_fast_shape<R>(c.d, chi) || gemm_shape(c.d, chi)
+                                                 : ext_ket_shape<R>(c.d, chi) || (c.d == 2 && gemm_shape(c.d, chi)))));
   if (sizeof(R) == sizeof(float) && need_generic) {
     const long cnt = (long)j->M * chi * chi;
     j->conv_msgs.ensure((size_t)cnt * sizeof(cplx<double>), j->dev_bytes, j->stream);
@@ -1316,19 +1328,46 @@ void upload(bqa_job* j, void* dev, size_t count, const double* in) {
   HIPX(hipStreamSynchronize(j->stream));
 }
 
-// Whether `count` chi x chi complex matrices are Hermitian to 1e-10 of their largest element.
-bool hermitian(const double* m, long count, int chi) {
+// Of `count` chi x chi messages: out[0] their largest component, out[1] the largest deviation from a Hermitian one.
+template <typename R>
+__global__ __launch_bounds__(64) void k_check_msgs(const cplx<R>* __restrict__ msgs, long count, int chi,
+                                                   unsigned long long* out) {
+  const int l = threadIdx.x, cc = chi * chi;
   double most = 0.0, off = 0.0;
-  for (long q = 0; q < count; ++q, m += 2 * (size_t)chi * chi)
-    for (int a = 0; a < chi; ++a)
-      for (int b = 0; b <= a; ++b) {
-        const double *x = m + 2 * (a * chi + b), *y = m + 2 * (b * chi + a);
-        most = std::max({most, std::abs(x[0]), std::abs(x[1]), std::abs(y[0]), std::abs(y[1])});
-        const double diff = std::max(std::abs(x[0] - y[0]), std::abs(x[1] + y[1]));
-        if (!(diff < INFINITY)) return false;
-        off = std::max(off, diff);
-      }
-  return off <= 1e-10 * most;
+  for (long q = blockIdx.x; q < count; q += gridDim.x) {
+    const cplx<R>* m = msgs + q * cc;
+    for (int x = l; x < cc; x += 64) {
+      const cplx<double> v = cast<double>(m[x]), w = cast<double>(m[x % chi * chi + x / chi]);
+      const double diff = fmax(fabs(v.x - w.x), fabs(v.y + w.y));
+      off = fabs(v.x - w.x) < INFINITY && fabs(v.y + w.y) < INFINITY ? fmax(off, diff) : INFINITY;
+      most = fmax(most, fmax(fabs(v.x), fabs(v.y)));
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    most = fmax(most, __shfl_xor(most, o, 64));
+    off = fmax(off, __shfl_xor(off, o, 64));
+  }
+  if (l == 0) {
+    atomic_max_nonneg(out, most);
+    atomic_max_nonneg(out + 1, off);
+  }
+}
+
+// Looks at uploaded messages: Hermitian to four units of the storage type's rounding of the largest component (sweeps
+// store exactly Hermitian ones).
+template <typename R>
+void check_msgs(bqa_job* j) {
+  j->hermitian = true;
+  if (j->M == 0) return;
+  unsigned long long* lm = reinterpret_cast<unsigned long long*>(j->lmax.p);
+  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, j->stream, lm, 2);
+  LAUNCH_CHECK();
+  hipLaunchKernelGGL((k_check_msgs<R>), dim3(std::min(j->M, 8192)), dim3(64), 0, j->stream, msg_ptr<R>(j, j->mcur),
+                     (long)j->M, j->chi, lm);
+  LAUNCH_CHECK();
+  HIPX(hipMemcpyAsync(j->lmax_host, lm, 2 * sizeof(double), hipMemcpyDeviceToHost, j->stream));
+  HIPX(hipStreamSynchronize(j->stream));
+  j->hermitian = j->lmax_host[1] <= 4.0 * std::numeric_limits<R>::epsilon() * j->lmax_host[0];
 }
 
 template <typename F>
@@ -2148,8 +2187,10 @@ int bqa_set_messages(bqa_job* j, int32_t chi, const double* in) {
     require(chi == j->chi, "messages must have the tensors' bond dimension");
     ensure_msgs(j, chi);
     const size_t count = (size_t)j->M * chi * chi;
-    dispatch(j, [&](auto r) { upload<decltype(r)>(j, j->msgs[j->mcur].p, count, in); });
-    j->hermitian = hermitian(in, j->M, chi);
+    dispatch(j, [&](auto r) {
+      upload<decltype(r)>(j, j->msgs[j->mcur].p, count, in);
+      check_msgs<decltype(r)>(j);
+    });
   });
 }
 

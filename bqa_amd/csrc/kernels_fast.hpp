@@ -45,7 +45,19 @@ inline bool ext_fast_shape(int d, int chi) {
   return small_shape(d, chi) || (sizeof(R) == sizeof(float) && d == 5 && small_bp_shape<R>(5, chi));
 }
 
-// Shapes whose readout has one (fast_density_launch returns true for them).
+// Of these, the shapes whose kernel (BP: variant 0) applies every message to the ket, as the reference does, and so
+// takes any message.  The other kernels move some to the bra side, which is the same for Hermitian messages only.
+template <typename R>
+inline bool bp_ket_shape(int d, int chi) {
+  return bp_fast_shape<R>(d, chi) && (d == 2 || chi == 16 || (d >= 4 && chi <= 4));
+}
+template <typename R>
+inline bool ext_ket_shape(int d, int chi) {
+  return ext_fast_shape<R>(d, chi) &&
+         (d == 2 || chi == 16 || (d >= 4 && chi <= 4) || (sizeof(R) == sizeof(float) && d == 3 && chi == 8));
+}
+
+// Shapes whose readout has one (fast_density_launch returns true for them; every message on the ket).
 inline bool density_fast_shape(int d, int chi) { return small_shape(d, chi) || (chi == 8 && (d == 2 || d == 3)); }
 
 template <typename R>
