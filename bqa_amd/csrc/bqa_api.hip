@@ -182,9 +182,11 @@ struct bqa_job {
   DevBuf msgs[2], lmbd, ext, canon, lmax, status, rho, bloch, edges, epart, gws, cws, conv, conv_msgs, zz, plist;
   std::vector<int32_t> node_cls, node_pos;  // qubit id -> (degree class, position in the class)
   bool zz_valid = false;  // zz holds the gates of the current simple update
-  // Whether the messages are Hermitian, as BP sweeps, the gauge and the initial state write them; an upload is looked
-  // at (k_check_msgs).  Others run the kernels that apply them to the ket only, until a sweep has replaced them.
-  bool hermitian = true;
+  // What is known of the messages.  BP sweeps store Hermitian ones, positive semidefinite if those they read are; the
+  // gauge and the initial state write positive diagonals; an upload is looked at (k_check_msgs).  Messages that are
+  // not Hermitian run the kernels that apply them to the ket only, until a sweep has replaced them; the canonicalisers'
+  // Cholesky needs both, and the generic one takes others.
+  bool hermitian = true, positive = true;
   BpStatus* st_host = nullptr;
   double* lmax_host = nullptr;
   hipStream_t stream = nullptr;
@@ -994,12 +996,13 @@ void canonicalise(bqa_job* j, double pinv_eps, bool sync) {
   canon_outputs(j);
   const size_t wsb = canon_ws_bytes(n2);
   const double deps = canon_deps(j);
-  if (!j->generic(kGenCanon) && canon_wide_shape(chi)) {
+  const bool generic = j->generic(kGenCanon) || !j->hermitian || !j->positive;
+  if (!generic && canon_wide_shape(chi)) {
     j->cws.ensure(canon_wide_ws_bytes(j->E, chi), j->dev_bytes, j->stream);
     canon_wide(reinterpret_cast<const cplx<double>*>(j->ext.p), j->E, chi, ccols, pinv_eps, deps,
                reinterpret_cast<zd*>(j->canon.p), reinterpret_cast<double*>(j->lmbd.p), j->cws.p, j->stream);
     LAUNCH_CHECK();
-  } else if (j->generic(kGenCanon) || !canon_reg_dispatch(j, chi, ccols, pinv_eps, deps)) {
+  } else if (generic || !canon_reg_dispatch(j, chi, ccols, pinv_eps, deps)) {
     int grid;
     size_t lds;
     unsigned char* ws = nullptr;
@@ -1040,7 +1043,7 @@ void local_update(bqa_job* j, int flags, int chi_out, double zz_time, double z_t
   const int ccols = std::min(n2, j->chimax);
   if (flags & kGauge) {
     ensure_msgs(j, chi_out);
-    j->hermitian = true;   // the gauge sets every message to diag(lambda) / sum(lambda)
+    j->hermitian = j->positive = true;   // the gauge sets every message to diag(lambda) / sum(lambda)
   }
   for (auto& c : j->cls) {
     if (c.n == 0) continue;
@@ -1266,7 +1269,7 @@ void project_impl(bqa_job* j, int count, const int32_t* ids, const int32_t* outc
 template <typename R>
 void init_state_impl(bqa_job* j) {
   j->chi = 1;
-  j->hermitian = true;
+  j->hermitian = j->positive = true;
   j->mcur = 0;
   j->lstride = 1;
   ensure_msgs(j, 1);
@@ -1328,12 +1331,16 @@ void upload(bqa_job* j, void* dev, size_t count, const double* in) {
   HIPX(hipStreamSynchronize(j->stream));
 }
 
-// Of `count` chi x chi messages: out[0] their largest component, out[1] the largest deviation from a Hermitian one.
+// Of `count` chi x chi messages, one wave each: out[0] their largest component, out[1] the largest deviation from a
+// Hermitian one, out[2] whether any is not positive (`pivots`: the L D L^H of its Hermitian part with `shift` times
+// the trace added meets a pivot that is not; the matrix in chi^2 elements of LDS).
 template <typename R>
-__global__ __launch_bounds__(64) void k_check_msgs(const cplx<R>* __restrict__ msgs, long count, int chi,
-                                                   unsigned long long* out) {
+__global__ __launch_bounds__(64) void k_check_msgs(const cplx<R>* __restrict__ msgs, long count, int chi, bool pivots,
+                                                   double shift, unsigned long long* out) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  cplx<double>* a = reinterpret_cast<cplx<double>*>(smem_raw);
   const int l = threadIdx.x, cc = chi * chi;
-  double most = 0.0, off = 0.0;
+  double most = 0.0, off = 0.0, bad = 0.0;
   for (long q = blockIdx.x; q < count; q += gridDim.x) {
     const cplx<R>* m = msgs + q * cc;
     for (int x = l; x < cc; x += 64) {
@@ -1341,7 +1348,28 @@ __global__ __launch_bounds__(64) void k_check_msgs(const cplx<R>* __restrict__ m
       const double diff = fmax(fabs(v.x - w.x), fabs(v.y + w.y));
       off = fabs(v.x - w.x) < INFINITY && fabs(v.y + w.y) < INFINITY ? fmax(off, diff) : INFINITY;
       most = fmax(most, fmax(fabs(v.x), fabs(v.y)));
+      if (pivots) a[x] = mk(0.5 * (v.x + w.x), 0.5 * (v.y - w.y));
     }
+    if (!pivots) continue;
+    __syncthreads();
+    double add = 0.0;
+    for (int k = 0; k < chi; ++k) add += a[k * chi + k].x;
+    add *= shift;
+    for (int k = 0; k < chi; ++k) {
+      const double pivot = a[k * chi + k].x + add;
+      if (!(pivot > 0.0)) {   // the same in every lane
+        bad = 1.0;
+        break;
+      }
+      const int rest = chi - 1 - k;
+      for (int x = l; x < rest * rest; x += 64) {
+        const int r = k + 1 + x / rest, c = k + 1 + x % rest;
+        const cplx<double> u = a[r * chi + k] * conj(a[c * chi + k]);
+        a[r * chi + c] = a[r * chi + c] - scale(u, 1.0 / pivot);
+      }
+      __syncthreads();
+    }
+    __syncthreads();
   }
   for (int o = 32; o > 0; o >>= 1) {
     most = fmax(most, __shfl_xor(most, o, 64));
@@ -1350,24 +1378,30 @@ __global__ __launch_bounds__(64) void k_check_msgs(const cplx<R>* __restrict__ m
   if (l == 0) {
     atomic_max_nonneg(out, most);
     atomic_max_nonneg(out + 1, off);
+    atomic_max_nonneg(out + 2, bad);
   }
 }
 
-// Looks at uploaded messages: Hermitian to four units of the storage type's rounding of the largest component (sweeps
-// store exactly Hermitian ones).
+// Looks at uploaded messages: Hermitian to four units of the storage type's rounding of the largest component (sweeps store
+// exactly Hermitian ones), positive to 64 units of each trace (sweeps sum in the storage type).
 template <typename R>
 void check_msgs(bqa_job* j) {
-  j->hermitian = true;
+  const int chi = j->chi;
+  j->hermitian = j->positive = true;
   if (j->M == 0) return;
+  const bool pivots = chi <= 32;   // above, the canonicaliser is the generic one anyway
+  const double rounding = 4.0 * std::numeric_limits<R>::epsilon();
   unsigned long long* lm = reinterpret_cast<unsigned long long*>(j->lmax.p);
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, j->stream, lm, 2);
+  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, j->stream, lm, 3);
   LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_check_msgs<R>), dim3(std::min(j->M, 8192)), dim3(64), 0, j->stream, msg_ptr<R>(j, j->mcur),
-                     (long)j->M, j->chi, lm);
+  hipLaunchKernelGGL((k_check_msgs<R>), dim3(std::min(j->M, 8192)), dim3(64),
+                     pivots ? sizeof(cplx<double>) * chi * chi : 0, j->stream, msg_ptr<R>(j, j->mcur), (long)j->M, chi,
+                     pivots, 64.0 * std::numeric_limits<R>::epsilon(), lm);
   LAUNCH_CHECK();
-  HIPX(hipMemcpyAsync(j->lmax_host, lm, 2 * sizeof(double), hipMemcpyDeviceToHost, j->stream));
+  HIPX(hipMemcpyAsync(j->lmax_host, lm, 3 * sizeof(double), hipMemcpyDeviceToHost, j->stream));
   HIPX(hipStreamSynchronize(j->stream));
-  j->hermitian = j->lmax_host[1] <= 4.0 * std::numeric_limits<R>::epsilon() * j->lmax_host[0];
+  j->hermitian = j->lmax_host[1] <= rounding * j->lmax_host[0];
+  j->positive = j->lmax_host[2] == 0.0;
 }
 
 template <typename F>
@@ -2322,7 +2356,8 @@ int bqa_batch_run_layer(bqa_batch* b, int32_t count, bqa_job* const* jobs, const
     // split-column kernel for its chi runs its own); the lambda maxima readbacks
     std::vector<char> shared(count);
     for (int k = 0; k < count; ++k)
-      shared[k] = !jobs[k]->generic(kGenCanon) && jobs[k]->E > 0 && canon_h_n(jobs[k]->chi) > 0;
+      shared[k] = !jobs[k]->generic(kGenCanon) && jobs[k]->hermitian && jobs[k]->positive && jobs[k]->E > 0 &&
+                  canon_h_n(jobs[k]->chi) > 0;
     for (int k = 0; k < count; ++k)
       dispatch(jobs[k], [&](auto r) {
         ext_and_canon<decltype(r)>(jobs[k], ztime[k], pinv_eps[k], false, !shared[k]);

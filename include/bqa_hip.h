@@ -183,8 +183,8 @@ int bqa_bond_dim(const bqa_job* job, int32_t* chi);
 
 /* State transfer (testing and checkpoint): complex128 host arrays.
  * tensors of class c: (n_c, 2, chi^d_c); messages: (2E, chi, chi); lambdas: (E, chi).
- * Messages may be any matrices.  Those that are not Hermitian (to rounding; what BP and the gauge produce is)
- * run on general kernels, slower, until a BP sweep or the gauge has replaced them. */
+ * Messages may be any matrices.  Those that are not Hermitian positive semidefinite (to rounding; what BP and
+ * the gauge produce is) run on general kernels, slower, until a BP sweep or the gauge has replaced them. */
 int bqa_get_tensors(bqa_job* job, int32_t class_index, double* out);
 int bqa_set_tensors(bqa_job* job, int32_t class_index, int32_t chi, const double* in);
 int bqa_get_messages(bqa_job* job, double* out);

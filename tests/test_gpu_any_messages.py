@@ -1,5 +1,5 @@
-"""Uploaded messages that are not Hermitian against the NumPy oracle: they need kernels that apply every message to the
-ket."""
+"""Uploaded messages that are not Hermitian, or Hermitian and not positive, against the NumPy oracle: they need kernels
+that apply every message to the ket and canonicalisers that factor any matrix."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,7 @@ U = {"single": 6e-8, "double": 1.2e-16}
 
 
 def _state(d, n, chi, precision, kind):
-    """Config, node tensors and messages as the job stores them; kind: "any" or "positive"."""
+    """Config, node tensors and messages as the job stores them; kind: "any", "indefinite" or "positive"."""
     if d == 2:
         nodes, edges = {i: 0.1 for i in range(n)}, {(i, (i + 1) % n): 0.1 + 0.01 * i for i in range(n)}
     else:
@@ -28,6 +28,8 @@ def _state(d, n, chi, precision, kind):
     m = rng.normal(size=(n * d, chi, chi)) + 1j * rng.normal(size=(n * d, chi, chi))
     if kind == "positive":
         m = m @ m.conj().transpose(0, 2, 1)
+    if kind != "any":
+        m = m + m.conj().transpose(0, 2, 1)
     # a trace of one, by the diagonal's mean: traces of random matrices may vanish
     m = m - (np.trace(m, axis1=1, axis2=2)[:, None, None] / chi - 1) * np.eye(chi) if kind != "positive" else m
     m = (m / np.trace(m, axis1=1, axis2=2)[:, None, None]).astype(store)
@@ -134,6 +136,13 @@ def _simple_update(d, chi, n, kind):
     assert np.abs(lam - want[:, :lam.shape[1]]).max() < tol
 
 
+@pytest.mark.parametrize("kind", ["any", "indefinite", "positive"])
+@pytest.mark.parametrize("d,chi,n", SHAPES + [(2, 17, 5), (2, 24, 5), (2, 32, 4)])
+def test_simple_update(d, chi, n, kind):
+    """Lambdas through the extended messages and the job's own canonicalisers, in FP64."""
+    _simple_update(d, chi, n, kind)
+
+
 @pytest.mark.parametrize("precision", ["single", "double"])
 @pytest.mark.parametrize("d,chi,n", [(3, 4, 10), (3, 8, 10), (3, 10, 6), (4, 8, 12)])
 def test_messages_after_a_sweep_are_the_jobs_own(d, chi, n, precision, monkeypatch):
@@ -168,3 +177,27 @@ def test_messages_after_a_sweep_are_the_jobs_own(d, chi, n, precision, monkeypat
         assert np.array_equal(job.get_messages(), own)
     finally:
         job.close()
+
+def test_batch_after_an_upload():
+    """A serving batch's step from such messages gives what the job's own step gives."""
+    from bqa_amd.native import Batch
+    out = []
+    for batched in (False, True):
+        jobs = []
+        try:
+            for d, chi, n, kind in ((3, 4, 10, "any"), (3, 8, 10, "indefinite"), (4, 8, 12, "any"), (3, 8, 10, "positive")):
+                cfg, t, m = _state(d, n, chi, "double", kind)
+                cfg["max_bond_dim"] = chi
+                jobs.append(_job(cfg, t, m, "double"))
+            if batched:
+                batch = Batch(len(jobs))
+                batch.run_layer(jobs, 0.3, 0.2, 1e-6, 40, 1e-9, 0.0)
+            else:
+                for job in jobs:
+                    job.run_layer(0.3, 0.2, 1e-6, 40, 1e-9, 0.0)
+            out.append([job.density()[0] for job in jobs])
+        finally:
+            for job in jobs:
+                job.close()
+    for a, b in zip(*out):
+        assert np.abs(a - b).max() < 1e-9   # pinv_eps = 1e-6 amplifies the rounding between launch variants
