@@ -1,0 +1,73 @@
+// Which shapes the matrix-product kernels (node_gemm.hpp) serve and how many nodes at a time.  Host code without HIP,
+// so its rules are tested on the CPU.
+#pragma once
+
+#include <cstddef>
+
+namespace bqa {
+
+constexpr int kGemmMaxDegree = 6;
+constexpr int kGemmMaxChi = 32;
+constexpr size_t kGemmElement = 16;   // bytes of a complex double
+
+// Shapes served: a node tensor's elements are counted in 32 bits, and without a product to make (degree 1) or
+// to sum (chi = 1) the kernels of kernels_node.hpp take fewer launches (300 degree-1 nodes at chi = 12: 16 against
+// 19 us a sweep; 1,000 degree-3 nodes at chi = 1: 66 against 79 us).
+inline bool gemm_shape(int d, int chi) {
+  if (d < 2 || chi < 2 || d > kGemmMaxDegree || chi > kGemmMaxChi) return false;
+  long s = 2;
+  for (int k = 0; k < d; ++k) s *= chi;
+  return s < (1L << 30);
+}
+
+// Products a node of degree d keeps in the workspace.
+inline int gemm_products(int d) { return d <= 3 ? d : d == 4 ? 6 : d == 5 ? 9 : 12; }
+
+// Nodes per round of launches: their products take at most kGemmBudget bytes (half of the Infinity Cache,
+// so the Grams read them from there), and one node at least.
+constexpr size_t kGemmBudget = 128u << 20;
+inline size_t gemm_node_bytes(int d, int chi, size_t csize) {
+  size_t s = 2 * csize * gemm_products(d);
+  for (int k = 0; k < d; ++k) s *= chi;
+  return s;
+}
+inline int gemm_chunk(int n, int d, int chi, size_t csize) {
+  const size_t node = gemm_node_bytes(d, chi, csize);
+  if (node == 0) return n;
+  const size_t c = kGemmBudget / node;
+  if (c >= (size_t)n) return n;
+  return c >= 8 ? (int)(c / 8 * 8) : c > 0 ? (int)c : 1;
+}
+
+// Classes served.  A single node's products may be many times its tensor (twelve at degree 6), where the generic kernel
+// keeps three node tensors a block: beyond kGemmNodeMost (a seventieth of the card) they may take no more than that, so
+// that a job of one or two large hubs that fits with the generic kernels fits with these.
+constexpr size_t kGemmNodeMost = (size_t)4 << 30;
+inline bool gemm_serves(int n, int d, int chi) {
+  return gemm_shape(d, chi) &&
+         (gemm_node_bytes(d, chi, kGemmElement) <= kGemmNodeMost || gemm_products(d) <= 3 * (n < 1024 ? n : 1024));
+}
+
+// The absorb serves node tensors of which k_node_local cannot keep two FP64 copies in 64 KB of LDS (with them, one
+// block does a node in one launch).
+inline bool gemm_local_shape(int d, int chi_in, int chi_out) {
+  const int most = chi_in > chi_out ? chi_in : chi_out;
+  if (!gemm_shape(d, most) || chi_in < 2 || chi_out < 1) return false;
+  long s = 2;
+  for (int k = 0; k < d; ++k) s *= most;
+  return 2 * s * (long)kGemmElement > 64 * 1024;
+}
+// Nodes per round: two FP64 tensors each, within kGemmBudget and within what 1,024 blocks of the generic kernel take.
+inline size_t gemm_local_node_bytes(int d, int chi) {
+  size_t s = 4 * kGemmElement;
+  for (int k = 0; k < d; ++k) s *= chi;
+  return s;
+}
+inline int gemm_local_chunk(int n, int d, int chi) {
+  size_t c = kGemmBudget / gemm_local_node_bytes(d, chi);
+  if (c > 1024) c = 1024;
+  if (c >= (size_t)n) return n;
+  return c >= 8 ? (int)(c / 8 * 8) : c > 0 ? (int)c : 1;
+}
+
+}  // namespace bqa
