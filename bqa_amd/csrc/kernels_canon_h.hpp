@@ -10,10 +10,11 @@
 //     pairs with only the bot columns moving by one lane-xor per round, then
 //     each half split in two by one re-layout, and so on: 2 P2 - 1 rounds), so
 //     a round moves one column per lane, through the LDS crossbar
-//     (ds_bpermute) rather than VALU moves and selects; other n than powers of
-//     two are padded with zero columns, which never rotate, and each column
-//     carries its number (at n = 24 a round-robin's DPP moves and selects took
-//     twice the rest of a round; 31 padded rounds are cheaper than 23 of them);
+//     (ds_bpermute) rather than VALU moves and selects.  It wants a power of
+//     two of column pairs; padding with zero columns, which never rotate, makes
+//     one, and each column then carries its number.  Where that is a third more
+//     rounds than the n - 1 of a round-robin (n = 6, 10, 12, 18..24), columns go
+//     round by DPP row shifts instead;
 //   * the Hermitian PSD extended messages are factored M = L L^H by pivoted
 //     Cholesky first; one-sided Jacobi on the columns of L then converges in
 //     about half the sweeps of Jacobi on M and yields V_M Sigma_L directly,
@@ -35,6 +36,11 @@ struct HCanon {
   static constexpr int G = 2 * P2;                                  // lanes per edge
   static constexpr int EPW = 64 / G;                                // edges per wave
   static constexpr int NH = N / 2;                                  // rows per lane
+  // The order of the Jacobi's rounds: xor where 2 P2 - 1 rounds are at most 4/3 of N - 1.  Milliseconds for 2 x 8,192
+  // (n <= 14: 16,384) edges, xor and round-robin: n = 10 0.58 and 0.48, 12 0.75 and 0.69, 14 0.94 and 1.02, 18 2.04
+  // and 1.58, 20 2.34 and 1.94, 22 2.63 and 2.35, 24 3.01 and 2.95, 26 3.22 and 3.39, 28 3.63 and 4.08, 30 4.11
+  // and 4.60.
+  static constexpr bool kXor = 3 * (2 * P2 - 1) <= 4 * (N - 1) || P == P2;
   // Split form (both sides of an edge at once): lanes and edges per wave, and the edges up to which it is taken.
   // A wave's serial chain of two factorisations and three Jacobi runs is then two thirds as long, but half of its
   // lanes idle in the third, so it pays while the waves of all edges run at once (two a SIMD).  Measured at that
@@ -88,6 +94,36 @@ __device__ __forceinline__ double half_sum(double v) {
     return v + xor_lane<HCanon<N>::P2>(v);
 }
 
+// Value of the next and of the previous lane of the row.
+__device__ __forceinline__ double dpp_from_next(double x) {  // row_shl:1
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x101, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x101, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double dpp_from_prev(double x) {  // row_shr:1
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x111, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x111, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// One step of the round-robin; after N - 1 of them every column is back in its place.  Padding lanes take copies.
+template <int N>
+__device__ __forceinline__ void hrotate_owners(HCol<N / 2>& top, HCol<N / 2>& bot, int k) {
+  constexpr int P = N / 2, NH = N / 2;
+#pragma unroll
+  for (int r = 0; r < NH; ++r) {
+    const double xr = dpp_from_next(top.re[r]), xi = dpp_from_next(top.im[r]);
+    const double yr = dpp_from_prev(bot.re[r]), yi = dpp_from_prev(bot.im[r]);
+    const double tr = k == 0 ? top.re[r] : (k < P - 1 ? xr : bot.re[r]);
+    const double ti = k == 0 ? top.im[r] : (k < P - 1 ? xi : bot.im[r]);
+    bot.re[r] = k == 0 ? xr : yr;
+    bot.im[r] = k == 0 ? xi : yi;
+    top.re[r] = tr;
+    top.im[r] = ti;
+  }
+}
+
 template <int NH>
 __device__ __forceinline__ double hnorm2(const HCol<NH>& c) {
   double s = 0.0;
@@ -99,8 +135,8 @@ __device__ __forceinline__ double hnorm2(const HCol<NH>& c) {
 // One Jacobi round: rotate the pair of split columns held by this lane pair
 // (top, bot) so that they become orthogonal; `rotated` / `unsettled` collect
 // whether the round rotated at all and whether a rotation was still large.
-// The squared column norms a, b are carried (exact at each sweep's start,
-// updated by the rotation's a - t|g|, b + t|g|, moved with their columns).
+// The xor order carries the squared column norms a, b (exact at each sweep's
+// start, updated by the rotation's a - t|g|, b + t|g|, moved with their columns).
 template <int N>
 __device__ __forceinline__ void hjacobi_round(HCol<N / 2>& top, HCol<N / 2>& bot, double& a, double& b,
                                               double small2, double tol, int& rotated, int& unsettled) {
@@ -151,10 +187,11 @@ __device__ __forceinline__ double bperm(double x, int addr4) {
 }
 
 // One-sided Jacobi on the columns held by the lane pairs of an edge.  it, ib: the columns'
-// numbers (-1: padding), which move with them when n / 2 is no power of two.
+// numbers (-1: padding), which move with them in the padded xor order.
 template <int N>
 __device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int& it, int& ib, int k) {
   constexpr int NH = N / 2, P = N / 2, P2 = HCanon<N>::P2;
+  constexpr bool kIds = HCanon<N>::kXor && P != P2;
   double sc = fmax(half_sum<N>(hnorm2(top)), half_sum<N>(hnorm2(bot)));
 #pragma unroll
   for (int o = 1; o < P2; o <<= 1) sc = fmax(sc, __shfl_xor(sc, o, 64));
@@ -163,6 +200,17 @@ __device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int& it, int& ib, in
   const int lane = threadIdx.x & 63;
   for (int sweep = 0; sweep < 30; ++sweep) {
     int rotated = 0, unsettled = 0;
+    if constexpr (!HCanon<N>::kXor) {
+#pragma unroll 1
+      for (int round = 0; round < N - 1; ++round) {
+        double a = half_sum<N>(hnorm2(top)), b = half_sum<N>(hnorm2(bot));
+        a = k < P ? a : 0.0;   // padding lanes hold copies and do not rotate
+        hjacobi_round<N>(top, bot, a, b, small2, tol, rotated, unsettled);
+        hrotate_owners<N>(top, bot, k);
+      }
+      if (!__any(rotated) || !__any(unsettled)) break;
+      continue;
+    }
     // recursive xor order: in the phase of group size L the tops and the
     // bots of each group of L lanes meet all pairs (bot at lane k holds the
     // bot that started at lane k ^ gray(t) in round t, so round t moves it by
@@ -182,7 +230,7 @@ __device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int& it, int& ib, in
             bot.im[r] = bperm(bot.im[r], addr);
           }
           b = bperm(b, addr);
-          if constexpr (P != P2) ib = __builtin_amdgcn_ds_bpermute(addr, ib);
+          if constexpr (kIds) ib = __builtin_amdgcn_ds_bpermute(addr, ib);
         }
         hjacobi_round<N>(top, bot, a, b, small2, tol, rotated, unsettled);
       }
@@ -201,7 +249,7 @@ __device__ void hjacobi(HCol<N / 2>& top, HCol<N / 2>& bot, int& it, int& ib, in
         const double fn = bperm(hi ? a : b, addr);
         a = hi ? b : a;
         b = fn;
-        if constexpr (P != P2) {
+        if constexpr (kIds) {
           const int fid = __builtin_amdgcn_ds_bpermute(addr, hi ? it : ib);
           it = hi ? ib : it;
           ib = fid;
