@@ -1538,7 +1538,7 @@ int canon_h_epw(int n) {
   const int p = n / 2, p2 = p <= 1 ? 1 : p <= 2 ? 2 : p <= 4 ? 4 : p <= 8 ? 8 : 16;
   return 64 / (2 * p2);
 }
-bool canon_h_split(int n, int E) { return E <= 2048 * (canon_h_epw(n) / 2); }
+bool canon_h_split(int n, int E) { return E <= canon_split_waves(n) * (canon_h_epw(n) / 2); }
 
 template <int N>
 void launch_canon_multi(bool split, const CanonEntry* tab, int entries, int blocks, hipStream_t s) {

@@ -29,6 +29,12 @@
 
 namespace bqa {
 
+// Waves of all edges up to which the split form pays: one a SIMD (0.7 to 0.8 of the time of one side after the other,
+// at every n).  With two, the other form's single wave takes as long or less: split over it at 1,100 and at 2,048 waves,
+// n = 6 1.04 and 1.06, 10 1.10 and 1.11, 16 1.00 and 1.01, 18 1.11 and 1.09, 24 1.12 and 1.05, 32 1.03 and 1.02; but
+// the shortest kernels still gain, n = 2 0.91 and 0.92, 4 0.91 and 0.91, 8 0.93 and 0.93.
+__host__ __device__ constexpr int canon_split_waves(int n) { return n <= 4 || n == 8 ? 2048 : 1024; }
+
 template <int N>
 struct HCanon {
   static constexpr int P = N / 2;                                   // column pairs
@@ -43,11 +49,10 @@ struct HCanon {
   static constexpr bool kXor = 3 * (2 * P2 - 1) <= 4 * (N - 1) || P == P2;
   // Split form (both sides of an edge at once): lanes and edges per wave, and the edges up to which it is taken.
   // A wave's serial chain of two factorisations and three Jacobi runs is then two thirds as long, but half of its
-  // lanes idle in the third, so it pays while the waves of all edges run at once (two a SIMD).  Measured at that
-  // line, split against not: n = 4 40 and 46 us, n = 8 110 and 144, n = 16 397 and 494, n = 22 861 and 1,050.
+  // lanes idle in the third, and there are twice the waves.
   static constexpr int GS = 2 * G;
   static constexpr int EPWS = 64 / GS;
-  static constexpr int kSplitEdges = 2048 * EPWS;
+  static constexpr int kSplitEdges = canon_split_waves(N) * EPWS;
   // workspace doubles per edge: U_f, U_b, Q (N x N complex each), sorted Us and Z columns
   // (N x N complex each), sq/ip of both sides, 1/Lambda of the sorted columns
   static constexpr int WS = 10 * N * N + 5 * N;
