@@ -38,6 +38,11 @@ __device__ __forceinline__ double sum8(double v) {
   return v;
 }
 
+__device__ __forceinline__ double first_lane(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+
 struct WideShared {
   double dg[64], norm[64], il[64];
   zd lcol[64];
@@ -98,8 +103,11 @@ __device__ void wide_cholesky(const zd* __restrict__ M, int n, zd* A, WideShared
         bc = oc;
       }
     }
+    // lanes agree but for NaNs; with the first one's, the branch is the same for all lanes and waves then too
+    bv = first_lane(bv);
+    bc = __builtin_amdgcn_readfirstlane(bc);
     if (step == 0) d0 = bv;
-    if (!(bv > 1e-20 * d0)) break;   // the same in every wave; also for a NaN
+    if (!(bv > 1e-20 * d0)) break;
     const double inv = rsqrt_pos(bv);
     const bool pt = active && bc == ct, pb = active && bc == cb;
     if (pt || pb) {
@@ -347,7 +355,7 @@ __global__ __launch_bounds__(kWideThreads) void k_canon_wide(int E, int edge0, i
     double nrm2 = 0.0;
     for (int j = 0; j < n; ++j) {
       const double o = sh.norm[j];
-      rank += (o > s || (o == s && j < t)) ? 1 : 0;
+      rank += ranks_before(o, j, s, t) ? 1 : 0;   // every rank has a column: they index LDS below
       nrm2 += o > pinv_eps ? o * o : 0.0;
     }
     const bool keep = s > pinv_eps;

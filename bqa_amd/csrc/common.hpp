@@ -92,6 +92,13 @@ __device__ __host__ inline void zz_split(double theta, cplx<double>& g0, cplx<do
   g1 = s * mk(h, -h);
 }
 
+// Whether singular value a of column j comes before b of column k in descending order, ties by column and NaNs first: a
+// total order, so that ranks are a permutation whatever the values (an unordered NaN left ranks without a column).
+__device__ __forceinline__ bool ranks_before(double a, int j, double b, int k) {
+  const bool an = a != a, bn = b != b;
+  return an != bn ? an : (!an && a != b) ? a > b : j < k;
+}
+
 // Non-negative double compares like its bit pattern as uint64.
 __device__ __forceinline__ void atomic_max_nonneg(unsigned long long* addr, double v) {
   if (!(v >= 0.0)) v = __longlong_as_double(0x7ff8000000000000ULL);  // NaN marker: largest pattern

@@ -101,7 +101,7 @@ __device__ void sorted_norms(const zd* A, int n, double* sig, int* perm) {
   __syncthreads();
   for (int j = threadIdx.x; j < n; j += blockDim.x) {
     int rank = 0;
-    for (int k = 0; k < n; ++k) rank += (sig[k] > sig[j]) || (sig[k] == sig[j] && k < j);
+    for (int k = 0; k < n; ++k) rank += ranks_before(sig[k], k, sig[j], j) ? 1 : 0;
     perm[rank] = j;
   }
   __syncthreads();
