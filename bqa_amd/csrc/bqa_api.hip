@@ -1690,7 +1690,7 @@ void batch_bp(bqa_batch* b, int count, bqa_job* const* jobs, const int32_t* max_
       });
       continue;
     }
-    Run r{j, k, BpStatus{}, 0};
+    Run r{j, k, BpHeader{}, 0};
     r.h.cur = j->mcur;
     r.h.best_dist = INFINITY;
     hipLaunchKernelGGL(k_bp_reset, dim3(1), dim3(kResetThreads), 0, b->stream, reinterpret_cast<BpStatus*>(j->status.p),

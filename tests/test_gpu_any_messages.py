@@ -95,6 +95,27 @@ def test_sweeps(d, chi, n, damping, sweeps, precision):
     assert np.abs(got - new).max() < tol
 
 
+@pytest.mark.parametrize("variant", range(5))
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("d,chi,n", [(2, 4, 9), (2, 8, 70), (3, 3, 8), (3, 4, 30), (3, 6, 8), (3, 8, 10), (3, 8, 600), (3, 16, 4),
+                                     (4, 4, 10), (4, 8, 12), (4, 8, 300)])
+def test_launch_variants_on_positive_messages(d, chi, n, precision, variant, monkeypatch):
+    """One sweep of the kernels that Hermitian messages run, under each launch variant (variants that a shape does not
+    have run as the first)."""
+    monkeypatch.setenv("BQA_BP_VARIANT", str(variant))
+    cfg, t, m = _state(d, n, chi, precision, "positive")
+    job = _job(cfg, t, m, precision)
+    try:
+        job.run_bp(1, 0.0, 0.0)
+        got = job.get_messages()
+    finally:
+        job.close()
+    want = _sweep(cfg, t, m, d)
+    # each of the d - 1 products sums chi terms, a Gram's chains a quarter of 2 chi^(d-1); nothing cancels in the trace
+    tol = U[precision] * ((d - 1) * chi + chi ** (d - 1) / 2 + 64) * np.abs(want).max()
+    assert np.abs(got - want).max() < tol
+
+
 @pytest.mark.parametrize("precision", ["single", "double"])
 @pytest.mark.parametrize("d,chi,n", SHAPES)
 def test_readout(d, chi, n, precision):
