@@ -74,6 +74,21 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
+# What the result line keeps of the workloads beside the headline: a reader of the last 8,000 characters gets the whole
+# line.  Everything else goes to stderr.
+BRIEF = {"qubit_steps_per_s", "ms_per_step", "timed_steps", "bp_sweeps_per_step_mean", "bp_sweeps_per_step", "device_bytes",
+         "seconds", "bound", "frac", "mfma_frac", "avg_launch_us", "max_abs_dz", "mean_abs_dz", "qubits_dz_above_1e-4",
+         "spin_mismatches_decided", "energy_rel_err", "jobs", "failed", "jobs_per_h", "p50_s", "p99_s",
+         "capacity_over_one_at_a_time"}
+
+
+def brief(x):
+    if isinstance(x, dict):
+        kept = {k: brief(v) for k, v in x.items() if isinstance(v, dict) or k in BRIEF}
+        return {k: v for k, v in kept.items() if v != {}}
+    return float(f"{x:.6g}") if isinstance(x, float) else x
+
+
 def qubo_config(n, chi, steps, precision):
     from bqa_amd import instances
     nodes, edges, _ = instances.regular_qubo(n, 3, seed=SEED, qmax=10)
@@ -502,14 +517,14 @@ def main():
         "cpu_baseline": cpu,
         "oracle_parity_sample": oracle_parity,
         "accuracy": accuracy_block,
-        TAG[other]: other_line,
-        "serving": serving,
     }
-    result.update(extra)
     from bqa_amd.native import tuning_report
-    result["autotuner"] = [{"precision": r["precision"], "degree": r["degree"], "chi": r["chi"], "n_log2": r["n_log2"],
-                            "chosen": r["variants"][r["chosen"]]["name"],
-                            "us": {v["name"]: v["us"] for v in r["variants"]}} for r in tuning_report()]
+    others = {TAG[other]: other_line, "serving": serving, **extra}
+    log("[bench] details " + json.dumps(dict(others, autotuner=[
+        {"precision": r["precision"], "degree": r["degree"], "chi": r["chi"], "n_log2": r["n_log2"],
+         "chosen": r["variants"][r["chosen"]]["name"], "us": {v["name"]: v["us"] for v in r["variants"]}}
+        for r in tuning_report()])))
+    result.update({k: brief(v) for k, v in others.items()})
     if copy_ms is not None:
         result["copy_calibration"] = {"bytes": args.copy_calibrate, "ms_per_copy": copy_ms,
                                       "GB_per_s": 2 * args.copy_calibrate / 1e6 / copy_ms}
