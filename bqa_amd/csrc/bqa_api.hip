@@ -1534,10 +1534,7 @@ namespace {
 // Split-column canonicaliser geometry of n: workspace doubles per edge, edges per 64-lane block of a job of E edges
 // (a job takes the same form of the kernel in a batch as alone).
 size_t canon_h_ws(int n) { return 10 * (size_t)n * n + 5 * (size_t)n; }
-int canon_h_epw(int n) {
-  const int p = n / 2, p2 = p <= 1 ? 1 : p <= 2 ? 2 : p <= 4 ? 4 : p <= 8 ? 8 : 16;
-  return 64 / (2 * p2);
-}
+int canon_h_epw(int n) { return 64 / (2 * canon_pairs(n)); }
 bool canon_h_split(int n, int E) { return E <= canon_split_waves(n) * (canon_h_epw(n) / 2); }
 
 template <int N>

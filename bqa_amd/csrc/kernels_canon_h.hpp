@@ -29,24 +29,33 @@
 
 namespace bqa {
 
-// Waves of all edges up to which the split form pays: one a SIMD (0.7 to 0.8 of the time of one side after the other,
-// at every n).  With two, the other form's single wave takes as long or less: split over it at 1,100 and at 2,048 waves,
-// n = 6 1.04 and 1.06, 10 1.10 and 1.11, 16 1.00 and 1.01, 18 1.11 and 1.09, 24 1.12 and 1.05, 32 1.03 and 1.02; but
-// the shortest kernels still gain, n = 2 0.91 and 0.92, 4 0.91 and 0.91, 8 0.93 and 0.93.
-__host__ __device__ constexpr int canon_split_waves(int n) { return n <= 4 || n == 8 ? 2048 : 1024; }
+// Column pairs of n = 2 chi, padded to a power of two.
+__host__ __device__ constexpr int canon_pairs(int n) {
+  const int p = n / 2;
+  return p <= 1 ? 1 : p <= 2 ? 2 : p <= 4 ? 4 : p <= 8 ? 8 : 16;
+}
+// The order of the Jacobi's rounds: xor (2 P2 - 1 rounds, P2 padded pairs) where that is at most 4/3 of a round-robin's
+// n - 1.  Milliseconds for 8,192 (n <= 14: 16,384) edges, xor and round-robin: n = 10 0.58 and 0.48, 12 0.75 and
+// 0.69, 14 0.94 and 1.02, 18 2.04 and 1.58, 20 2.34 and 1.94, 22 2.63 and 2.35, 24 3.01 and 2.95, 26 3.22 and 3.39, 28
+// 3.63 and 4.08, 30 4.11 and 4.60.
+__host__ __device__ constexpr bool canon_xor(int n) {
+  return 3 * (2 * canon_pairs(n) - 1) <= 4 * (n - 1) || canon_pairs(n) == n / 2;
+}
+// Waves of all edges up to which the split form is taken.  With one a SIMD (1,024) it takes 0.7 to 0.8 of the time of
+// one side after the other at every n.  With two, split over the other form's single wave at 1,100, 1,536 and 2,048: n = 2
+// 0.91, 0.93, 0.92, 4 0.91, 0.92, 0.91, 8 0.93, 0.91, 0.93, 14 0.98, 1.01, 1.00 and 16 1.00, 1.06, 1.01 (kept, so that a
+// batch's jobs fall into one launch), but 6 1.04, 1.06, 1.06, 10 1.10, 1.13, 1.11, 12 1.06, 1.11, 1.12, 18 1.11, 1.11,
+// 1.09, 24 1.12, 1.10, 1.05, 26 1.03, 1.06, 1.05 and 32 1.03, 0.99, 1.02.
+__host__ __device__ constexpr int canon_split_waves(int n) { return canon_xor(n) && n <= 16 ? 2048 : 1024; }
 
 template <int N>
 struct HCanon {
   static constexpr int P = N / 2;                                   // column pairs
-  static constexpr int P2 = P <= 1 ? 1 : P <= 2 ? 2 : P <= 4 ? 4 : P <= 8 ? 8 : 16;
+  static constexpr int P2 = canon_pairs(N);
   static constexpr int G = 2 * P2;                                  // lanes per edge
   static constexpr int EPW = 64 / G;                                // edges per wave
   static constexpr int NH = N / 2;                                  // rows per lane
-  // The order of the Jacobi's rounds: xor where 2 P2 - 1 rounds are at most 4/3 of N - 1.  Milliseconds for 2 x 8,192
-  // (n <= 14: 16,384) edges, xor and round-robin: n = 10 0.58 and 0.48, 12 0.75 and 0.69, 14 0.94 and 1.02, 18 2.04
-  // and 1.58, 20 2.34 and 1.94, 22 2.63 and 2.35, 24 3.01 and 2.95, 26 3.22 and 3.39, 28 3.63 and 4.08, 30 4.11
-  // and 4.60.
-  static constexpr bool kXor = 3 * (2 * P2 - 1) <= 4 * (N - 1) || P == P2;
+  static constexpr bool kXor = canon_xor(N);                        // order of the Jacobi's rounds
   // Split form (both sides of an edge at once): lanes and edges per wave, and the edges up to which it is taken.
   // A wave's serial chain of two factorisations and three Jacobi runs is then two thirds as long, but half of its
   // lanes idle in the third, and there are twice the waves.

@@ -14,7 +14,7 @@ from oracle import bqa_oracle as O
 pytestmark = pytest.mark.gpu
 
 
-# few edges: both sides of an edge at once; more than 1,024 (chi = 4: 2,048) waves of them: one side after the other
+# few edges: both sides of an edge at once; more than 1,024 (chi = 4 and 8: 2,048) waves: one side after the other
 @pytest.mark.parametrize("chi,edges", [(c, 6) for c in (2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 13, 14, 15, 16)]
                          + [(3, 4096), (3, 4097), (4, 8193), (8, 2048), (8, 2049), (11, 1024), (11, 1025)]
                          + [(3, 8193), (5, 4097), (6, 4097), (7, 4097), (9, 2049), (12, 2049), (15, 2049)])
