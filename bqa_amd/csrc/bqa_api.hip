@@ -595,7 +595,7 @@ void launch_bp_class(bqa_job* j, ClassDev& c, int sweep, bool first, bool any = 
   }
   if (!fast || !fast_bp_launch<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0),
                          msg_ptr<R>(j, 1), reinterpret_cast<BpStatus*>(j->status.p), j->stream, variant)) {
-    if (!j->generic(kGenBP) && gemm_serves(c.n, c.d, chi) && (!any || c.d == 2)) {   // degree 2: its message on the ket
+    if (!j->generic(kGenBP) && gemm_serves(kGemmBp, c.n, c.d, chi, sizeof(cplx<R>)) && (!any || c.d == 2)) {   // degree 2: its message on the ket
       const int chunk = plan_gemm(j, c, chi, sizeof(cplx<R>));
       gemm_bp<R>(view, chi, reinterpret_cast<const cplx<R>*>(c.T[c.tcur].p), msg_ptr<R>(j, 0), msg_ptr<R>(j, 1),
                  reinterpret_cast<BpStatus*>(j->status.p), j->gws.p, chunk, j->stream);
@@ -892,7 +892,7 @@ void ext_class(bqa_job* j, ClassDev& c, double ztime, const cplx<double>* msgs64
     LAUNCH_CHECK();
     return;
   }
-  if (!j->generic(kGenExt) && gemm_serves(c.n, c.d, chi) && (j->hermitian || c.d == 2)) {
+  if (!j->generic(kGenExt) && gemm_serves(kGemmExt, c.n, c.d, chi, sizeof(cplx<double>)) && (j->hermitian || c.d == 2)) {
     const int chunk = plan_gemm(j, c, chi, sizeof(cplx<double>));
     gemm_ext<R>(v, chi, T, msg_ptr<R>(j, j->mcur), ext, j->gws.p, chunk, j->stream);
     LAUNCH_CHECK();
@@ -941,7 +941,7 @@ void ext_and_canon(bqa_job* j, double ztime, double pinv_eps, bool sync = true, 
     need_generic |= c.d != 0 && c.n > 0 &&
                     (j->generic(kGenExt) ||
                      !(chi == 1 || (j->hermitian ? ext_fast_shape<R>(c.d, chi) : ext_ket_shape<R>(c.d, chi)) ||
-                       (gemm_serves(c.n, c.d, chi) && (j->hermitian || c.d == 2))));
+                       (gemm_serves(kGemmExt, c.n, c.d, chi, sizeof(cplx<double>)) && (j->hermitian || c.d == 2))));
   if (sizeof(R) == sizeof(float) && need_generic) {
     const long cnt = (long)j->M * chi * chi;
     j->conv_msgs.ensure((size_t)cnt * sizeof(cplx<double>), j->dev_bytes, j->stream);
@@ -1209,7 +1209,7 @@ void density_impl(bqa_job* j, double* rho_out, double* bloch_out) {
       LAUNCH_CHECK();
       continue;
     }
-    if (!j->generic(kGenDensity) && gemm_serves(c.n, c.d, chi) && j->hermitian) {
+    if (!j->generic(kGenDensity) && gemm_serves(kGemmDensity, c.n, c.d, chi, sizeof(cplx<R>)) && j->hermitian) {
       const int chunk = plan_gemm(j, c, chi, sizeof(cplx<R>));
       gemm_density<R>(c.view(), chi, T, msg_ptr<R>(j, j->mcur), reinterpret_cast<double*>(j->rho.p),
                       reinterpret_cast<double*>(j->bloch.p), j->gws.p, chunk, j->stream);
@@ -1453,7 +1453,7 @@ size_t estimate(int N, int M, const std::vector<int>& deg, const std::vector<int
       const bool fast = density_fast_shape(deg[c], chi) &&
                         (prec == BQA_PREC_SINGLE ? bp_fast_shape<float>(deg[c], chi) && ext_fast_shape<float>(deg[c], chi)
                                                  : bp_fast_shape<double>(deg[c], chi) && ext_fast_shape<double>(deg[c], chi));
-      if (size[c] > 0 && !fast && gemm_serves(size[c], deg[c], chi))
+      if (size[c] > 0 && !fast && gemm_fits(size[c], deg[c], chi))
         gws = std::max(gws, (double)gemm_chunk(size[c], deg[c], chi, 16) * (double)gemm_node_bytes(deg[c], chi, 16));
     }
   b += gws;
@@ -1497,6 +1497,18 @@ void sv_passes(bqa_sv* s, const double* ez, double ztime, double xtime, F&& each
   const double c = std::cos(xtime), sn = std::sin(xtime);
   auto* psi = reinterpret_cast<cplx<double>*>(s->psi.p);
   auto* part = reinterpret_cast<double*>(s->part.p);
+  if (n <= (MODE == 0 ? kSvLdsLayer : kSvLdsRead)) {
+    for (int b0 = 0; b0 < n;) {
+      const int row = std::min(b0, kSvRowBits), t = std::min(kSvLdsBits - row, n - b0);
+      const int g = sv_grid(1ULL << (n - row - t));
+      hipLaunchKernelGGL((k_sv_lds<MODE>), dim3(g), dim3(kSvThreads), 0, s->stream, psi, n, b0, t, row,
+                         b0 == 0 ? ez : nullptr, ztime, c, sn, part);
+      LAUNCH_CHECK();
+      each(g, b0, t, 0);
+      b0 += t;
+    }
+    return;
+  }
   const int tb = std::min(n, kSvTileBits);
   const int g0 = sv_grid(1ULL << (n - tb));
   hipLaunchKernelGGL((k_sv_low<MODE>), dim3(g0), dim3(kSvThreads), 0, s->stream, psi, n, ez, ztime, c, sn, part);

@@ -18,6 +18,10 @@
 // a layer is three passes and the readout three reads (0.70 + 2 x 0.41 and 0.72 ms); with tiles of 1,024 amplitudes and every rotation through
 // LDS they were four passes (2.0 ms a layer) and the readout took 9.6 ms, most of it in lane reductions of every
 // qubit of every tile and in a serial sum over the blocks.
+// Few amplitudes run on tiles of 1,024 in LDS instead (k_sv_lds): up to 2^17 the register tiles are at most 32 blocks,
+// each with the latency of its loads, sixteen sincos a thread and four exchanges.  Microseconds of a layer's call, LDS
+// and register tiles: 4 qubits 12.9 and 18.0, 10 16.6 and 19.5, 12 20.0 and 21.1, 13 20.4 and 24.5, 16 23.2 and 26.0, 18
+// 29.8 and 29.9, 20 47.6 and 38.4; of a readout's, 4 qubits 41.7 and 51.5, 10 48.7 and 51.8, 11 69.7 and 51.5.
 #pragma once
 
 #include "common.hpp"
@@ -29,6 +33,9 @@ constexpr int kSvTileBits = 12;            // amplitudes per tile: 4,096, sixtee
 constexpr int kSvRowBits = 4;              // least contiguous amplitudes per row in the high-qubit passes
 constexpr int kSvThreads = 256;
 constexpr int kSvMaxEdges = 2048;          // edges kept in LDS by the energy kernel
+constexpr int kSvLdsBits = 10;             // amplitudes per LDS tile: 1,024
+constexpr int kSvLdsLayer = 17;            // most qubits whose layers run on LDS tiles
+constexpr int kSvLdsRead = kSvLdsBits;     // and whose readout does: one tile
 
 // Ez(x) for every basis state; fields and edges staged in LDS.
 __global__ __launch_bounds__(kSvThreads) void k_sv_energy(double* __restrict__ ez, int n, const double* __restrict__ h,
@@ -62,6 +69,73 @@ __global__ void k_sv_init(cplx<double>* __restrict__ psi, int n) {
   for (unsigned long long x = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; x < dim;
        x += (unsigned long long)gridDim.x * blockDim.x)
     psi[x] = mk(__popcll(x) & 1 ? -a : a, 0.0);
+}
+
+// One pass over qubits b0 .. b0 + t - 1 on LDS tiles of 2^row contiguous amplitudes times the 2^t values of the qubits
+// (row <= b0, row + t <= 10).  MODE 0: the diagonal phase exp(-i ztime Ez) (when ez != nullptr), then the qubits' X
+// rotations, each by all threads between two barriers.  MODE 1: the sums of the qubits' readout to part, where a wave
+// adds its lanes' pairs by shuffles.
+template <int MODE>
+__global__ __launch_bounds__(kSvThreads) void k_sv_lds(cplx<double>* __restrict__ psi, int n, int b0, int t, int row,
+                                                       const double* __restrict__ ez, double ztime, double c, double sn,
+                                                       double* part) {
+  __shared__ cplx<double> s[1 << kSvLdsBits];
+  __shared__ double sums[4 * kSvLdsBits][kSvThreads / 64];
+  const int size = 1 << (row + t), half = size >> 1, mid = b0 - row;
+  const unsigned long long tiles = 1ULL << (n - row - t);
+  for (unsigned long long T = blockIdx.x; T < tiles; T += gridDim.x) {
+    const unsigned long long base = (T & ((1ULL << mid) - 1ULL)) << row | (T >> mid) << (b0 + t);
+    auto at = [&](int k) { return base | (unsigned long long)(k & ((1 << row) - 1)) | (unsigned long long)(k >> row) << b0; };
+    for (int k = threadIdx.x; k < size; k += kSvThreads) {
+      cplx<double> a = psi[at(k)];
+      if (MODE == 0 && ez) {
+        double sp, cp;
+        sincos(-ztime * ez[at(k)], &sp, &cp);
+        a = a * mk(cp, sp);
+      }
+      s[k] = a;
+    }
+    __syncthreads();
+    for (int b = row; b < row + t; ++b) {
+      const int m = 1 << b;
+      double v[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int p = threadIdx.x; p < half; p += kSvThreads) {
+        const int k0 = (p >> b) << (b + 1) | (p & (m - 1)), k1 = k0 | m;   // the p-th pair of bit b
+        const cplx<double> a0 = s[k0], a1 = s[k1];
+        if (MODE == 0) {
+          // (cos t) a - i (sin t) X a
+          s[k0] = mk(c * a0.x + sn * a1.y, c * a0.y - sn * a1.x);
+          s[k1] = mk(c * a1.x + sn * a0.y, c * a1.y - sn * a0.x);
+        } else {
+          v[0] += abs2(a0);
+          v[1] += abs2(a1);
+          v[2] = fma(a0.x, a1.x, fma(a0.y, a1.y, v[2]));
+          v[3] = fma(a0.x, a1.y, fma(-a0.y, a1.x, v[3]));
+        }
+      }
+      if (MODE == 0) {
+        __syncthreads();
+      } else {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          for (int o = 32; o > 0; o >>= 1) v[x] += __shfl_xor(v[x], o, 64);
+          if ((threadIdx.x & 63) == 0) sums[4 * (b - row) + x][threadIdx.x >> 6] = v[x];
+        }
+      }
+    }
+    if (MODE == 0) {
+      for (int k = threadIdx.x; k < size; k += kSvThreads) psi[at(k)] = s[k];
+      __syncthreads();
+    }
+  }
+  if (MODE == 1) {   // one tile (n <= 10), so the sums are whole
+    __syncthreads();
+    for (int x = threadIdx.x; x < 4 * t; x += kSvThreads) {
+      double v = 0.0;
+      for (int w = 0; w < kSvThreads / 64; ++w) v += sums[x][w];
+      part[(size_t)blockIdx.x * 4 * kSvTileBits + x] = v;
+    }
+  }
 }
 
 // Tile element of register j in the three layouts: the registers' tile bits are 8..11 (A), 4..7 (B) or 0..3 (C).

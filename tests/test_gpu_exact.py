@@ -156,3 +156,10 @@ def test_passes_at_every_split_of_the_qubits(n):
         ref = v @ v.conj().T
         assert np.abs(np.asarray(rho)[q] - ref).max() < 2 * tol
         assert abs(np.asarray(bloch)[q][2] - (ref[0, 0] - ref[1, 1]).real) < 4 * tol
+
+
+@pytest.mark.parametrize("n", [2, 3, 9, 10, 14, 15, 18, 20])
+def test_passes_at_the_edges_of_the_tiles(n):
+    """One LDS tile with whole and partial waves, layers over further LDS tiles, and the first sizes on register tiles
+    (readout 11, layers 18)."""
+    test_passes_at_every_split_of_the_qubits(n)

@@ -1,5 +1,5 @@
 """Which classes the matrix-product kernels serve (csrc/node_gemm_shape.hpp), compiled for the CPU: their workspace is
-small, or no larger than the generic kernels'."""
+small, or no larger than the generic kernels', and small tensors of many nodes are left to those."""
 import os
 import shutil
 import subprocess
@@ -19,7 +19,7 @@ int main() {
   for (int d = 1; d <= 7; ++d)
     for (int chi = 1; chi <= 40; ++chi)
       for (int n : {1, 2, 3, 4, 5, 8, 100, 1024, 5000}) {
-        if (!gemm_serves(n, d, chi)) {
+        if (!gemm_fits(n, d, chi)) {
           refused += gemm_shape(d, chi);
           continue;
         }
@@ -38,9 +38,25 @@ int main() {
         }
       }
   // a single hub of degree 6 at chi = 24 (6 GB in FP64, 73 GB of products) and the shapes of ordinary graphs
-  if (gemm_serves(1, 6, 24) || gemm_serves(2, 6, 24) || !gemm_serves(4, 6, 24) || !gemm_serves(1, 5, 24) ||
-      !gemm_serves(1, 4, 32) || !gemm_serves(120, 5, 8) || !gemm_serves(100, 3, 32))
+  if (gemm_fits(1, 6, 24) || gemm_fits(2, 6, 24) || !gemm_fits(4, 6, 24) || !gemm_fits(1, 5, 24) || !gemm_fits(1, 4, 32) ||
+      !gemm_fits(120, 5, 8) || !gemm_fits(100, 3, 32))
     return 2;
+  // tensors above 2,048 elements never go back to the generic kernel for being small, nor any below for few nodes in BP
+  for (GemmUse use : {kGemmBp, kGemmExt, kGemmDensity})
+    for (int d = 2; d <= 6; ++d)
+      for (int chi = 2; chi <= 32; ++chi) {
+        double tensor = 2;
+        for (int k = 0; k < d; ++k) tensor *= chi;
+        for (int n : {1, 100, 300, 1024, 100000})
+          for (size_t element : {8, 16})
+            if (gemm_too_small(use, n, d, chi, element) && (tensor > 2048 || (use != kGemmDensity && (n <= 100 || tensor > 512))))
+              return 4;
+      }
+  if (!gemm_too_small(kGemmBp, 578, 5, 2, 16) || gemm_too_small(kGemmBp, 120, 5, 2, 16) || gemm_too_small(kGemmBp, 3000, 5, 4, 16) ||
+      !gemm_too_small(kGemmBp, 1200, 2, 13, 16) || gemm_too_small(kGemmBp, 1200, 2, 13, 8) || gemm_too_small(kGemmBp, 10000, 2, 13, 16) ||
+      !gemm_too_small(kGemmExt, 3000, 5, 3, 16) || gemm_too_small(kGemmExt, 600, 5, 3, 16) || gemm_too_small(kGemmExt, 3000, 3, 9, 16) ||
+      !gemm_too_small(kGemmDensity, 20, 5, 2, 16) || gemm_too_small(kGemmDensity, 20, 5, 4, 16) || gemm_too_small(kGemmDensity, 3000, 3, 9, 8))
+    return 5;
   std::printf("%d %d\n", served, refused);
   return served > 0 && refused > 0 ? 0 : 3;
 }
