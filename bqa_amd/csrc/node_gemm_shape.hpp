@@ -44,20 +44,23 @@ inline int gemm_chunk(int n, int d, int chi, size_t csize) {
 //   BP sweep, FP64: degree 2, 600 nodes chi = 9 29 and 16, 11 30 and 20, 12 32 and 26, 13 35 and 29, 14 36 and 32, 15 37 and
 //   36; 10,000 nodes chi = 9 223 and 108, 12 241 and 228, 13 256 and 258; degree 5, chi = 2 400 nodes 38 and 34, 3,000 116
 //   and 83, chi = 3 400 nodes 52 and 44, 10,000 703 and 502; but 260 nodes 38 and 43, and chi = 4 144 and 306 for 600.
-//   FP32: degree 2, 600 nodes chi = 9 23 and 15, 11 24 and 18, 12 3,000 nodes 56 and 72.
 //   Simple update: degree 5, 3,000 nodes chi = 2 164 and 128, 3 321 and 288; 600 nodes 69 and 69, 110 and 112; degree 2,
 //   3,000 nodes chi = 9 716 and 692, 12 1,287 and 1,292.
 //   Readout call: degree 5, 20 nodes chi = 2 48 and 39, chi = 4 47 and 63; 1,200 nodes chi = 2 60 and 43, 3 74 and 53, 4 172
 //   and 157; degree 4, chi = 5 600 nodes 73 and 84, 3,000 195 and 187; degree 3, 3,000 nodes chi = 9 182 and 242; degree 2,
 //   3,000 nodes chi = 9 78 and 61, 12 83 and 86.
+// FP32 sweeps and readouts stay with the products, whose Grams are summed in FP64 (readouts within 0.7 times the generic
+// kernel's distance from 64 bits), though degree 2 with 600 nodes at chi = 9 takes 23 us a sweep for 15; extended messages
+// are FP64 arithmetic in both.
 enum GemmUse { kGemmBp, kGemmExt, kGemmDensity };
 inline bool gemm_too_small(GemmUse use, int n, int d, int chi, size_t element) {
+  if (element != kGemmElement) return false;
   long s = 2;
   for (int k = 0; k < d && s <= 4096; ++k) s *= chi;
   switch (use) {
     case kGemmBp:
-      if (element == kGemmElement && d == 2 && s > 288) return s <= 400 && n >= 384 && n * s <= 500000;
-      return s <= (element == kGemmElement ? 512 : 256) && n >= (d == 2 ? 256 : 384);
+      if (d == 2 && s > 288) return s <= 400 && n >= 384 && n * s <= 500000;
+      return s <= 512 && n >= (d == 2 ? 256 : 384);
     case kGemmExt:
       return s <= (d == 2 ? 256 : 512) && n >= 1024;
     default:

@@ -52,6 +52,9 @@ int main() {
             if (gemm_too_small(use, n, d, chi, element) && (tensor > 2048 || (use != kGemmDensity && (n <= 100 || tensor > 512))))
               return 4;
       }
+  // FP32 products are summed with more bits than the generic kernel's
+  for (GemmUse use : {kGemmBp, kGemmDensity})
+    if (gemm_too_small(use, 5000, 2, 9, 8) || gemm_too_small(use, 5000, 6, 2, 8)) return 6;
   if (!gemm_too_small(kGemmBp, 578, 5, 2, 16) || gemm_too_small(kGemmBp, 120, 5, 2, 16) || gemm_too_small(kGemmBp, 3000, 5, 4, 16) ||
       !gemm_too_small(kGemmBp, 1200, 2, 13, 16) || gemm_too_small(kGemmBp, 1200, 2, 13, 8) || gemm_too_small(kGemmBp, 10000, 2, 13, 16) ||
       !gemm_too_small(kGemmExt, 3000, 5, 3, 16) || gemm_too_small(kGemmExt, 600, 5, 3, 16) || gemm_too_small(kGemmExt, 3000, 3, 9, 16) ||
